@@ -8,8 +8,7 @@ int launch_fwd_d64(const float* A, const float* B, const float* Q, const float* 
                   float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s, int flags,
                   int32_t* /*rescue_ws: no fp64 rescue at d = 64*/) {
   // fp32 sweeps without per-step gains run on the matrix cores unless the row-layout kernel
-  // is asked for: the certified symplectic sweep by default (head counts that are multiples
-  // of 4), per-step Riccati when asked for
+  // is asked for: the certified symplectic sweep by default, per-step Riccati when asked for
   if (!(flags & (TTC_LQR_FLAG_FP64_RICCATI | TTC_LQR_FLAG_ROW_KERNEL)) && sm != STASH_GAINS)
     return launch_fwd_d64_mfma(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, sm, status, s,
                                !(flags & TTC_LQR_FLAG_RICCATI_STEPS));

@@ -1,0 +1,476 @@
+// ttc_lqr_symw.hpp -- d = du = 32 / 64 forward: the certified symplectic sweep on the bf16 matrix
+// cores with three-way splits (ttc_lqr_split.hpp), then the final solve and Riccati step 0.
+//
+// The sweep (the reference's transposed row-block update, symplectic_iter.py:226-251) keeps
+// Y-hat = [Y1'; Y2'] with V_t = Y1^{-1} Y2 and per step forms
+//   M = R^{-1} B_k' Y2'      Y1' <- A_k^{-1} (Y1' + B_k M)      Y2' <- A_k Y2' + Qc_k Y1'
+// Only left products, so the columns of Y-hat are independent: a wave owns 32 of them -- a whole
+// problem at d = 32, half of one at d = 64 -- and no wave waits for another inside the loop.  32
+// columns let one 32 x 32 x 16 instruction read each A operand once (half the LDS traffic of 16
+// columns, which at d = 64 would be as long as the matrix work), and hold the state of a wave in
+// 64 registers at d = 64 (32 at d = 32), so two waves share a SIMD there (three at d = 32).
+// The A operands B', B and -sym(Q) are the token's, the same for every head: split once into LDS
+// (72 KB at d = 64, 18 KB at d = 32), in the order a lane reads them (16 bytes per lane and part).
+//
+// 32 x 32 tile in the MFMA C layout: lane l = 32 h + m holds, in register r, row
+// 8 (r >> 2) + 4 h + (r & 3) of column m.  Registers 8 b .. 8 b + 7 are the rows 16 b + 8 (j >> 2)
+// + 4 h + (j & 3) of k-block b: a C tile is a B operand as it stands, with the A operand's k
+// permuted the same way.
+//
+// Bound at d = 64: 288 matrix instructions per problem-step (9,200 busy cycles per SIMD) beside about
+// 1,300 vector instructions, and the power they draw: at 32,768 problems x 128 steps the matrix cores
+// are busy 67 % of the time at 1.27 PFLOP/s (bf16), and the clock falls from 2.4 to 1.8 GHz, so that
+// fewer cycles (dot-product residuals, 6.55e7, against masked subtractions and interleaved issue,
+// 5.64e7) gave the same time.  47.1 -> 30.5 ms there against the fp32 matrix cores (90 % of their
+// peak); 256 problems 1.65 -> 0.66 ms; one head (1,024 problems), which ran Riccati steps, 3.87 ->
+// 1.75 ms.
+#pragma once
+#include "ttc_lqr_mfma_blk.hpp"
+#include "ttc_lqr_split.hpp"
+
+namespace ttc {
+
+template <int D>
+struct SymW {
+  static_assert(D == 32 || D == 64, "wide symplectic sweep");
+  static constexpr int NI = D / 32;    // 32 x 32 tiles per dimension
+  static constexpr int NK = D / 16;    // k-blocks of a product
+  static constexpr int NB = D / 16;    // 16 x 16 tiles per dimension (step 0)
+  static constexpr int WPP = D / 32;   // waves per problem
+  static constexpr int RPP = 64 / D;   // problems per pair of waves (row layout: 64 lanes, D rows each)
+  static constexpr int MAXPB = D == 64 ? 2 : 8;  // problems per workgroup
+  static constexpr int LDX = D + kPad;
+  static constexpr int REG = D * LDX;  // per problem, after the sweep: D rows
+  static constexpr int FRAG = 9 * NI * NK * 256;  // floats of the split operands [matrix][part][I][kb][lane]
+  static constexpr int VEC = 4 * D;    // per wave: alpha, q, -beta^2 R^{-1}, 1 / alpha
+  static constexpr int AUGW = D == 32 ? 3 * D : 2 * D;  // final solve: [Y1 | -Y2 | I] (d = 64: no identity)
+  static constexpr int MINW = D == 32 ? 3 : 2;     // waves per SIMD the registers must allow
+  static_assert(REG >= AUGW + 4, "pivot row fits a problem's region");
+  // problems of a workgroup rounded up to whole pairs of waves
+  __host__ __device__ static constexpr int regions(int PB) { return (PB + RPP - 1) / RPP * RPP; }
+  __host__ __device__ static constexpr int body(int PB) {
+    return FRAG > regions(PB) * REG ? FRAG : regions(PB) * REG;
+  }
+  static size_t lds_bytes(int PB) {
+    return sizeof(float) * (size_t)(body(PB) + regions(PB) * WPP * VEC + regions(PB));
+  }
+};
+
+template <int D, int SM, bool WRITE_U>
+__global__ __launch_bounds__(64 * SymW<D>::WPP * SymW<D>::MAXPB)
+__attribute__((amdgpu_waves_per_eu(SymW<D>::MINW, SymW<D>::MINW))) void
+lqr_symw_kernel(const float* __restrict__ A_diag, const float* __restrict__ Bg, const float* __restrict__ Qg,
+                const float* __restrict__ Rinv, const float* __restrict__ Qf, const float* __restrict__ lgA,
+                const float* __restrict__ lgB, const float* __restrict__ lgQ, const float* __restrict__ h0, int H,
+                int T, int PB, float* __restrict__ u_out, float* __restrict__ kstash, float* __restrict__ q0stash,
+                int* __restrict__ status) {
+  using G = SymW<D>;
+  constexpr int NI = G::NI, NK = G::NK, NB = G::NB, WPP = G::WPP, LDX = G::LDX, RPP = G::RPP;
+  extern __shared__ __align__(16) float sm[];
+  constexpr float kLog2e = 1.4426950408889634f;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l31 = lane & 31, hh = lane >> 5;  // 32 x 32 tiles: column, row half
+  const int g = lane >> 4, c = lane & 15;     // 16 x 16 tiles (step 0)
+  const int li = lane % D;                    // row layout
+  // XCD-aware block order (consecutive workgroups go round-robin to the 8 XCDs, each with its own
+  // L2): a contiguous run of workgroups per XCD, so that those of one token share an L2
+  const unsigned nblk = gridDim.x, bid = blockIdx.x;
+  const unsigned lblk = (nblk % 8u == 0u) ? (bid % 8u) * (nblk / 8u) + bid / 8u : bid;
+  const int groups = (H + PB - 1) / PB;
+  const int64_t n = lblk / (unsigned)groups;
+  const int head0 = (int)(lblk % (unsigned)groups) * PB;
+  const int pb = wv / WPP;                    // my problem of the workgroup
+  const int ch = wv % WPP;                    // my 32 columns of it
+  const int64_t pid = n * H + (head0 + pb < H ? head0 + pb : H - 1);  // idle: recompute, never store
+  const float* bq = Bg + n * D * D;
+  const float* qq = Qg + n * D * D;
+  float* vec = sm + G::body(PB) + wv * G::VEC;
+  float* okf = sm + G::body(PB) + G::regions(PB) * WPP * G::VEC;
+
+  // split operands of the token: matrix 0: B' , 1: B, 2: -sym(Q); lane (m, h), slot j holds
+  // X[32 I + m][16 kb + 8 (j >> 2) + 4 h + (j & 3)]
+  v8bf* frag = reinterpret_cast<v8bf*>(sm);
+  for (int e = threadIdx.x; e < 3 * NI * NK * 64; e += blockDim.x) {
+    const int ln = e & 63, kb = (e >> 6) % NK, I = (e >> 6) / NK % NI, mat = (e >> 6) / (NK * NI);
+    const int m = 32 * I + (ln & 31), k0 = 16 * kb + 4 * (ln >> 5);
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int k = k0 + 8 * (j >> 2) + (j & 3);
+      x[j] = mat == 0 ? bq[k * D + m] : mat == 1 ? bq[m * D + k] : -0.5f * (qq[m * D + k] + qq[k * D + m]);
+    }
+    const Split8 s = split8(v4f{x[0], x[1], x[2], x[3]}, v4f{x[4], x[5], x[6], x[7]});
+    const int at = ((mat * 3 * NI + I) * NK + kb) * 64 + ln;
+    frag[at] = s.hi;
+    frag[at + NI * NK * 64] = s.mid;
+    frag[at + 2 * NI * NK * 64] = s.lo;
+  }
+
+  // my 32 columns of Y1' = I and of -Y2' = -sym(Q_f)
+  v16f Y1[NI], NV[NI];
+  {
+    const float* fq = Qf + pid * D * D;
+    const int j = 32 * ch + l31;
+#pragma unroll
+    for (int I = 0; I < NI; ++I)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = 32 * I + 8 * (r >> 2) + 4 * hh + (r & 3);
+        NV[I][r] = -0.5f * (fq[i * D + j] + fq[j * D + i]);
+        Y1[I][r] = (i == j) ? 1.0f : 0.0f;
+      }
+  }
+  const float a_l = A_diag[pid * D + li];
+  const float lb2_l = lgB[pid * D + li] * kLog2e, lq2_l = lgQ[pid * D + li] * kLog2e;
+  const float la2_l = lgA[pid] * kLog2e;
+  const float rinv_l = Rinv[pid * D + li];
+  // step ratios of the discount factors (t runs down): q(t-1) = q(t) 2^{-lq2} and
+  // beta(t-1)^2 = beta(t)^2 2^{-2 lb2}, as pairs hi + lo from a double exp2 (no drift)
+  float rQ, rQe, rB2, rB2e;
+  {
+    const double x = exp2((double)-lq2_l), y = exp2((double)(-2.0f * lb2_l));
+    rQ = (float)x;
+    rQe = (float)(x - (double)rQ);
+    rB2 = (float)y;
+    rB2e = (float)(y - (double)rB2);
+  }
+  __syncthreads();  // operands written
+
+  auto operand = [&](int mat, int I, int kb) {
+    const v8bf* f = frag + ((mat * 3 * NI + I) * NK + kb) * 64 + lane;
+    return Split8{f[0], f[NI * NK * 64], f[2 * NI * NK * 64]};
+  };
+  // acc[I] += X S for one matrix X; src(kb, i): rows 16 kb + 8 i + 4 h .. + 3 of S, i = 0, 1
+  // (software pipelined: the operands and the split of k-block kb + 1 are issued between the matrix
+  // instructions of kb, so that one wave keeps both units busy)
+  auto product = [&](int mat, auto&& src, v16f (&acc)[NI]) {
+    Split8 b = split8(src(0, 0), src(0, 1)), a[NI];
+#pragma unroll
+    for (int I = 0; I < NI; ++I) a[I] = operand(mat, I, 0);
+#pragma unroll
+    for (int kb = 0; kb < NK; ++kb) {
+      Split8 an[NI], bn = b;
+      if (kb + 1 < NK) {
+#pragma unroll
+        for (int I = 0; I < NI; ++I) an[I] = operand(mat, I, kb + 1);
+        bn = split8(src(kb + 1, 0), src(kb + 1, 1));
+      }
+      mfma32_split(a, b, acc);
+      if (kb + 1 < NK) {
+#pragma unroll
+        for (int i = 0; i < 3 * NI; ++i) {  // matrix instruction, LDS read, vector instructions
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 3 * NI; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+        }
+#pragma unroll
+        for (int I = 0; I < NI; ++I) a[I] = an[I];
+        b = bn;
+      }
+    }
+  };
+  // row vector `which` of the wave, rows 32 I + 8 i + 4 h .. + 3
+  auto rows4 = [](const v16f& x, int i) { return v4f{x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3]}; };
+  auto rowvec = [&](int which, int I, int i) { return ld4(vec + which * D + 32 * I + 8 * i + 4 * hh); };
+
+  float q_l = 0.f, nb2_l = 0.f;
+  for (int t = T - 1; t >= 1; --t) {
+    // e_A is an exp2 every step (by recurrence it costs the gradients accuracy), the other
+    // factors one every kSymRefresh steps
+    if ((T - 1 - t) % kSymRefresh == 0) {
+      const float beta = __builtin_amdgcn_exp2f(lb2_l * (float)(t + 1));
+      q_l = __builtin_amdgcn_exp2f(lq2_l * (float)t);
+      nb2_l = -(beta * beta) * rinv_l;
+    } else {
+      q_l = fmaf(q_l, rQ, q_l * rQe);
+      nb2_l = fmaf(nb2_l, rB2, nb2_l * rB2e);
+    }
+    const float alpha = fmaf(a_l, __builtin_amdgcn_exp2f(la2_l * (float)(t + 1)), 1.0f);
+    wave_sync();  // the previous step's reads
+    vec[li] = alpha;
+    vec[D + li] = q_l;
+    vec[2 * D + li] = nb2_l;
+    vec[3 * D + li] = __builtin_amdgcn_rcpf(alpha);
+    wave_sync();
+    v16f M[NI];
+#pragma unroll
+    for (int I = 0; I < NI; ++I)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) M[I][r] = 0.f;
+    // M = diag(-beta^2 R^{-1}) B' (-Y2')
+    product(0, [&](int kb, int i) { return rows4(NV[kb >> 1], 2 * (kb & 1) + i); }, M);
+#pragma unroll
+    for (int I = 0; I < NI; ++I)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const v4f s = rowvec(2, I, i);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) M[I][4 * i + r] *= s[r];
+      }
+    // Y1' <- A^{-1} (Y1' + B M)
+    product(1, [&](int kb, int i) { return rows4(M[kb >> 1], 2 * (kb & 1) + i); }, Y1);
+    v16f P[NI];
+#pragma unroll
+    for (int I = 0; I < NI; ++I) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const v4f s = rowvec(3, I, i), al = rowvec(0, I, i);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          Y1[I][4 * i + r] *= s[r];
+          NV[I][4 * i + r] *= al[r];
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) P[I][r] = 0.f;
+    }
+    // -Y2' <- -A Y2' + q o (-Q (q o Y1'))
+    product(2, [&](int kb, int i) {
+      const int i4 = 2 * (kb & 1) + i;
+      return rows4(Y1[kb >> 1], i4) * rowvec(1, kb >> 1, i4);
+    }, P);
+#pragma unroll
+    for (int I = 0; I < NI; ++I)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const v4f s = rowvec(1, I, i);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) NV[I][4 * i + r] = fmaf(s[r], P[I][4 * i + r], NV[I][4 * i + r]);
+      }
+    // columns of Y-hat (rows of Y, which leave Y1^{-1} Y2 unchanged) rescaled by powers of 2
+    if ((T - 1 - t) % TTC_SYM_RENORM == TTC_SYM_RENORM - 1) {
+      float mk = 0.f;
+#pragma unroll
+      for (int I = 0; I < NI; ++I)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mk = maxnan(mk, absmax(Y1[I][r], NV[I][r]));
+      mk = maxnan(mk, lane_read(mk, (lane ^ 32) << 2));
+      const int e = 1 - __builtin_amdgcn_frexp_expf(mk);  // m * 2^e in [1, 2)
+#pragma unroll
+      for (int I = 0; I < NI; ++I)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          Y1[I][r] = __builtin_amdgcn_ldexpf(Y1[I][r], e);
+          NV[I][r] = __builtin_amdgcn_ldexpf(NV[I][r], e);
+        }
+    }
+  }
+
+  // ---- final solve: -V_1 = Y1^{-1} (-Y2) by pivoted Gauss-Jordan, in the row layout (the first
+  // wave of each pair, D lanes per problem), and the certificate --------------------------------
+  float* region = sm + pb * G::REG;             // my problem's rows
+  const bool solver = (wv & 1) == 0;            // one wave per pair
+  const int spb = (wv >> 1) * RPP + lane / D;   // my lanes' problem in the row layout
+  float* sreg = sm + spb * G::REG;
+  const bool svalid = spb < PB && head0 + spb < H;
+  const int64_t spid = n * H + (svalid ? head0 + spb : H - 1);
+  float aug[G::AUGW];
+#pragma unroll
+  for (int mtx = 0; mtx < 2; ++mtx) {
+    __syncthreads();  // the operands / the previous rows have been read
+    const v16f(&X)[NI] = mtx == 0 ? Y1 : NV;    // column m of Y-hat = row m of Y
+#pragma unroll
+    for (int I = 0; I < NI; ++I)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        st4(region + (32 * ch + l31) * LDX + 32 * I + 8 * i + 4 * hh, rows4(X[I], i));
+    __syncthreads();
+    if (solver) {
+      float row[D];
+      ld_row<D>(sreg + li * LDX, row);
+#pragma unroll
+      for (int k = 0; k < D; ++k) aug[mtx * D + k] = row[k];
+    }
+  }
+  if (solver) {
+    if constexpr (D == 32) {
+#pragma unroll
+      for (int k = 0; k < D; ++k) aug[2 * D + k] = (k == li) ? 1.0f : 0.0f;
+    }
+    float rs = 0.f;
+#pragma unroll
+    for (int k = 0; k < D; ++k) rs += fabsf(aug[k]);
+    const float n1 = dgroup_max<D>(rs);  // ||Y1||_inf
+    wave_sync();  // every row read before the pivot-row buffer (aliasing them) is written
+    float piv;
+    int pos;
+    gauss_jordan<D, G::AUGW, 8>(aug, li, sreg, piv, pos);
+    const float ip = 1.0f / piv;
+    float pn[D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) pn[k] = aug[D + k] * ip;  // row pos of -V_1
+    float n2;
+    if constexpr (D == 32) {
+      float ri = 0.f;
+#pragma unroll
+      for (int k = 0; k < D; ++k) ri += fabsf(aug[2 * D + k]);
+      n2 = dgroup_max<D>(ri * fabsf(ip));  // ||Y1^{-1}||_inf
+    } else {
+      // the spread of the pivots (the diagonal of U in Y1 = L U), ||Y1||_inf for the largest
+      n2 = dgroup_max<D>(fabsf(ip));
+    }
+    st_row<D>(sreg + pos * LDX, pn);
+    wave_sync();
+    float da = 0.f, mx = 0.f;
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+      da = fmaxf(da, fabsf(pn[k] - sreg[k * LDX + pos]));
+      mx = fmaxf(mx, fabsf(pn[k]));
+    }
+    da = dgroup_max<D>(da);
+    mx = dgroup_max<D>(mx);
+    const bool ok = (n1 * n2 <= kSymCondMax) && (da <= kSymAsymMax * mx);  // false on NaN
+    if (li == 0) okf[spb] = ok ? 1.0f : 0.0f;
+    if (li == 0 && svalid && !ok) {  // marked for the rescue pass
+      const float nan = __builtin_nanf("");
+      if (WRITE_U) u_out[spid * D] = nan;
+      else q0stash[spid * D * D] = nan;
+      if (status != nullptr) atomicOr(status, TTC_LQR_STATUS_RESCUED);
+    }
+  }
+  __syncthreads();
+
+  // ---- step 0: stash V_1, W_0 = V_1 B_0 and Quu_0 = R + B_0' W_0 on 16 x 16 tiles (fp32 matrix
+  // cores; my two tile columns J), u0 = -Quu_0^{-1} W_0' (alpha_0 h0) ----------------------------
+  const bool store = head0 + pb < H && okf[pb] != 0.0f;
+  constexpr int JW = NB / WPP;
+  const int J0 = ch * JW;
+  v4f N[NB][NB];  // -V_1, symmetrised: tile (I, J) holds rows 16 I + 4 g + r of column 16 J + c
+#pragma unroll
+  for (int I = 0; I < NB; ++I)
+#pragma unroll
+    for (int J = 0; J < NB; ++J) {
+      const v4f tr = ld4(region + (16 * J + c) * LDX + 16 * I + 4 * g);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) N[I][J][r] = 0.5f * (region[(16 * I + 4 * g + r) * LDX + 16 * J + c] + tr[r]);
+    }
+  const float al0 = fmaf(a_l, __builtin_amdgcn_exp2f(la2_l), 1.0f);
+  vec[li] = al0 * h0[pid * D + li];                // (A_0 h0)_li
+  vec[D + li] = __builtin_amdgcn_exp2f(lb2_l);     // beta_0
+  wave_sync();
+  if (SM == STASH_V1 && store) {
+    float* vp = kstash + pid * D * D;
+#pragma unroll
+    for (int I = 0; I < NB; ++I)
+#pragma unroll
+      for (int J = 0; J < NB; ++J)
+        if (J >= J0 && J < J0 + JW) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) vp[(16 * I + 4 * g + r) * D + 16 * J + c] = -N[I][J][r];
+        }
+  }
+  v4f nW[NB][JW], nQ[NB][JW];
+#pragma unroll
+  for (int I = 0; I < NB; ++I)
+#pragma unroll
+    for (int jj = 0; jj < JW; ++jj) {
+      const int j = 16 * (J0 + jj) + c;
+      const float rr = 1.0f / Rinv[pid * D + j];
+      nW[I][jj] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) nQ[I][jj][r] = (16 * I + 4 * g + r == j) ? -rr : 0.0f;
+    }
+#pragma unroll
+  for (int K = 0; K < NB; ++K) {
+    float Bk[JW][4];
+#pragma unroll
+    for (int jj = 0; jj < JW; ++jj)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        Bk[jj][s] = bq[(16 * K + 4 * g + s) * D + 16 * (J0 + jj) + c] * vec[D + 16 * (J0 + jj) + c];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int jj = 0; jj < JW; ++jj) nW[I][jj] = mfma16x16x4(N[K][I][s], Bk[jj][s], nW[I][jj]);
+  }
+#pragma unroll
+  for (int K = 0; K < NB; ++K)
+#pragma unroll
+    for (int I = 0; I < NB; ++I) {
+      float Bk[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) Bk[s] = bq[(16 * K + 4 * g + s) * D + 16 * I + c] * vec[D + 16 * I + c];
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int jj = 0; jj < JW; ++jj) nQ[I][jj] = mfma16x16x4(Bk[s], nW[K][jj][s], nQ[I][jj]);
+    }
+  // y = W' A_0 h0, to the third vector slot of the problem's first wave
+  float* yv = sm + G::body(PB) + pb * WPP * G::VEC + 2 * D;
+#pragma unroll
+  for (int jj = 0; jj < JW; ++jj) {
+    float ny = 0.f;
+#pragma unroll
+    for (int I = 0; I < NB; ++I) {
+      const v4f ah = ld4(vec + 16 * I + 4 * g);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ny = fmaf(nW[I][jj][r], ah[r], ny);
+    }
+    ny += __shfl_xor(ny, 16, 64);
+    ny += __shfl_xor(ny, 32, 64);
+    if (g == 0) yv[16 * (J0 + jj) + c] = -ny;
+  }
+  __syncthreads();  // every wave has read N
+  // rows of Quu_0, the lower tiles mirrored from the upper ones
+#pragma unroll
+  for (int I = 0; I < NB; ++I)
+#pragma unroll
+    for (int jj = 0; jj < JW; ++jj) {
+      const int J = J0 + jj;
+      if (I > J) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float x = -nQ[I][jj][r];
+        region[(16 * I + 4 * g + r) * LDX + 16 * J + c] = x;
+        if (I < J) region[(16 * J + c) * LDX + 16 * I + 4 * g + r] = x;
+      }
+    }
+  __syncthreads();
+  if (!solver) return;
+  float row[D + 4];
+  ld_row<D>(sreg + li * LDX, *reinterpret_cast<float(*)[D]>(row));
+  row[D] = sm[G::body(PB) + spb * WPP * G::VEC + 2 * D + li];
+  row[D + 1] = row[D + 2] = row[D + 3] = 0.f;
+  const bool sstore = svalid && okf[spb] != 0.0f;
+  if (SM == STASH_V1 && sstore)
+    st_global_row<D>(q0stash + (spid * D + li) * D, *reinterpret_cast<float(*)[D]>(row));
+  wave_sync();  // all rows read before the pivot-row buffer (aliasing them) is written
+  float piv;
+  int pos;
+  gauss_jordan<D, D + 4, (D + 4) % 8 == 0 ? 8 : 4, D + 1>(row, li, sreg, piv, pos);
+  const float u0 = -row[D] / piv;
+  if (sstore) {
+    if (WRITE_U) u_out[spid * D + pos] = u0;
+    if (status != nullptr && !isfinite(u0)) atomicOr(status, TTC_LQR_STATUS_NONFINITE);
+  }
+}
+
+// Workgroups of PB heads of one token.  At d = 64 two problems (four waves) share one copy of the
+// operands and two workgroups fill a CU; at d = 32 up to eight, the largest count that leaves no
+// or few idle waves.
+template <int D>
+inline int symw_heads(int H) {
+  constexpr int M = SymW<D>::MAXPB;
+  const int n = (H + M - 1) / M;
+  return (H + n - 1) / n;
+}
+
+template <int D, int SM, bool WU>
+inline void launch_symw(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
+                        const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T,
+                        float* u, float* st_a, float* st_b, int32_t* status, hipStream_t s) {
+  const int PB = symw_heads<D>(H);
+  const int64_t blocks = P / H * ((H + PB - 1) / PB);
+  hipLaunchKernelGGL((lqr_symw_kernel<D, SM, WU>), dim3((unsigned)blocks), dim3(64 * SymW<D>::WPP * PB),
+                     SymW<D>::lds_bytes(PB), s, A, B, Q, R, Qf, lA, lB, lQ, h0, H, T, PB, u, st_a, st_b, status);
+}
+
+}  // namespace ttc
