@@ -282,12 +282,12 @@ def test_wide_symplectic_stress(d, H, T):
                precision="fp32")
 
 
-@pytest.mark.parametrize("d", [64])
+@pytest.mark.parametrize("d", [32, 64])
 @pytest.mark.parametrize("N,H,T", [(1, 1, 1), (5, 1, 10), (3, 3, 17), (2, 5, 9), (1, 9, 24), (2, 12, 2)])
 @pytest.mark.parametrize("stash", ["always", "never"])
 def test_wide_symplectic_any_head_count(d, N, H, T, stash):
     """The wide symplectic sweep at head counts that leave idle waves in its workgroups (two heads at
-    d = 64, up to eight at d = 32), at the ends of its renormalisation and refresh intervals, with
+    d = 64, up to four at d = 32), at the ends of its renormalisation and refresh intervals, with
     and without a stash; the second input set is barely discounted with spread scales, so that its
     rescue pass runs at those head counts too."""
     ins = bench_solver_inputs(N, H, d, seed=d + N + H + T)

@@ -17,7 +17,7 @@ SOURCES = ["ttc_lqr_capi.hip", "ttc_lqr_d16.hip", "ttc_lqr_d16_mfma.hip", "ttc_l
            "ttc_lqr_d32_mfma.hip", "ttc_lqr_d64_mfma.hip", "ttc_lqr_d16_sym.hip",
            "ttc_lqr_factored.hip", "ttc_lqr_d16_ham.hip", "ttc_lqr_d32_ham.hip", "ttc_lqr_d64_ham.hip",
            "ttc_lqr_epilogue.hip", "ttc_lqr_stash.hip", "ttc_lqr_noalloc.hip", "ttc_lqr_d16_f64.hip",
-           "ttc_lqr_d64_symw.hip"]
+           "ttc_lqr_d64_symw.hip", "ttc_lqr_d32_symw.hip"]
 HOST_SOURCES = ["ttc_lqr_host.cpp"]  # CPU code (no GPU kernels): compiled by the host compiler
 ARCH = os.environ.get("TTC_LQR_ARCH", "gfx950")
 
@@ -31,7 +31,8 @@ HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
 # of routing every product through an AGPR tile and back (at one wave per SIMD their registers are
 # full; the symplectic step's loop falls from 489 to 321 instructions, with no accumulator moves).
 # So do the split sweeps, whose accumulators are the next product's operands.
-EXTRA_FLAGS = {s: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for s in ("ttc_lqr_d16_f64.hip", "ttc_lqr_d64_symw.hip")}
+EXTRA_FLAGS = {s: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
+               for s in ("ttc_lqr_d16_f64.hip", "ttc_lqr_d64_symw.hip", "ttc_lqr_d32_symw.hip")}
 
 
 def _run(cmd, verbose):

@@ -239,8 +239,9 @@ static bool fp64_rollout(int flags, int d) {
 
 // Flags of a forward sweep (stash mode sm): TTC_LQR_FLAG_FP64_FALLBACK's forward is
 // TTC_LQR_FLAG_FP64_RESCUE's -- the fp32 symplectic sweep with its rejected problems recomputed in
-// fp64, and the stable path's gains in fp64 -- except at d = 32 with an odd head count, which has
-// no symplectic sweep to certify and keeps the fp32 Riccati-step tiers for u and the stash.
+// fp64, and the stable path's gains in fp64 -- except at d = 32 with an odd head count, whose
+// rejected problems take the fp32 tiers for u and the stash (TTC_LQR_FLAG_FP64_RESCUE itself sweeps
+// every problem of an odd head count in fp64 there).
 static int forward_flags(int flags, int d, int H, int sm) {
   if (!(flags & TTC_LQR_FLAG_FP64_FALLBACK)) return flags;
   flags &= ~TTC_LQR_FLAG_FP64_FALLBACK;

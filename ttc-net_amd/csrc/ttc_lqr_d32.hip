@@ -8,9 +8,9 @@ int launch_fwd_d32(const float* A, const float* B, const float* Q, const float* 
                   float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s, int flags,
                   int32_t* rescue_ws) {
   // fp32 sweeps without per-step gains run on the matrix cores unless the row-layout kernel
-  // is asked for: the certified symplectic sweep by default (even head counts), per-step
-  // Riccati when asked for
-  // fp64 rescue of a symplectic sweep (even head counts); otherwise fp64 throughout
+  // is asked for: the certified symplectic sweep by default, per-step Riccati when asked for.
+  // fp64 rescue of a symplectic sweep at even head counts; odd ones, per-step Riccati and the
+  // row-layout kernel run fp64 throughout
   if ((flags & TTC_LQR_FLAG_FP64_RESCUE) &&
       (sm == STASH_GAINS || (flags & (TTC_LQR_FLAG_ROW_KERNEL | TTC_LQR_FLAG_RICCATI_STEPS)) || H % 2 != 0))
     flags |= TTC_LQR_FLAG_FP64_RICCATI;

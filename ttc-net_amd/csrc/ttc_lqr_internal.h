@@ -53,8 +53,11 @@ int launch_fwd_d32_mfma(const float* A, const float* B, const float* Q, const fl
                         const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H,
                         int T, float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s,
                         bool sym, bool fp64_rescue, int32_t* rescue_ws = nullptr);
-// the certified symplectic sweep of d = 64 (ttc_lqr_symw.hpp), any head count; rejected problems
+// the certified symplectic sweeps of d = 32 / 64 (ttc_lqr_symw.hpp), any head count; rejected problems
 // are left with the NaN marker
+int launch_symw_d32(const float* A, const float* B, const float* Q, const float* R, const float* Qf, const float* lA,
+                    const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T, float* u, float* st_a,
+                    float* st_b, int sm, int32_t* status, hipStream_t s);
 int launch_symw_d64(const float* A, const float* B, const float* Q, const float* R, const float* Qf, const float* lA,
                     const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T, float* u, float* st_a,
                     float* st_b, int sm, int32_t* status, hipStream_t s);

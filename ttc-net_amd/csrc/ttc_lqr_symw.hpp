@@ -8,7 +8,7 @@
 // problem at d = 32, half of one at d = 64 -- and no wave waits for another inside the loop.  32
 // columns let one 32 x 32 x 16 instruction read each A operand once (half the LDS traffic of 16
 // columns, which at d = 64 would be as long as the matrix work), and hold the state of a wave in
-// 64 registers at d = 64 (32 at d = 32), so two waves share a SIMD there (three at d = 32).
+// 64 registers at d = 64 (32 at d = 32), so two waves share a SIMD there (four at d = 32).
 // The A operands B', B and -sym(Q) are the token's, the same for every head: split once into LDS
 // (72 KB at d = 64, 18 KB at d = 32), in the order a lane reads them (16 bytes per lane and part).
 //
@@ -24,6 +24,10 @@
 // 5.64e7) gave the same time.  47.1 -> 30.5 ms there against the fp32 matrix cores (90 % of their
 // peak); 256 problems 1.65 -> 0.66 ms; one head (1,024 problems), which ran Riccati steps, 3.87 ->
 // 1.75 ms.
+// At d = 32 the matrix cores (36 instructions of 34 cycles per problem-step) and the vector ALU (375
+// instructions) bound it together, and the waves to overlap them decide: 131,072 problems x 256 steps
+// 36.8 ms with two waves per SIMD (workgroups of 8 waves), 30.6 with three of 4 waves, 29.4 with
+// four, 29.6 with five; 48.5 ms on the fp32 matrix cores.
 #pragma once
 #include "ttc_lqr_mfma_blk.hpp"
 #include "ttc_lqr_split.hpp"
@@ -38,13 +42,13 @@ struct SymW {
   static constexpr int NB = D / 16;    // 16 x 16 tiles per dimension (step 0)
   static constexpr int WPP = D / 32;   // waves per problem
   static constexpr int RPP = 64 / D;   // problems per pair of waves (row layout: 64 lanes, D rows each)
-  static constexpr int MAXPB = D == 64 ? 2 : 8;  // problems per workgroup
+  static constexpr int MAXPB = D == 64 ? 2 : 4;  // problems per workgroup
   static constexpr int LDX = D + kPad;
   static constexpr int REG = D * LDX;  // per problem, after the sweep: D rows
   static constexpr int FRAG = 9 * NI * NK * 256;  // floats of the split operands [matrix][part][I][kb][lane]
   static constexpr int VEC = 4 * D;    // per wave: alpha, q, -beta^2 R^{-1}, 1 / alpha
   static constexpr int AUGW = D == 32 ? 3 * D : 2 * D;  // final solve: [Y1 | -Y2 | I] (d = 64: no identity)
-  static constexpr int MINW = D == 32 ? 3 : 2;     // waves per SIMD the registers must allow
+  static constexpr int MINW = D == 32 ? 4 : 2;     // waves per SIMD the registers must allow
   static_assert(REG >= AUGW + 4, "pivot row fits a problem's region");
   // problems of a workgroup rounded up to whole pairs of waves
   __host__ __device__ static constexpr int regions(int PB) { return (PB + RPP - 1) / RPP * RPP; }
@@ -453,9 +457,9 @@ lqr_symw_kernel(const float* __restrict__ A_diag, const float* __restrict__ Bg, 
   }
 }
 
-// Workgroups of PB heads of one token.  At d = 64 two problems (four waves) share one copy of the
-// operands and two workgroups fill a CU; at d = 32 up to eight, the largest count that leaves no
-// or few idle waves.
+// Workgroups of PB heads of one token, four waves: two problems at d = 64, where two workgroups'
+// copies of the operands fill a CU's LDS, up to four at d = 32 (eight measured 1.5 % slower, two
+// 0.5 %), evened out over the token's workgroups.
 template <int D>
 inline int symw_heads(int H) {
   constexpr int M = SymW<D>::MAXPB;
