@@ -1,0 +1,89 @@
+"""The layer's front-end kernel (``ttc_lqr_front_end`` / ``_backward``) against the same formulas as torch
+operators in 64 bits, and the layer's route through it."""
+import ctypes
+
+import pytest
+import torch
+
+from ttc.layers.front_end import front_end, front_end_torch
+
+# (tokens, heads, d, du, b_rank, q_rank): one wave's width and its neighbours, ranks beyond it, no rank
+SHAPES = [(1, 1, 1, 1, 1, 1), (3, 2, 16, 16, 16, 16), (5, 3, 63, 20, 65, 7), (2, 8, 64, 64, 32, 64), (4, 1, 65, 3, 0, 130),
+          (33, 5, 24, 20, 8, 33)]
+
+
+def _proj(N, H, d, du, rb, rq, dtype, device):
+    g = torch.Generator().manual_seed(N + d)
+    x = torch.randn(N, (3 * d + 2 * du + rq + 1) * H + rb + rq, generator=g) * 4.0
+    x[0, ::7] = 25.0   # softplus is the identity above 20
+    x[-1, ::5] = -40.0  # and underflows; R is clamped at 1e-6
+    if N > 2:
+        x[1] = 0.0
+    return x.to(device=device, dtype=dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_front_end_kernel(shape, with_bias):
+    """Values and gradients, relative to each output's largest entry: a sum of n squares in fp32, a
+    reciprocal root, exp and log1p leave at most (n / 2 + 10) 2^-24 of it."""
+    N, H, d, du, rb, rq = shape
+    dims = (H, d, du, rb, rq)
+    tol = (max(d, du, rb, rq) / 2 + 10) * 2.0 ** -24 * 4
+    a = _proj(*shape, torch.float32, "cuda").requires_grad_(True)
+    b = a.detach().double().cpu().requires_grad_(True)
+    bias = torch.linspace(-2, 1, 1 + du + d) if with_bias else None
+    ba = None if bias is None else bias.cuda().requires_grad_(True)
+    bb = None if bias is None else bias.double().requires_grad_(True)
+    ya, yb = front_end(a, ba, dims), front_end_torch(b, bb, dims)
+    g = torch.Generator().manual_seed(9)
+    # (R's clamp is a step in its gradient: entries within rounding of it are left out)
+    ws = [torch.randn(y.shape, generator=g, dtype=torch.float64) for y in yb]
+    ws[3] = ws[3] * ((yb[3].detach() - 1e-6).abs() > 1e-9)
+    ins_a, ins_b = [a] + ([ba] if with_bias else []), [b] + ([bb] if with_bias else [])
+    ga = torch.autograd.grad([(y * w.float().cuda()).sum() for y, w in zip(ya, ws)], ins_a)
+    gb = torch.autograd.grad([(y * w).sum() for y, w in zip(yb, ws)], ins_b)
+    # l2norm in front_end_torch works in fp32 whatever the input; redo it in 64 bits for the bound
+    for x, y in list(zip(ya, yb)) + list(zip(ga, gb)):
+        assert x.is_contiguous() and x.shape == y.shape
+        if y.numel():
+            scale = max(float(y.detach().abs().max()), 1e-30)
+            assert float((x.detach().double().cpu() - y.detach()).abs().max()) <= 2 * tol * scale + 1e-12
+
+
+@pytest.mark.gpu
+def test_front_end_second_derivative_and_partial_gradients():
+    """Under create_graph the backward is differentiable, as the operators' is; outputs without a
+    gradient count as zero."""
+    dims = (2, 6, 5, 3, 4)
+    a = _proj(3, *dims, torch.float32, "cuda").requires_grad_(True)
+    b = a.detach().clone().requires_grad_(True)
+    for t, f in ((a, front_end), (b, front_end_torch)):
+        y = f(t, None, dims)
+        (g,) = torch.autograd.grad((y[3] ** 2).sum() + (y[0] * 3).sum(), t, create_graph=True)
+        t.first = g.detach()
+        (t.second,) = torch.autograd.grad((g ** 2).sum(), t)
+    assert torch.allclose(a.first, b.first, rtol=1e-4, atol=1e-6)
+    assert torch.allclose(a.second, b.second, rtol=1e-3, atol=1e-6)
+    (p,) = torch.autograd.grad(front_end(a, None, dims)[8].sum(), a)
+    assert float(p.sum()) == 3 * 2 * 6
+
+
+def test_front_end_argument_validation():
+    from ttc.solvers._lib import lib
+    p = ctypes.c_void_p(16)
+    assert lib.ttc_lqr_front_end(p, None, 0, 1, 4, 4, 2, 2, *[p] * 9, None) == 0      # nothing to do
+    assert lib.ttc_lqr_front_end(None, None, 1, 1, 4, 4, 2, 2, *[p] * 9, None) == 1
+    assert lib.ttc_lqr_front_end(p, None, 1, 0, 4, 4, 2, 2, *[p] * 9, None) == 1
+    assert lib.ttc_lqr_front_end(p, None, 1, 1, 4, 4, 2, 2, *[p] * 8, None, None) == 1
+    assert lib.ttc_lqr_front_end_backward(p, 1, 1, 4, 4, 2, 2, *[p] * 9, None, None) == 1
+    assert lib.ttc_lqr_front_end_backward(p, 0, 1, 4, 4, 2, 2, *[None] * 9, None, None) == 0
+
+
+def test_cpu_and_other_dtypes_use_the_operators():
+    dims = (2, 6, 5, 3, 4)
+    for dt in (torch.float32, torch.bfloat16):
+        x = _proj(2, *dims, dt, "cpu")
+        for u, v in zip(front_end(x, None, dims), front_end_torch(x, None, dims)):
+            assert u.dtype == dt and torch.equal(u, v)

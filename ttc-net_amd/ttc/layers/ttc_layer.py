@@ -7,7 +7,8 @@ holds the gfx950 HIP solver under ``"hip"`` and the reference's keys ``"fused"``
 HIP solver), ``"riccati"`` and ``"kkt"`` (HIP kernels on CUDA tensors, the library's native
 host solver on CPU tensors, so the layer runs without a GPU).  The front-end (projections, ``l2norm``, softplus and
 the low-rank ``B``/``Q``/``Q_f`` mixtures) and the back-end (rescale, ``out_proj``)
-are ordinary torch ops around that call.
+are ordinary torch ops around that call, except that fp32 CUDA projections are split and
+normalised by one kernel each way (:mod:`ttc.layers.front_end`).
 
 With ``factored=True`` (the default wherever the solver has a factored form,
 ``LQR_FACTORED_IMPL_MAP``) the layer hands the solver the mixture coefficients and
@@ -35,8 +36,8 @@ import math
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
+from .front_end import front_end, l2norm
 from ..solvers.fused_lqr import fused_lqr_solve
 from ..solvers.hip_lqr import hip_lqr_solve, hip_lqr_solve_factored
 from ..solvers.torch_lqr import direct_lqr_solve, kkt_lqr_solve
@@ -56,11 +57,6 @@ LQR_FACTORED_IMPL_MAP = {
     "hip": hip_lqr_solve_factored,
     "fused": hip_lqr_solve_factored,
 }
-
-
-def l2norm(x: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:
-    xf = x.float()
-    return (xf * torch.rsqrt((xf * xf).sum(-1, keepdim=True) + eps)).to(x.dtype)
 
 
 class TTCLayer(nn.Module):
@@ -117,24 +113,14 @@ class TTCLayer(nn.Module):
     def _front_end(self, x: torch.Tensor):
         """Projections, normalisations and discounts (``ttc_layer.py:104-135``) up to the
         low-rank mixtures: per-token coefficients, the bases they mix, the per-head inputs."""
-        H, hd, ud, qr = self.num_heads, self.h_dim, self.u_dim, self.q_rank
-        xt = x.reshape(-1, self.in_dim)
-        heads, coeff_B, coeff_Q = torch.split(self.in_proj(xt), [sum(self._head_split) * H, self.b_rank, qr], dim=-1)
-        h0, A_diag, R_inv_diag, coeff_Qf, log_gammas = torch.split(
-            heads.reshape(-1, H, sum(self._head_split)), self._head_split, dim=-1)
-        A_diag = l2norm(A_diag)
-        coeff_B, coeff_Q, coeff_Qf = l2norm(coeff_B), l2norm(F.softplus(coeff_Q)), l2norm(F.softplus(coeff_Qf))
+        A_diag, coeff_B, coeff_Q, R_inv_diag, coeff_Qf, lgA, lgB, lgQ, h0 = front_end(
+            self.in_proj(x.reshape(-1, self.in_dim)), self.bias_gamma,
+            (self.num_heads, self.h_dim, self.u_dim, self.b_rank, self.q_rank))
         if self.q_reparam == "plain":
             Q_basis = self.Qs
         else:  # "...r,rmn,rkn->...mk" / sqrt(h_dim) = sum_r coeff_r (Qs_r Qs_r') / sqrt(h_dim)
-            Q_basis = torch.matmul(self.Qs, self.Qs.transpose(1, 2)) / math.sqrt(hd)
-        R_inv_diag = torch.clamp(l2norm(F.softplus(R_inv_diag)), min=1e-6)
-        if self.bias_gamma is not None:
-            log_gammas = -F.softplus(log_gammas) - F.relu(-self.bias_gamma[None, None, :])
-        else:
-            log_gammas = -F.softplus(log_gammas)
-        lgA, lgB, lgQ = torch.split(log_gammas, [1, ud, hd], dim=-1)
-        return A_diag, coeff_B, coeff_Q, R_inv_diag, coeff_Qf, lgA.squeeze(-1), lgB, lgQ, h0, Q_basis
+            Q_basis = torch.matmul(self.Qs, self.Qs.transpose(1, 2)) / math.sqrt(self.h_dim)
+        return A_diag, coeff_B, coeff_Q, R_inv_diag, coeff_Qf, lgA, lgB, lgQ, h0, Q_basis
 
     def solver_inputs(self, x: torch.Tensor):
         """Front-end (``ttc_layer.py:104-135``): ``x [..., in_dim]`` -> the nine solver inputs."""

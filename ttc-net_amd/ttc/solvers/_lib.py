@@ -93,6 +93,10 @@ def _load():
     L.ttc_lqr_rescale.argtypes = [f32p, f32p, i64, i32, i32, i32, i32, f32p, ctypes.c_void_p]
     L.ttc_lqr_rescale_backward.restype = ctypes.c_int
     L.ttc_lqr_rescale_backward.argtypes = [f32p, f32p, f32p, i64, i32, i32, i32, i32, f32p, ctypes.c_void_p]
+    L.ttc_lqr_front_end.restype = ctypes.c_int
+    L.ttc_lqr_front_end.argtypes = [f32p, f32p, i64, i32, i32, i32, i32, i32] + [f32p] * 9 + [ctypes.c_void_p]
+    L.ttc_lqr_front_end_backward.restype = ctypes.c_int
+    L.ttc_lqr_front_end_backward.argtypes = [f32p, i64, i32, i32, i32, i32, i32] + [f32p] * 10 + [ctypes.c_void_p]
     L.ttc_lqr_noalloc_scratch_bytes.restype = sz
     L.ttc_lqr_noalloc_scratch_bytes.argtypes = []
     L.ttc_lqr_backward_noalloc.restype = ctypes.c_int
