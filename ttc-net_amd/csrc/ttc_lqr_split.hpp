@@ -65,13 +65,28 @@ __device__ __forceinline__ Split8 split8(const v4f x, const v4f y) {
                 __builtin_bit_cast(v8bf, v4u{l[0], l[1], l[2], l[3]})};
 }
 
-// acc[I] += A_I B over 16 k (32 x 32 tiles), the small terms first; the accumulators of one term
-// are independent.
-template <int NI>
-__device__ __forceinline__ void mfma32_split(const Split8 (&a)[NI], const Split8& b, v16f (&acc)[NI]) {
+// CW x CW tiles (16 or 32): the accumulator of a lane, and the matrix instruction over 16 k (CW = 32)
+// or 32 k (CW = 16).
+template <int CW> struct SplitTile;
+template <> struct SplitTile<32> {
+  using T = v16f;
+  static __device__ __forceinline__ T mfma(v8bf a, v8bf b, T c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+  }
+};
+template <> struct SplitTile<16> {
+  using T = v4f;
+  static __device__ __forceinline__ T mfma(v8bf a, v8bf b, T c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+};
+
+// acc[I] += A_I B, the small terms first; the accumulators of one term are independent.
+template <int CW, int NI>
+__device__ __forceinline__ void mfma_split(const Split8 (&a)[NI], const Split8& b, typename SplitTile<CW>::T (&acc)[NI]) {
   auto term = [&](auto&& x, const v8bf& y) {
 #pragma unroll
-    for (int I = 0; I < NI; ++I) acc[I] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x(a[I]), y, acc[I], 0, 0, 0);
+    for (int I = 0; I < NI; ++I) acc[I] = SplitTile<CW>::mfma(x(a[I]), y, acc[I]);
   };
   term([](const Split8& v) { return v.lo; }, b.hi);
   term([](const Split8& v) { return v.hi; }, b.lo);
