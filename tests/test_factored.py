@@ -395,3 +395,30 @@ def test_bf16_storage_against_oracle(cfg, n_tok):
           flush=True)
     bad = {k: v for k, v in errs.items() if not (v <= BF16_TOL)}
     assert not bad, f"bf16 cfg{cfg}: rel err above {BF16_TOL}: {bad}"
+
+
+@pytest.mark.parametrize("cfg,N", [(4, 75), (3, 75)])
+def test_last_chunk_takes_the_call_s_kernel(cfg, N, monkeypatch):
+    """A workspace that leaves a last chunk small enough for the narrow form of the wide symplectic sweep
+    (2,400 / 1,200 problems, the last 3 tokens apart): the form follows the whole call, so u and the
+    gradients equal those of one pass bit for bit (the basis gradients: their sums run per chunk)."""
+    from ttc.solvers._lib import lib
+    from ttc.solvers.hip_lqr import hip_lqr_solve_factored, riccati_flags
+    ins = factored_inputs(cfg, N)
+    dev = torch.device("cuda:0")
+    T, d, H = 9, ins[0].shape[-1], ins[0].shape[1]
+    rb, rq = ins[9].shape[0], ins[10].shape[0]
+    dU = torch.randn(N, H, d, device=dev, generator=torch.Generator(device=dev).manual_seed(4))
+
+    def run():
+        xs = [t.to(dev).float().requires_grad_(True) for t in ins]
+        u = hip_lqr_solve_factored(*xs, T, stash="never")
+        (u * dU).sum().backward()
+        return [u.detach()] + [x.grad for x in xs[:9]]
+
+    whole = run()
+    flags = riccati_flags("auto", T, d)
+    need = max(lib.ttc_lqr_factored_workspace_bytes(N - 3, H, d, d, rb, rq, T, 0, k, 0, flags) for k in (0, 1))
+    monkeypatch.setenv("TTC_LQR_WORKSPACE_BYTES", str(need))
+    for a, b in zip(whole, run()):
+        assert torch.equal(a, b)

@@ -302,6 +302,21 @@ def test_wide_symplectic_any_head_count(d, N, H, T, stash):
                    grad_limit=math.inf, stash=stash, precision="fp32")
 
 
+@pytest.mark.parametrize("N,H,T", [(1, 1, 1), (3, 3, 9), (7, 5, 17), (2, 8, 2), (1025, 2, 9), (683, 3, 9), (600, 6, 10),
+                                   (1100, 4, 9), (4099, 1, 9), (821, 5, 10)])
+def test_d16_symplectic_problems_per_wave(N, H, T):
+    """The d = 16 sweep with one (up to 2,048 problems, odd heads 4,096), two (even heads up to 4,096) and
+    four problems a wave, of one token (H % 4 == 0) or consecutive ones, with idle slots in the last
+    wave, at the ends of its renormalisation and refresh intervals; a part of the problems barely
+    discounted with spread scales, so that certificates and rescue meet every form."""
+    ins = bench_solver_inputs(N, H, 16, seed=N + H + T)
+    A_diag, B, Q, R_inv, Qf, lgA, lgB, lgQ, h0 = ins
+    R_inv[::7] = R_inv[::7] * 30.0
+    for lg in (lgA, lgB, lgQ):
+        lg[::7] = lg[::7] * 0.02
+    check_case(f"ppw N={N} H={H}", ins, T, grad_limit=math.inf, precision="fp32", tol=1e-4)
+
+
 @pytest.mark.parametrize("cfg,T,seed", [(5, 64, 5), (5, 1024, 5), ("5b", 1024, 55), (5, 2048, 7), ("5b", 2048, 57)])
 def test_config5_stress(cfg, T, seed):
     """Config 5 / 5b share the layer and the log-normal token scales; 5b draws its own tokens

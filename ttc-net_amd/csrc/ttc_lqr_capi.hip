@@ -272,9 +272,11 @@ static StableLayout stable_layout(int64_t chunk_tokens, int H, int d, int T, boo
   return L;
 }
 
+// call: the problems of the whole call, of which these P may be a chunk (its choice of kernel must not
+// depend on the chunk, or a token's last bits would depend on where the chunks end).
 static int fwd_d(int d, const float* a, const float* b, const float* q, const float* r, const float* qf,
                  const float* la, const float* lb, const float* lq, const float* hz, int64_t P, int H, int T, float* u,
-                 float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s, int flags,
+                 float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s, int flags, int64_t call,
                  int32_t* rescue_ws = nullptr, RescueSlots rs = RescueSlots{}) {
   flags = forward_flags(flags, d, H, sm);
   switch (d) {
@@ -282,9 +284,10 @@ static int fwd_d(int d, const float* a, const float* b, const float* q, const fl
       return launch_fwd_d16(a, b, q, r, qf, la, lb, lq, hz, P, H, T, u, st_a, st_b, sm, status, s, flags, rescue_ws,
                             rs);
     case 32:
-      return launch_fwd_d32(a, b, q, r, qf, la, lb, lq, hz, P, H, T, u, st_a, st_b, sm, status, s, flags, rescue_ws);
+      return launch_fwd_d32(a, b, q, r, qf, la, lb, lq, hz, P, H, T, u, st_a, st_b, sm, status, s, flags, call,
+                            rescue_ws);
     case 64:
-      return launch_fwd_d64(a, b, q, r, qf, la, lb, lq, hz, P, H, T, u, st_a, st_b, sm, status, s, flags, rescue_ws);
+      return launch_fwd_d64(a, b, q, r, qf, la, lb, lq, hz, P, H, T, u, st_a, st_b, sm, status, s, flags, call);
   }
   return TTC_LQR_EUNSUPPORTED;
 }
@@ -324,7 +327,7 @@ static int stable_backward(const float* A, const float* B, const float* Q, const
     int64_t sw = Pc;  // problems of this chunk that the sweep takes (the leading ones)
     if (gidx != nullptr && nsweep >= 0) sw = nsweep <= p0 ? 0 : (nsweep - p0 < Pc ? nsweep - p0 : Pc);
     if (sw > 0) {
-      rc = fwd_d(d, a, b, q, r, qf, la, lb, lq, hz, sw, H, T, nullptr, kst, q0s, kStashGains, nullptr, s, flags);
+      rc = fwd_d(d, a, b, q, r, qf, la, lb, lq, hz, sw, H, T, nullptr, kst, q0s, kStashGains, nullptr, s, flags, sw);
       if (rc != TTC_LQR_OK) return rc;
     }
     void* traj = ws + L.traj;
@@ -499,7 +502,8 @@ static Compact compact_at(char* base, int64_t F64, int d, int du) {
 // Gradients of n_tokens tokens (inputs already validated), token chunk by token chunk
 // inside ws: the certified Hamiltonian rollout with its per-problem fallback, or the
 // stable path for every problem under TTC_LQR_FLAG_STABLE_BWD.  v1s / q0s: the forward's
-// stash halves (V_1 [P,d,d], Quu_0 [P,du,du]) or null to recompute them per chunk.
+// stash halves (V_1 [P,d,d], Quu_0 [P,du,du]) or null to recompute them per chunk; call: the
+// problems of the whole call (fwd_d).
 static int backward_core(const float* A_diag, const float* B, const float* Q, const float* R_inv, const float* Q_f,
                          const float* log_gamma_A, const float* log_gamma_B, const float* log_gamma_Q,
                          const float* h0, const float* u, const float* d_u, int64_t n_tokens, int H, int d, int du,
@@ -507,7 +511,7 @@ static int backward_core(const float* A_diag, const float* B, const float* Q, co
                          float* grad_Q, float* grad_R_inv, float* grad_Q_f, float* grad_log_gamma_A,
                          float* grad_log_gamma_B, float* grad_log_gamma_Q, float* grad_h0, char* ws,
                          size_t workspace_bytes, float grad_limit, int32_t* status, int64_t* n_fallback,
-                         hipStream_t s, RescueSlots rs = RescueSlots{}) {
+                         hipStream_t s, int64_t call, RescueSlots rs = RescueSlots{}) {
   const bool fp64 = fp64_stable(flags, d);
   if (flags & TTC_LQR_FLAG_STABLE_BWD) {
     if (n_fallback) *n_fallback = n_tokens * H;
@@ -556,7 +560,7 @@ static int backward_core(const float* A_diag, const float* B, const float* Q, co
     } else {
       float* v1w = reinterpret_cast<float*>(ws + L.v1);
       float* q0w = reinterpret_cast<float*>(ws + L.q0);
-      rc = fwd_d(d, a, b, q, r, qf, la, lb, lq, hz, Pc, H, T, nullptr, v1w, q0w, kStashV1, nullptr, s, flags);
+      rc = fwd_d(d, a, b, q, r, qf, la, lb, lq, hz, Pc, H, T, nullptr, v1w, q0w, kStashV1, nullptr, s, flags, call);
       if (rc != TTC_LQR_OK) return rc;
       v1 = v1w;
       q0 = q0w;
@@ -1022,7 +1026,7 @@ static int forward_factored(const TS* A_diag, const TS* coeff_B, const TS* coeff
     }
     int32_t* rlist = fp64 ? reinterpret_cast<int32_t*>(ws + L.rlist) : nullptr;
     rc = fwd_d(d, a, Bx, Qx, r, Qfx, la, lb, lq, hz, nc * H, H, T, u + p0 * du, v1, q0, stash ? kStashV1 : 0, status,
-               s, flags & ~TTC_LQR_FLAG_COMPACT_STASH, rlist);
+               s, flags & ~TTC_LQR_FLAG_COMPACT_STASH, P, rlist);
     if (compact && rc == TTC_LQR_OK) rc = launch_pack_upper(v1, nc * H, d, stash + p0 * (dd + d) / 2, s);
   }
   return rc;
@@ -1124,7 +1128,7 @@ static int backward_factored(const TS* A_diag, const TS* coeff_B, const TS* coef
     int64_t nfb = 0;
     rc = backward_core(a, Bx, Qx, r, Qfx, la, lb, lq, hz, u ? u + p0 * du : nullptr, dz, nc, H, d, du, T, flags, v1,
                        q0, gA, gB, gQ, gR, gQf, glA, glB, glQ, gh, ws + L.inner, ws_bytes - L.inner, grad_limit, status,
-                       &nfb, s);  // the workspace beyond the chunk's layout widens the fallback passes
+                       &nfb, s, P);  // the workspace beyond the chunk's layout widens the fallback passes
     if (rc != TTC_LQR_OK) return rc;
     total_fb += nfb;
     // chain rule of the expansion: coefficient gradients, then the basis sums
@@ -1321,7 +1325,7 @@ int ttc_lqr_forward_ws(const float* A_diag, const float* B, const float* Q, cons
     if (rws == nullptr) rs = RescueSlots{};
   }
   return fwd_d(d, A_diag, B, Q, R_inv, Q_f, log_gamma_A, log_gamma_B, log_gamma_Q, h0, P, heads, T, u, v1, q0,
-               stash ? kStashV1 : 0, status, s, flags, rws, rs);
+               stash ? kStashV1 : 0, status, s, flags, P, rws, rs);
 }
 
 int ttc_lqr_backward(const float* A_diag, const float* B, const float* Q, const float* R_inv, const float* Q_f,
@@ -1368,7 +1372,7 @@ int backward_entry(const float* A_diag, const float* B, const float* Q, const fl
                        d, du, T, flags, v1s, q0s, grad_A_diag, grad_B, grad_Q, grad_R_inv, grad_Q_f,
                        grad_log_gamma_A, grad_log_gamma_B, grad_log_gamma_Q, grad_h0,
                        static_cast<char*>(workspace), workspace_bytes, grad_limit, status, n_fallback,
-                       reinterpret_cast<hipStream_t>(stream), rs);
+                       reinterpret_cast<hipStream_t>(stream), n_tokens * heads, rs);
 }
 
 }  // namespace ttc

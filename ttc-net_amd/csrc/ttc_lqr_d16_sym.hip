@@ -1,7 +1,7 @@
 // ttc_lqr_d16_sym.hip -- launcher of the d = du = 16 symplectic matrix-core forward kernel
 // and its rescue pass (the per-step Riccati kernel on the problems the certificate rejects, or
 // the fp64 row-layout sweep under TTC_LQR_FLAG_FP64_RESCUE).
-#include "ttc_lqr_mfma_blk.hpp"
+#include "ttc_lqr_sym16.hpp"
 
 namespace ttc {
 
@@ -10,16 +10,7 @@ static void launch_s16(const float* A, const float* B, const float* Q, const flo
                        const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T,
                        float* u, float* st_a, float* st_b, int32_t* status, hipStream_t s, bool fp64_rescue,
                        int32_t* rescue_ws, RescueSlots rs) {
-  using G = MB<16, 4, 1, true>;
-  using GT = MB<16, 4, 1, true, true>;
-  const dim3 grid((unsigned)((P + G::PPW - 1) / G::PPW)), block(G::THREADS);
-  // H % 4 == 0: the four problems of a wave are heads of one token and share its B and Q
-  if (H % 4 == 0)
-    hipLaunchKernelGGL((lqr_fwd_blk_kernel<16, 4, 1, SM, WU, true, false, true>), grid, block, GT::LDS_BYTES, s, A, B,
-                       Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status);
-  else
-    hipLaunchKernelGGL((lqr_fwd_blk_kernel<16, 4, 1, SM, WU, true>), grid, block, G::LDS_BYTES, s, A, B, Q, R, Qf,
-                       lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status);
+  launch_sym16<SM, WU>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s);
   if (fp64_rescue) {
     // long horizons: the rejected problems are the ill-conditioned ones, recomputed in fp64 --
     // listed, on the matrix cores (the LU row-layout sweep finishing any whose Cholesky breaks

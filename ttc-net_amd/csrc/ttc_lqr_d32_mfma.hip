@@ -12,7 +12,7 @@ static void launch_b32_w(const float* A, const float* B, const float* Q, const f
   using G = MB<32, PPW, WPB>;
   constexpr int PPB = PPW * WPB;
   const dim3 grid((unsigned)((P + PPB - 1) / PPB)), block(G::THREADS);
-  hipLaunchKernelGGL((lqr_fwd_blk_kernel<32, PPW, WPB, SM, WU, false, RESC>), grid, block, G::LDS_BYTES, s, A, B, Q, R,
+  hipLaunchKernelGGL((lqr_fwd_blk_kernel<32, PPW, WPB, SM, WU, RESC>), grid, block, G::LDS_BYTES, s, A, B, Q, R,
                      Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status);
 }
 
@@ -24,17 +24,17 @@ template <int SM, bool WU>
 static void launch_b32(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                        const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T,
                        float* u, float* st_a, float* st_b, int32_t* status, hipStream_t s, bool sym,
-                       bool fp64_rescue, int32_t* rescue_ws) {
+                       int64_t call, bool fp64_rescue, int32_t* rescue_ws) {
   if (fp64_rescue) {
     // long horizons: the symplectic sweep, its rejected problems recomputed by the pivoted
     // row-layout sweep in fp64
-    launch_symw_d32(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, SM, status, s);
+    launch_symw_d32(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, SM, status, s, call);
     launch_rescue_k<32, SM, WU, double>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s,
                                         rescue_ws);
     return;
   }
   if (sym) {
-    launch_symw_d32(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, SM, status, s);
+    launch_symw_d32(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, SM, status, s, call);
     // problems the certificate rejected: Riccati steps on the matrix cores first (only the
     // workgroups that hold one run), the row layout for what still breaks down
     if (H % 16 == 0)
@@ -53,20 +53,20 @@ static void launch_b32(const float* A, const float* B, const float* Q, const flo
 int launch_fwd_d32_mfma(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                         const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H,
                         int T, float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s,
-                        bool sym, bool fp64_rescue, int32_t* rescue_ws) {
+                        bool sym, int64_t call, bool fp64_rescue, int32_t* rescue_ws) {
   if (P <= 0) return TTC_LQR_OK;
   switch (sm) {
     case STASH_NONE:
-      launch_b32<STASH_NONE, true>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, sym, fp64_rescue,
-                                   rescue_ws);
+      launch_b32<STASH_NONE, true>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, sym, call,
+                                   fp64_rescue, rescue_ws);
       break;
     case STASH_V1:
       if (u != nullptr)
         launch_b32<STASH_V1, true>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, sym,
-                                   fp64_rescue, rescue_ws);
+                                   call, fp64_rescue, rescue_ws);
       else
         launch_b32<STASH_V1, false>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, sym,
-                                    fp64_rescue, rescue_ws);
+                                   call, fp64_rescue, rescue_ws);
       break;
     default:
       return TTC_LQR_EINVAL;

@@ -11,7 +11,7 @@ static void launch_b64_w(const float* A, const float* B, const float* Q, const f
                          float* u, float* st_a, float* st_b, int32_t* status, hipStream_t s) {
   using G = MB<64, 1, WPB>;
   const dim3 grid((unsigned)((P + WPB - 1) / WPB)), block(G::THREADS);
-  hipLaunchKernelGGL((lqr_fwd_blk_kernel<64, 1, WPB, SM, WU, false, RESC>), grid, block, G::LDS_BYTES, s, A, B, Q, R,
+  hipLaunchKernelGGL((lqr_fwd_blk_kernel<64, 1, WPB, SM, WU, RESC>), grid, block, G::LDS_BYTES, s, A, B, Q, R,
                      Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status);
 }
 
@@ -21,9 +21,9 @@ static void launch_b64_w(const float* A, const float* B, const float* Q, const f
 template <int SM, bool WU>
 static void launch_b64(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                        const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T,
-                       float* u, float* st_a, float* st_b, int32_t* status, hipStream_t s, bool sym) {
+                       float* u, float* st_a, float* st_b, int32_t* status, hipStream_t s, bool sym, int64_t call) {
   if (sym) {
-    launch_symw_d64(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, SM, status, s);
+    launch_symw_d64(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, SM, status, s, call);
     // problems the certificate rejected: Riccati steps on the matrix cores first (only the
     // workgroups that hold one run), the row layout for what still breaks down
     if (H % 4 == 0)
@@ -42,17 +42,17 @@ static void launch_b64(const float* A, const float* B, const float* Q, const flo
 int launch_fwd_d64_mfma(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                         const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H,
                         int T, float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s,
-                        bool sym) {
+                        bool sym, int64_t call) {
   if (P <= 0) return TTC_LQR_OK;
   switch (sm) {
     case STASH_NONE:
-      launch_b64<STASH_NONE, true>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, sym);
+      launch_b64<STASH_NONE, true>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, sym, call);
       break;
     case STASH_V1:
       if (u != nullptr)
-        launch_b64<STASH_V1, true>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, sym);
+        launch_b64<STASH_V1, true>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, sym, call);
       else
-        launch_b64<STASH_V1, false>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, sym);
+        launch_b64<STASH_V1, false>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, sym, call);
       break;
     default:
       return TTC_LQR_EINVAL;

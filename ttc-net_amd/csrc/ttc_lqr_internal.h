@@ -52,19 +52,19 @@ int launch_v1slots64_d16(const float* A, const float* B, const float* Q, const f
 int launch_fwd_d32_mfma(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                         const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H,
                         int T, float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s,
-                        bool sym, bool fp64_rescue, int32_t* rescue_ws = nullptr);
+                        bool sym, int64_t call, bool fp64_rescue, int32_t* rescue_ws = nullptr);
 // the certified symplectic sweeps of d = 32 / 64 (ttc_lqr_symw.hpp), any head count; rejected problems
-// are left with the NaN marker
+// are left with the NaN marker.  call: the problems of the whole call, which choose the kernel's form
 int launch_symw_d32(const float* A, const float* B, const float* Q, const float* R, const float* Qf, const float* lA,
                     const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T, float* u, float* st_a,
-                    float* st_b, int sm, int32_t* status, hipStream_t s);
+                    float* st_b, int sm, int32_t* status, hipStream_t s, int64_t call);
 int launch_symw_d64(const float* A, const float* B, const float* Q, const float* R, const float* Qf, const float* lA,
                     const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T, float* u, float* st_a,
-                    float* st_b, int sm, int32_t* status, hipStream_t s);
+                    float* st_b, int sm, int32_t* status, hipStream_t s, int64_t call);
 int launch_fwd_d64_mfma(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                         const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H,
                         int T, float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s,
-                        bool sym);
+                        bool sym, int64_t call);
 int launch_fwd_d16(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                   const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T,
                   float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s, int flags,
@@ -86,7 +86,7 @@ int launch_ham_d16(const float* A, const float* B, const float* Q, const float* 
 int launch_fwd_d32(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                   const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T,
                   float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s, int flags,
-                  int32_t* rescue_ws = nullptr);
+                  int64_t call, int32_t* rescue_ws = nullptr);
 int launch_bwd_d32(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                   const float* lA, const float* lB, const float* lQ, const float* h0, const float* dU,
                   const float* kst, const float* q0s, int64_t P, int H, int T, void* traj, bool fp64, float* gA,
@@ -101,7 +101,7 @@ int launch_ham_d32(const float* A, const float* B, const float* Q, const float* 
 int launch_fwd_d64(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                   const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T,
                   float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s, int flags,
-                  int32_t* rescue_ws = nullptr);
+                  int64_t call);
 int launch_bwd_d64(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                   const float* lA, const float* lB, const float* lQ, const float* h0, const float* dU,
                   const float* kst, const float* q0s, int64_t P, int H, int T, void* traj, bool fp64, float* gA,

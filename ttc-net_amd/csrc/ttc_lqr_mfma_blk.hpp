@@ -19,10 +19,8 @@
 //   N + M M' = -(V - W Quu^{-1} W'), upper tiles, one operand -> exactly symmetric
 //   N <- diag(a)(N + M M')diag(a) - diag(q) Q diag(q), lower tiles mirrored via LDS.
 // Step 0 forms W and Quu the same way and solves Quu_0 z = W_0' A_0 h0 (u0 = -z) by
-// Gauss-Jordan in the row layout (lane li owns row li): at d = 16 first without row
-// exchanges, the pivot rows broadcast by DPP (Quu_0 is positive definite for a certified
-// problem), and with partial pivoting through LDS when a pivot is not positive or wider d;
-// it also writes the compact stash V_1 / Quu_0.
+// Gauss-Jordan with partial pivoting in the row layout (lane li owns row li); it also writes
+// the stash V_1 / Quu_0.
 //
 // Multi-wave workgroups (and every d = 64 launch) keep B and -sym(Q) in LDS, shared by the
 // WPB waves of the workgroup: its WPB * PPW problems are consecutive heads of one token
@@ -37,25 +35,10 @@
 #pragma once
 #include "ttc_lqr_mfma16.hpp"
 
-#ifndef TTC_SYM_WAVES
-#define TTC_SYM_WAVES 3   // waves per SIMD of the symplectic kernel (144 VGPRs, no spills)
-#endif
-#ifndef TTC_SYM_WAVES_TOK
-#define TTC_SYM_WAVES_TOK 6  // the same with one register copy of B / Q per wave (80 VGPRs; a few
-                             // spills, none in the time loop)
-#endif
-#ifndef TTC_SYMW32_WAVES
-#define TTC_SYMW32_WAVES 3  // the d = 32 symplectic sweep in 4-wave workgroups sharing B / Q (145 VGPRs)
-#endif
-#ifndef TTC_SYM_RENORM
-#define TTC_SYM_RENORM 8  // steps between power-of-2 renormalisations of the symplectic sweep
-#endif
-
 namespace ttc {
 
-template <int D, int PPW_, int WPB_, bool SYM_ = false, bool TOK_ = false>
+template <int D, int PPW_, int WPB_>
 struct MB {
-  static constexpr bool SYM = SYM_;                 // symplectic sweep (d = 16) instead of Riccati steps
   static constexpr int NB = D / 16;                 // tiles per dimension
   static constexpr int PPW = PPW_;                  // problems per wave
   static constexpr int WPB = WPB_;                  // waves per workgroup
@@ -66,75 +49,25 @@ struct MB {
   static constexpr int NT = NB * (NB + 1) / 2;      // upper tiles (I <= J)
   static constexpr int LDX = D + kPad;              // LDS row stride of D-wide rows
   static constexpr int LDG = 20;                    // LDS row stride of a 16 x 16 tile
-  // symplectic sweep over NB x NB tiles (d = 32): its three products take B', B and -sym(Q)
-  // as A operands, read from LDS
-  static constexpr bool SYMW = SYM && D > 16;
-  // B and -sym(Q) in LDS, shared by the workgroup (d = 64 always; d = 32 with several waves
-  // or the symplectic sweep)
-  static constexpr bool BQ_LDS = D == 64 || WPB > 1 || SYMW;
-  // workgroup-shared region: [B' (column-major B) | -sym(Q) fragments], or for SYMW
-  // [B' | B (row-major) | -sym(Q) (row-major)]
-  static constexpr int OFF_BR = D * LDX;
-  static constexpr int OFF_Q = SYMW ? 2 * D * LDX : D * LDX;
-  static constexpr int SH = !BQ_LDS ? 0 : (SYMW ? 3 * D * LDX : OFF_Q + NT * 256);
+  // B and -sym(Q) in LDS, shared by the workgroup (d = 64 always; d = 32 with several waves)
+  static constexpr bool BQ_LDS = D == 64 || WPB > 1;
+  // workgroup-shared region: [B' (column-major B) | -sym(Q) fragments]
+  static constexpr int OFF_Q = D * LDX;
+  static constexpr int SH = BQ_LDS ? OFF_Q + NT * 256 : 0;
   // per-problem region: transpose buffer (CH block-rows per round), also the 16x16 tile
   // buffer and the step-0 row buffer
-  static constexpr int CH = SYMW ? 1 : (BQ_LDS ? NB / 2 : NB);
+  static constexpr int CH = BQ_LDS ? NB / 2 : NB;
   static constexpr int XROWS = CH * 16;
-  static constexpr int REG0 = XROWS * LDX;
-  // the symplectic final solve stages 16 rows of D at a time through it (Y1, then -Y2, then
-  // the solution)
-  static constexpr int REG = (SYMW && 16 * LDX > REG0) ? 16 * LDX : REG0;
-  // the final solve of the symplectic sweep works on [Y1 | -Y2 | I] (Y1^{-1} for the condition
-  // number) at d = 32; at d = 16 and 64 on [Y1 | -Y2], with the pivots' spread as the estimate
-  static constexpr bool SYM_INV = D == 32;
-  static constexpr int AUGW = SYM_INV ? 3 * D : 2 * D;
-  static_assert(REG % 4 == 0 && REG >= 16 * LDG && REG >= D + 4 && (!SYMW || REG >= AUGW + 4) &&
-                    (!SYM || SYMW || REG >= 3 * D),
-                "per-problem LDS region");
-  static_assert(!SYM || (D == 16 && !BQ_LDS) || (D >= 32 && BQ_LDS), "symplectic sweep: d = 16, or d = 32 / 64 from LDS");
-  // per-problem vectors: alpha, q (step 0: alpha*h0), beta (step 0: rhs), -beta^2 R^{-1}, 1/alpha
-  static constexpr int VEC = 5 * D;
+  static constexpr int REG = XROWS * LDX;
+  static_assert(REG % 4 == 0 && REG >= 16 * LDG && REG >= D + 4, "per-problem LDS region");
+  // per-problem vectors: alpha, q (step 0: alpha*h0), beta (step 0: rhs)
+  static constexpr int VEC = 3 * D;
   static constexpr int PER_WAVE = PPW * (REG + VEC);
   static constexpr int THREADS = 64 * WPB;
-  // two waves per SIMD, except with four problems per wave that keep B and Q in registers;
-  // the symplectic sweep's small state leaves room for four
-  // the problems of a wave belong to one token (H % PPW == 0): one register copy of B, B' and
-  // -sym(Q) for all of them
-  static constexpr bool TOK = TOK_ && !BQ_LDS;
-  static constexpr int NBQ = (BQ_LDS || TOK) ? 1 : PPW;
-  static constexpr int MINW = SYMW ? (D == 32 && WPB > 1 ? TTC_SYMW32_WAVES : 2)
-                                  : SYM ? (TOK ? TTC_SYM_WAVES_TOK : TTC_SYM_WAVES) : (PPW == 4 && !BQ_LDS) ? 1 : 2;
-  static constexpr int MAXW = MINW;
+  // two waves per SIMD, except with four problems per wave that keep B and Q in registers
+  static constexpr int MINW = (PPW == 4 && !BQ_LDS) ? 1 : 2;
   static constexpr size_t LDS_BYTES = sizeof(float) * ((size_t)SH + (size_t)WPB * PER_WAVE);
 };
-
-// Certificate of the symplectic sweep: the final solve P = Y1^{-1} Y2 is accepted when the
-// condition number of Y1 (cond_inf at d = 32; at d = 16 and 64 its estimate ||Y1||_inf / min|u_kk|
-// from the pivots of the same elimination) is <= kSymCondMax and max|P - P'| <= kSymAsymMax max|P|;
-// problems that miss it are recomputed by the rescue pass.
-constexpr float kSymCondMax = 1.0e7f;
-// steps between exact (exp2) evaluations of the symplectic sweep's discount factors; the
-// steps in between multiply the previous step's by a constant ratio
-constexpr int kSymRefresh = 8;
-constexpr float kSymAsymMax = 1.0e-6f;
-
-// max over the D lanes of a problem (D = 16, 32, 64)
-template <int D>
-__device__ __forceinline__ float dgroup_max(float v) {
-  v = fmaxf(v, ror16f<8>(v));
-  v = fmaxf(v, ror16f<4>(v));
-  v = fmaxf(v, ror16f<2>(v));
-  v = fmaxf(v, ror16f<1>(v));
-  if constexpr (D >= 32) v = fmaxf(v, __shfl_xor(v, 16, 64));
-  if constexpr (D >= 64) v = fmaxf(v, __shfl_xor(v, 32, 64));
-  return v;
-}
-
-// v of the lane whose byte address (4 * lane) is xaddr
-__device__ __forceinline__ float lane_read(float v, int xaddr) {
-  return __int_as_float(__builtin_amdgcn_ds_bpermute(xaddr, __float_as_int(v)));
-}
 
 // upper tile (I, J), I <= J, in row-major order of the upper triangle
 template <int NB>
@@ -142,20 +75,20 @@ __host__ __device__ constexpr int utile(int I, int J) {
   return I * NB - I * (I - 1) / 2 + (J - I);
 }
 
-// RESC_: rescue pass after the symplectic sweep (Riccati steps only): a workgroup runs only when
+// RESC_: rescue pass after the symplectic sweep: a workgroup runs only when
 // one of its problems carries the NaN marker, and stores the marked problems only.
-template <int D, int PPW_, int WPB_, int SM, bool WRITE_U, bool SYM_ = false, bool RESC_ = false, bool TOK_ = false>
-__global__ __launch_bounds__(64 * WPB_) __attribute__((amdgpu_waves_per_eu(MB<D, PPW_, WPB_, SYM_, TOK_>::MINW,
-                                                                           MB<D, PPW_, WPB_, SYM_, TOK_>::MAXW))) void
+template <int D, int PPW_, int WPB_, int SM, bool WRITE_U, bool RESC_ = false>
+__global__ __launch_bounds__(64 * WPB_)
+__attribute__((amdgpu_waves_per_eu(MB<D, PPW_, WPB_>::MINW, MB<D, PPW_, WPB_>::MINW))) void
 lqr_fwd_blk_kernel(const float* __restrict__ A_diag, const float* __restrict__ Bg, const float* __restrict__ Qg,
                    const float* __restrict__ Rinv, const float* __restrict__ Qf, const float* __restrict__ lgA,
                    const float* __restrict__ lgB, const float* __restrict__ lgQ, const float* __restrict__ h0,
                    int64_t P, int H, int T, float* __restrict__ u_out, float* __restrict__ kstash,
                    float* __restrict__ q0stash, int* __restrict__ status) {
-  using G = MB<D, PPW_, WPB_, SYM_, TOK_>;
+  using G = MB<D, PPW_, WPB_>;
   constexpr int NB = G::NB, PPW = G::PPW, NT = G::NT, LDX = G::LDX, LDG = G::LDG;
-  constexpr int NBQ = G::NBQ;
-  auto bqi = [](int q) { return NBQ == 1 ? 0 : q; };  // register copy of B / Q of problem q
+  constexpr int NBQ = G::BQ_LDS ? 1 : PPW;  // register copies of B / Q
+  auto bqi = [](int q) { return NBQ == 1 ? 0 : q; };
   constexpr int RPP = G::RPP, NPASS = G::NPASS;
   constexpr bool BQL = G::BQ_LDS;
   extern __shared__ __align__(16) float sm[];
@@ -176,7 +109,6 @@ lqr_fwd_blk_kernel(const float* __restrict__ A_diag, const float* __restrict__ B
   int64_t pid[PPW];
 #pragma unroll
   for (int q = 0; q < PPW; ++q) pid[q] = (pbase + q < P) ? (pbase + q) : (P - 1);  // idle: recompute, never store
-  static_assert(!(RESC_ && SYM_), "the rescue pass takes Riccati steps");
   unsigned marked = ~0u;  // the problems this launch may store
   if constexpr (RESC_) {
     // the same decision in every wave of the workgroup, before its only barrier
@@ -193,13 +125,13 @@ lqr_fwd_blk_kernel(const float* __restrict__ A_diag, const float* __restrict__ B
   float* shq = sm + G::OFF_Q;  // shared -sym(Q) fragments (d = 64)
   float* wbase = sm + G::SH + wv * G::PER_WAVE;
   auto region = [&](int q) { return wbase + q * G::REG; };
-  float* vecs = wbase + PPW * G::REG;  // [q][alpha D | q D | beta D | -beta^2/R D | 1/alpha D]
+  float* vecs = wbase + PPW * G::REG;  // [q][alpha D | q D | beta D]
 
   // row layout, pass pa: lane li of problem qr = pa * RPP + lane / D
   int qr[NPASS];
   int64_t po[NPASS];
   bool own_valid[NPASS];
-  float a_l[NPASS], lb2_l[NPASS], lq2_l[NPASS], la2_o[NPASS], rinv_l[NPASS];
+  float a_l[NPASS], lb2_l[NPASS], lq2_l[NPASS], la2_o[NPASS];
 #pragma unroll
   for (int pa = 0; pa < NPASS; ++pa) {
     qr[pa] = pa * RPP + lane / D;
@@ -209,7 +141,6 @@ lqr_fwd_blk_kernel(const float* __restrict__ A_diag, const float* __restrict__ B
     lb2_l[pa] = lgB[po[pa] * D + li] * kLog2e;
     lq2_l[pa] = lgQ[po[pa] * D + li] * kLog2e;
     la2_o[pa] = lgA[po[pa]] * kLog2e;
-    rinv_l[pa] = Rinv[po[pa] * D + li];
   }
 
   // C-layout state: N = -V (all tiles); B and -sym(Q) (registers, or shared LDS for d = 64)
@@ -217,10 +148,6 @@ lqr_fwd_blk_kernel(const float* __restrict__ A_diag, const float* __restrict__ B
   float Bm[NBQ][NB][NB][4];
   v4f Qn[NBQ][NT];
   float rr[PPW][NB];  // 1 / R_inv[16I + c]
-  // symplectic sweep: B in the transposed operand layout, Bt[q][I][K][s] = B[16I + c][16K + 4g + s],
-  // and Y1' (the sweep keeps Y-hat = Y' in the C layout; Y2' is -N)
-  float Bt[(G::SYM && !G::SYMW) ? NBQ : 1][NB][NB][4];
-  v4f Y1[G::SYM ? PPW : 1][NB][NB];
   if constexpr (BQL) {
     // the workgroup's token: B column-major, -sym(Q) as per-lane C-layout fragments
     const int64_t n = pid[0] / H;
@@ -229,12 +156,8 @@ lqr_fwd_blk_kernel(const float* __restrict__ A_diag, const float* __restrict__ B
     for (int e = threadIdx.x; e < D * D; e += G::THREADS) {
       const int i = e / D, j = e % D;
       shb[j * LDX + i] = bq[e];
-      if constexpr (G::SYMW) {
-        sm[G::OFF_BR + i * LDX + j] = bq[e];
-        shq[i * LDX + j] = -0.5f * (qq[e] + qq[j * D + i]);
-      }
     }
-    for (int e = threadIdx.x; e < (G::SYMW ? 0 : NT * 64); e += G::THREADS) {
+    for (int e = threadIdx.x; e < NT * 64; e += G::THREADS) {
       const int tile = e >> 6, ln = e & 63;
       int I = 0, rem = tile;
       while (rem >= NB - I) {
@@ -269,18 +192,14 @@ lqr_fwd_blk_kernel(const float* __restrict__ A_diag, const float* __restrict__ B
             Bm[bqi(q)][I][J][r] = bq[i * D + j];
             if (I <= J) Qn[bqi(q)][utile<NB>(I, J)][r] = -0.5f * (qq[i * D + j] + qq[j * D + i]);
           }
-          if constexpr (G::SYM) {
-            if (!G::SYMW && q < NBQ) Bt[bqi(q)][I][J][r] = bq[(16 * I + c) * D + 16 * J + 4 * g + r];
-            Y1[q][I][J][r] = (i == j) ? 1.0f : 0.0f;
-          }
         }
       }
     }
   }
   // R = 1 / R_inv per problem, and the pivot floor of my elimination problem: half of
-  // min_j 1 / R_inv_j (the symplectic sweep needs them only from step 0 on, after its loop)
+  // min_j 1 / R_inv_j
   float piv_floor = 0.f;
-  auto load_r = [&]() {
+  {
 #pragma unroll
     for (int q = 0; q < PPW; ++q)
 #pragma unroll
@@ -293,8 +212,7 @@ lqr_fwd_blk_kernel(const float* __restrict__ A_diag, const float* __restrict__ B
       m = 0.5f * row16_min(m);
       if (q == qe) piv_floor = m;
     }
-  };
-  if constexpr (!G::SYM) load_r();
+  }
   if constexpr (BQL) __syncthreads();  // shared B / Q written (the only workgroup barrier)
 
   // B_k = B diag(beta), block-row K: Bk[J][s] = B[16K + 4g + s][16J + c] beta[16J + c]
@@ -511,392 +429,16 @@ lqr_fwd_blk_kernel(const float* __restrict__ A_diag, const float* __restrict__ B
     return false;
   };
 
-  // One step t >= 1 of the symplectic sweep (the reference's transposed row-block update,
-  // symplectic_iter.py:226-251, with V_t = Y1^{-1} Y2).  The registers hold Y-hat = Y' in the
-  // C layout: Y1' in Y1, Y2' as -N.  With B_k = B diag(beta) and R^{-1} = diag(R_inv):
-  //   M = R^{-1} B_k' Y2'      Y1' <- A_k^{-1} (Y1' + B_k M)      Y2' <- A_k Y2' + Qc_k Y1'
-  // (beta enters once, squared, in the row scaling of M).  Every TTC_SYM_RENORM steps the columns of
-  // Y-hat (rows of Y, which leave Y1^{-1} Y2 unchanged) are rescaled by powers of 2.
-  // step ratios of the sweep's discount factors (t runs down): q(t-1) = q(t) 2^{-lq2},
-  // beta(t-1)^2 = beta(t)^2 2^{-2 lb2}, each as a pair hi + lo of floats from a double exp2
-  // (the multiplications add only their rounding, no drift from a rounded ratio); lane
-  // addresses of the renormalisation's column maximum (lanes c, 16 + c, 32 + c, 48 + c)
-  float rQ_l[NPASS], rB2_l[NPASS], rQ_e[NPASS], rB2_e[NPASS];
-  auto ratio2 = [](float x, float& hi, float& lo) {
-    const double r = exp2((double)x);
-    hi = (float)r;
-    lo = (float)(r - (double)hi);
-  };
-#pragma unroll
-  for (int pa = 0; pa < NPASS; ++pa) {
-    ratio2(-lq2_l[pa], rQ_l[pa], rQ_e[pa]);
-    ratio2(-2.0f * lb2_l[pa], rB2_l[pa], rB2_e[pa]);
-  }
-  const int x16 = (lane ^ 16) << 2, x32 = (lane ^ 32) << 2;
-  if constexpr (G::SYM) {
-    // the sweep leaves the per-problem tile regions unused until its final solve
-#pragma unroll
-    for (int pa = 0; pa < NPASS; ++pa) region(qr[pa])[li] = rinv_l[pa];
-    wave_sync();
-  }
-  auto sym_step = [&](const int t) {
-    if constexpr (G::SYM) {
-    // the discount factors q = 2^{lq2 t} and -beta^2 R^{-1} (beta = 2^{lb2 (t+1)}) from the
-    // previous step's (slots D, 3D) times the step ratios, recomputed exactly every kSymRefresh
-    // steps
-    // (e_A stays an exp2 every step: by recurrence it moved the gradients' largest error
-    // against fp64 on the bench's config-2 sample from 1.3e-6 to 1.7e-6, for 0.6 % of the sweep)
-    const bool exact = (T - 1 - t) % kSymRefresh == 0;
-#pragma unroll
-    for (int pa = 0; pa < NPASS; ++pa) {
-      float* v = vecs + qr[pa] * G::VEC;
-      const float eA = __builtin_amdgcn_exp2f(la2_o[pa] * (float)(t + 1));
-      float q, nb2;
-      if (exact) {
-        const float beta = __builtin_amdgcn_exp2f(lb2_l[pa] * (float)(t + 1));
-        q = __builtin_amdgcn_exp2f(lq2_l[pa] * (float)t);
-        nb2 = -(beta * beta) * region(qr[pa])[li];  // R_inv, parked in the free tile region
-      } else {
-        const float q0 = v[D + li], n0 = v[3 * D + li];
-        q = fmaf(q0, rQ_l[pa], q0 * rQ_e[pa]);
-        nb2 = fmaf(n0, rB2_l[pa], n0 * rB2_e[pa]);
-      }
-      const float alpha = fmaf(a_l[pa], eA, 1.0f);
-      v[li] = alpha;
-      v[D + li] = q;
-      v[3 * D + li] = nb2;
-      v[4 * D + li] = __builtin_amdgcn_rcpf(alpha);
-    }
-    wave_sync();
-    const bool renorm = (T - 1 - t) % TTC_SYM_RENORM == TTC_SYM_RENORM - 1;
-    if constexpr (!G::SYMW) {
-#pragma unroll
-    for (int q = 0; q < PPW; ++q) {
-      const float* v = vecs + q * G::VEC;
-      // M = (B' N) diag-row(-beta^2 R^{-1}) = R^{-1} B_k' Y2'
-      v4f M = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < 4; ++s) M = mfma16x16x4(Bm[bqi(q)][0][0][s], NV[q][0][0][s], M);
-      const v4f nf = ld4(v + 3 * D + 4 * g);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) M[r] *= nf[r];
-      // Y1' <- A^{-1} (Y1' + B M)
-#pragma unroll
-      for (int s = 0; s < 4; ++s) Y1[q][0][0] = mfma16x16x4(Bt[bqi(q)][0][0][s], M[s], Y1[q][0][0]);
-      const v4f ia = ld4(v + 4 * D + 4 * g);
-      const v4f al = ld4(v + 4 * g);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        Y1[q][0][0][r] *= ia[r];
-        NV[q][0][0][r] *= al[r];
-      }
-      // -Y2' <- -A Y2' - Qc Y1'  (operand -Qc[c][4g+s] = q_c (-Q)[4g+s][c] q_{4g+s})
-      const float qc = v[D + c];
-      const v4f qrw = ld4(v + D + 4 * g);
-      float op[4];
-#pragma unroll
-      for (int s = 0; s < 4; ++s) op[s] = Qn[bqi(q)][0][s] * (qc * qrw[s]);
-#pragma unroll
-      for (int s = 0; s < 4; ++s) NV[q][0][0] = mfma16x16x4(op[s], Y1[q][0][0][s], NV[q][0][0]);
-      if (renorm) {
-        const v4f& y = Y1[q][0][0];
-        const v4f& n = NV[q][0][0];
-        float mk = maxnan(absmax(y[0], n[0]), fabsf(y[1]));
-        mk = maxnan(maxnan(mk, fabsf(n[1])), fabsf(y[2]));
-        mk = maxnan(maxnan(mk, fabsf(n[2])), fabsf(y[3]));
-        mk = maxnan(mk, fabsf(n[3]));
-        mk = maxnan(mk, lane_read(mk, x16));
-        mk = maxnan(mk, lane_read(mk, x32));
-        const int e = 1 - __builtin_amdgcn_frexp_expf(mk);  // m * 2^e in [1, 2)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          Y1[q][0][0][r] = __builtin_amdgcn_ldexpf(Y1[q][0][0][r], e);
-          NV[q][0][0][r] = __builtin_amdgcn_ldexpf(NV[q][0][0][r], e);
-        }
-      }
-    }
-    } else {
-    // NB x NB tiles; A operands from the workgroup's LDS: tile (I, K) of B' is
-    // B[16K + 4g + s][16I + c] (shb, column-major B), of B is B[16I + c][16K + 4g + s] and of
-    // -sym(Q) is -Q[16I + c][16K + 4g + s] (row-major copies)
-    const float* shbr = sm + G::OFF_BR;
-#pragma unroll
-    for (int q = 0; q < PPW; ++q) {
-      const float* v = vecs + q * G::VEC;
-      v4f M[NB][NB];
-#pragma unroll
-      for (int I = 0; I < NB; ++I)
-#pragma unroll
-        for (int J = 0; J < NB; ++J) M[I][J] = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int I = 0; I < NB; ++I)
-#pragma unroll
-        for (int K = 0; K < NB; ++K) {
-          const v4f a = ld4(shb + (16 * I + c) * LDX + 16 * K + 4 * g);
-#pragma unroll
-          for (int J = 0; J < NB; ++J)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) M[I][J] = mfma16x16x4(a[s], NV[q][K][J][s], M[I][J]);
-        }
-#pragma unroll
-      for (int I = 0; I < NB; ++I) {
-        const v4f nf = ld4(v + 3 * D + 16 * I + 4 * g);
-#pragma unroll
-        for (int J = 0; J < NB; ++J)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) M[I][J][r] *= nf[r];
-      }
-#pragma unroll
-      for (int I = 0; I < NB; ++I) {
-#pragma unroll
-        for (int K = 0; K < NB; ++K) {
-          const v4f a = ld4(shbr + (16 * I + c) * LDX + 16 * K + 4 * g);
-#pragma unroll
-          for (int J = 0; J < NB; ++J)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) Y1[q][I][J] = mfma16x16x4(a[s], M[K][J][s], Y1[q][I][J]);
-        }
-        const v4f ia = ld4(v + 4 * D + 16 * I + 4 * g);
-        const v4f al = ld4(v + 16 * I + 4 * g);
-#pragma unroll
-        for (int J = 0; J < NB; ++J)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            Y1[q][I][J][r] *= ia[r];
-            NV[q][I][J][r] *= al[r];
-          }
-      }
-#pragma unroll
-      for (int I = 0; I < NB; ++I) {
-        const float qc = v[D + 16 * I + c];
-#pragma unroll
-        for (int K = 0; K < NB; ++K) {
-          const v4f qa = ld4(shq + (16 * I + c) * LDX + 16 * K + 4 * g);
-          const v4f qrw = ld4(v + D + 16 * K + 4 * g);
-          float op[4];
-#pragma unroll
-          for (int s = 0; s < 4; ++s) op[s] = qa[s] * (qc * qrw[s]);
-#pragma unroll
-          for (int J = 0; J < NB; ++J)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) NV[q][I][J] = mfma16x16x4(op[s], Y1[q][K][J][s], NV[q][I][J]);
-        }
-      }
-      if (renorm) {  // per column 16J + c of Y-hat
-#pragma unroll
-        for (int J = 0; J < NB; ++J) {
-          float mk = 0.f;
-#pragma unroll
-          for (int I = 0; I < NB; ++I)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) mk = maxnan(mk, absmax(Y1[q][I][J][r], NV[q][I][J][r]));
-          mk = maxnan(mk, lane_read(mk, x16));
-          mk = maxnan(mk, lane_read(mk, x32));
-          const int e = 1 - __builtin_amdgcn_frexp_expf(mk);
-#pragma unroll
-          for (int I = 0; I < NB; ++I)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              Y1[q][I][J][r] = __builtin_amdgcn_ldexpf(Y1[q][I][J][r], e);
-              NV[q][I][J][r] = __builtin_amdgcn_ldexpf(NV[q][I][J][r], e);
-            }
-        }
-      }
-    }
-    }
-    wave_sync();
-    }
-  };
-
-  // End of the symplectic sweep: -V_1 = Y1^{-1} (-Y2) by pivoted Gauss-Jordan on the rows
-  // [Y1 | -Y2] ([Y1 | -Y2 | I] at d = 32, for Y1^{-1}; lane li owns row li of problem qr), the
-  // certificate, and N = sym(-V_1) in the C layout.  Returns the accepted problems as bits.
-  auto sym_finish = [&]() -> unsigned {
-    if constexpr (!G::SYM) {
-      return ~0u;
-    } else if constexpr (G::SYMW) {
-    // NB x NB tiles: rows go through each problem's region 16 at a time (Y1, then -Y2, then
-    // the solution), pass by pass (RPP problems of D lanes each)
-    unsigned bits = 0u;
-    constexpr int W = G::AUGW;
-#pragma unroll
-    for (int pa = 0; pa < NPASS; ++pa) {
-      float aug[W];
-#pragma unroll
-      for (int mtx = 0; mtx < 2; ++mtx)
-#pragma unroll
-        for (int h = 0; h < NB; ++h) {
-          wave_sync();  // the region's previous rows have been read
-#pragma unroll
-          for (int k = 0; k < RPP; ++k) {
-            const int q = pa * RPP + k;
-            float* buf = region(q);
-            // row 16h + c of Y1 (of -Y2) = column 16h + c of Y1' (of -Y2' = N)
-#pragma unroll
-            for (int I = 0; I < NB; ++I) st4(buf + c * LDX + 16 * I + 4 * g, mtx == 0 ? Y1[q][I][h] : NV[q][I][h]);
-          }
-          wave_sync();
-          if (li >= 16 * h && li < 16 * h + 16) {
-            float row[D];
-            ld_row<D>(region(qr[pa]) + (li - 16 * h) * LDX, row);
-#pragma unroll
-            for (int k = 0; k < D; ++k) aug[mtx * D + k] = row[k];
-          }
-        }
-      if constexpr (G::SYM_INV) {
-#pragma unroll
-        for (int k = 0; k < D; ++k) aug[2 * D + k] = (k == li) ? 1.0f : 0.0f;
-      }
-      float rs = 0.f;
-#pragma unroll
-      for (int k = 0; k < D; ++k) rs += fabsf(aug[k]);
-      const float n1 = dgroup_max<D>(rs);  // ||Y1||_inf
-      wave_sync();  // every row read before the pivot-row buffer (aliasing them) is written
-      float* buf = region(qr[pa]);
-      float piv;
-      int pos;
-      gauss_jordan<D, W, 8>(aug, li, buf, piv, pos);
-      const float ip = 1.0f / piv;
-      float pn[D];
-#pragma unroll
-      for (int k = 0; k < D; ++k) pn[k] = aug[D + k] * ip;  // row pos of -V_1
-      float n2;
-      if constexpr (G::SYM_INV) {
-        float ri = 0.f;
-#pragma unroll
-        for (int k = 0; k < D; ++k) ri += fabsf(aug[2 * D + k]);
-        n2 = dgroup_max<D>(ri * fabsf(ip));  // ||Y1^{-1}||_inf
-      } else {
-        // spread of the pivots (the diagonal of U in Y1 = L U): max|u_kk| / min|u_kk| <= cond(Y1),
-        // with ||Y1||_inf standing in for max|u_kk| (at most n times larger)
-        n2 = dgroup_max<D>(fabsf(ip));
-      }
-      float da = 0.f, mx = 0.f;
-#pragma unroll
-      for (int k = 0; k < D; ++k) mx = fmaxf(mx, fabsf(pn[k]));
-#pragma unroll
-      for (int k = 0; k < RPP; ++k) {
-        const int q = pa * RPP + k;
-#pragma unroll
-        for (int I = 0; I < NB; ++I)
-#pragma unroll
-          for (int J = 0; J < NB; ++J) NV[q][I][J] = v4f{0.f, 0.f, 0.f, 0.f};
-      }
-      // rows 16h..16h+15 of -V_1: the asymmetry against my row, and their halves of
-      // N = sym(-V_1) in the C layout
-#pragma unroll
-      for (int h = 0; h < NB; ++h) {
-        wave_sync();
-        if (pos >= 16 * h && pos < 16 * h + 16) st_row<D>(buf + (pos - 16 * h) * LDX, pn);
-        wave_sync();
-#pragma unroll
-        for (int kk = 0; kk < 16; ++kk) da = fmaxf(da, fabsf(pn[16 * h + kk] - buf[kk * LDX + pos]));
-#pragma unroll
-        for (int k = 0; k < RPP; ++k) {
-          const int q = pa * RPP + k;
-          const float* b = region(q);
-#pragma unroll
-          for (int J = 0; J < NB; ++J)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) NV[q][h][J][r] += 0.5f * b[(4 * g + r) * LDX + 16 * J + c];
-#pragma unroll
-          for (int I = 0; I < NB; ++I)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) NV[q][I][h][r] += 0.5f * b[c * LDX + 16 * I + 4 * g + r];
-        }
-      }
-      da = dgroup_max<D>(da);
-      mx = dgroup_max<D>(mx);
-      const bool ok = (n1 * n2 <= kSymCondMax) && (da <= kSymAsymMax * mx);  // false on NaN
-      const unsigned long long bal = __ballot(ok);
-#pragma unroll
-      for (int k = 0; k < RPP; ++k) bits |= (unsigned)((bal >> (k * D)) & 1ull) << (pa * RPP + k);
-    }
-    wave_sync();
-    return bits;
-    } else {
-    // d = 16: one pass (16 lanes per problem); Y1, then -Y2, go through each problem's region
-    // (row c of Y1 = column c of Y1'), which then holds the pivot row and the solution
-    static_assert(NPASS == 1, "d = 16 final solve: one row-layout pass");
-    constexpr int L2 = LDX;
-    float* buf = region(qr[0]);
-    float aug[2 * D];
-#pragma unroll
-    for (int mtx = 0; mtx < 2; ++mtx) {
-      wave_sync();  // the previous rows have been read
-#pragma unroll
-      for (int q = 0; q < PPW; ++q) st4(region(q) + c * L2 + 4 * g, mtx == 0 ? Y1[q][0][0] : NV[q][0][0]);
-      wave_sync();
-      ld_row<D>(buf + li * L2, *reinterpret_cast<float(*)[D]>(aug + mtx * D));
-    }
-    float rs = 0.f;
-#pragma unroll
-    for (int k = 0; k < D; ++k) rs += fabsf(aug[k]);
-    const float n1 = dgroup_max<D>(rs);  // ||Y1||_inf
-    wave_sync();  // every row read before the pivot-row buffer (aliasing them) is written
-    float piv;
-    int pos;
-    gauss_jordan<D, 2 * D, 8>(aug, li, buf, piv, pos);
-    const float ip = 1.0f / piv;
-    float pn[D];
-#pragma unroll
-    for (int k = 0; k < D; ++k) pn[k] = aug[D + k] * ip;
-    // the condition number from the pivots, the diagonal of U in Y1 = L U:
-    // ||Y1||_inf / min|u_kk| <= n cond_inf(Y1) (|l_ij| <= 1 under partial pivoting); the
-    // asymmetry test below is the one that separates the inaccurate problems
-    const float n2 = dgroup_max<D>(fabsf(ip));
-    st_row<D>(buf + pos * L2, pn);
-    wave_sync();
-    float da = 0.f, mx = 0.f;
-#pragma unroll
-    for (int k = 0; k < D; ++k) {
-      da = fmaxf(da, fabsf(pn[k] - buf[k * L2 + pos]));
-      mx = fmaxf(mx, fabsf(pn[k]));
-    }
-    da = dgroup_max<D>(da);
-    mx = dgroup_max<D>(mx);
-    const bool ok = (n1 * n2 <= kSymCondMax) && (da <= kSymAsymMax * mx);  // false on NaN
-    const unsigned long long bal = __ballot(ok);
-    unsigned bits = 0u;
-#pragma unroll
-    for (int q = 0; q < PPW; ++q) bits |= (unsigned)((bal >> (q * D)) & 1ull) << q;
-#pragma unroll
-    for (int q = 0; q < PPW; ++q) {
-      const float* b = region(q);
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        NV[q][0][0][r] = 0.5f * (b[(4 * g + r) * L2 + c] + b[c * L2 + 4 * g + r]);
-    }
-    wave_sync();
-    return bits;
-    }
-  };
-
-  unsigned okbits = marked;  // problems whose results are stored (the symplectic certificate; rescue: marked)
+  unsigned okbits = marked;  // problems whose results are stored (rescue: marked)
 
   // Step 0: stash V_1, form W_0 and Quu_0, u0 = -Quu_0^{-1} W_0' (alpha_0 * h0).
   auto step0 = [&]() {
-    // the row-layout problem indices once more, from an opaque copy of the lane index: after
-    // the symplectic sweep's loop, which needs every register, they are cheaper to recompute
-    // than to keep across it
-    int64_t po0[NPASS];
-    bool own0[NPASS];
-    {
-      int ln = lane;
-      asm volatile("" : "+v"(ln));
-#pragma unroll
-      for (int pa = 0; pa < NPASS; ++pa) {
-        const int q = pa * RPP + ln / D;
-        own0[pa] = pbase + q < P;
-        po0[pa] = own0[pa] ? (pbase + q) : (P - 1);
-      }
-    }
 #pragma unroll
     for (int pa = 0; pa < NPASS; ++pa) {
       float* v = vecs + qr[pa] * G::VEC;
       const float alpha = fmaf(a_l[pa], __builtin_amdgcn_exp2f(la2_o[pa]), 1.0f);
       v[li] = alpha;
-      v[D + li] = alpha * h0[po0[pa] * D + li];            // (A_0 h0)_li
+      v[D + li] = alpha * h0[po[pa] * D + li];            // (A_0 h0)_li
       v[2 * D + li] = __builtin_amdgcn_exp2f(lb2_l[pa]);  // beta_0
     }
     wave_sync();
@@ -967,53 +509,30 @@ lqr_fwd_blk_kernel(const float* __restrict__ A_diag, const float* __restrict__ B
           ld_row<D>(region(qr[pa]) + (li - h) * LDX, *reinterpret_cast<float(*)[D]>(aug));
       }
       aug[D] = vecs[qr[pa] * G::VEC + 2 * D + li];
-      const bool store = own0[pa] && ((okbits >> qr[pa]) & 1u);
+      const bool store = own_valid[pa] && ((okbits >> qr[pa]) & 1u);
       if (SM == STASH_V1 && store)
-        st_global_row<D>(q0stash + (po0[pa] * D + li) * D, *reinterpret_cast<float(*)[D]>(aug));
+        st_global_row<D>(q0stash + (po[pa] * D + li) * D, *reinterpret_cast<float(*)[D]>(aug));
       wave_sync();  // all rows read before the pivot-row buffer (aliasing them) is written
       float piv;
       int pos;
-      bool pivot = true;
-      if constexpr (D == 16) {
-        // Quu_0 is positive definite for a certified problem: elimination without row
-        // exchanges by DPP broadcasts; a pass where a pivot says otherwise is solved again
-        // with partial pivoting
-        float x[17];
-#pragma unroll
-        for (int k = 0; k < 17; ++k) x[k] = aug[k];
-        bool bad;
-        gj_spd16x1(x, li, piv, bad);
-        pivot = __any(bad);  // uniform
-        if (!pivot) {
-          aug[D] = x[16];
-          pos = li;
-        }
-      }
-      if (pivot) gauss_jordan<D, D + 4, (D + 4) % 8 == 0 ? 8 : 4, D + 1>(aug, li, region(qr[pa]), piv, pos);
+      gauss_jordan<D, D + 4, (D + 4) % 8 == 0 ? 8 : 4, D + 1>(aug, li, region(qr[pa]), piv, pos);
       const float u0 = -aug[D] / piv;
       if (store) {
-        if (WRITE_U) u_out[po0[pa] * D + pos] = u0;
+        if (WRITE_U) u_out[po[pa] * D + pos] = u0;
         if (status != nullptr && !isfinite(u0)) atomicOr(status, TTC_LQR_STATUS_NONFINITE);
       }
     }
   };
 
-  if constexpr (G::SYM) {
-    for (int t = T - 1; t >= 1; --t) sym_step(t);
-    okbits = sym_finish();
-    load_r();
-    step0();
-  } else {
-    int t = T - 1;
-    bool failed = false;
-    while (!failed && t >= 1) {
-      failed = step(t);
-      --t;
-    }
-    if (!failed) step0();
-    else okbits = 0u;
+  int t = T - 1;
+  bool failed = false;
+  while (!failed && t >= 1) {
+    failed = step(t);
+    --t;
   }
-  // problems whose sweep broke down or was not certified: mark them for lqr_rescue_kernel
+  if (!failed) step0();
+  else okbits = 0u;
+  // problems whose sweep broke down: mark them for lqr_rescue_kernel
   if (lane < PPW && pbase + lane < P && ((marked >> lane) & 1u) && !((okbits >> lane) & 1u)) {
     const float nan = __builtin_nanf("");
     if (WRITE_U) u_out[(pbase + lane) * D] = nan;

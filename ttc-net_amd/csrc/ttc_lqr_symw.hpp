@@ -30,7 +30,7 @@
 // 36.8 ms with two waves per SIMD (workgroups of 8 waves), 30.6 with three of 4 waves, 29.4 with
 // four, 29.6 with five; 48.5 ms on the fp32 matrix cores.
 #pragma once
-#include "ttc_lqr_mfma_blk.hpp"
+#include "ttc_lqr_sym.hpp"
 #include "ttc_lqr_split.hpp"
 
 namespace ttc {
@@ -484,14 +484,15 @@ inline void launch_symw_cw(const float* A, const float* B, const float* Q, const
 template <int D, int SM, bool WU>
 inline void launch_symw(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                         const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T,
-                        float* u, float* st_a, float* st_b, int32_t* status, hipStream_t s) {
+                        float* u, float* st_a, float* st_b, int32_t* status, hipStream_t s, int64_t call) {
+  // (by the whole call's problems: the two forms round differently, and a call's chunks must not)
   // 16 columns a wave: twice the waves, each with half the work, for batches that would leave most
   // SIMDs idle or with one wave (measured, T = 128, whole call: d = 64, 256 problems 476 against 644 us,
   // 512 663 / 677, 1,024 1,157 / 1,097; d = 32, 512 problems 248 / 318, 1,024 301 / 325, 2,048 482 /
   // 443); the operands are read from LDS twice as often, which costs 9 % when the chip is full, so at
   // d = 64 also for the odd head counts whose idle waves cost more (1 head 29.1 / 38.2 ms, 3 heads
   // 29.2 / 35.6, 5 heads 28.9 / 31.9 for 30,000 problems; at 9 heads 10 / 9 of the wide form's time)
-  if (P * D <= 32768 || (D == 64 && H % 2 != 0 && H <= 9))
+  if (call * D <= 32768 || (D == 64 && H % 2 != 0 && H <= 9))
     launch_symw_cw<D, 16, SM, WU>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s);
   else
     launch_symw_cw<D, 32, SM, WU>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s);
