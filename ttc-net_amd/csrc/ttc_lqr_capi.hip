@@ -927,28 +927,18 @@ static int64_t fact_chunk(int64_t n_tokens, int H, int d, int du, int rb, int rq
   return chunk;
 }
 
-template <typename TC>
-static int expand_chunk(const TC* cB, const TC* cQ, const TC* cQf, const float* Bs, const float* Gs,
-                        int64_t nc, int H, int d, int du, int rb, int rq, float* Bx, float* Qx, float* Qfx,
-                        hipStream_t s) {
-  int rc = launch_expand(cB, nc, rb, Bs, d * du, Bx, s);
-  if (rc == TTC_LQR_OK) rc = launch_expand(cQ, nc, rq, Gs, d * d, Qx, s);
-  if (rc == TTC_LQR_OK) rc = launch_expand(cQf, nc * H, rq, Gs, d * d, Qfx, s);
-  return rc;
-}
-
 // Storage of the factored inputs and gradients: fp32 as is, bf16 (bit patterns) converted
 // to / from fp32 arrays in the workspace.
 template <typename TS>
 struct Store {
   static constexpr bool BF16 = std::is_same<TS, uint16_t>::value;
-  // fp32 view of in[off .. off + n): the array itself, or its conversion into dst
-  static const float* in(const TS* a, int64_t off, size_t n, float* dst, hipStream_t s, int& rc) {
+  // fp32 view of in[off .. off + n): the array itself, or its conversion into dst, queued in `batch`
+  static const float* in(const TS* a, int64_t off, size_t n, float* dst, ConvBatch& batch) {
     if constexpr (BF16) {
-      if (rc == TTC_LQR_OK) rc = launch_bf16_to_f32(a + off, (int64_t)n, dst, s);
+      batch.add(a + off, dst, (int64_t)n);
       return dst;
     } else {
-      (void)n; (void)dst; (void)s;
+      (void)n; (void)dst; (void)batch;
       return a + off;
     }
   }
@@ -962,11 +952,11 @@ struct Store {
       return a + off;
     }
   }
-  static void flush(TS* a, int64_t off, size_t n, const float* tmp, hipStream_t s, int& rc) {
+  static void flush(TS* a, int64_t off, size_t n, const float* tmp, ConvBatch& batch) {
     if constexpr (BF16) {
-      if (rc == TTC_LQR_OK) rc = launch_f32_to_bf16(tmp, (int64_t)n, a + off, s);
+      batch.add(tmp, a + off, (int64_t)n);
     } else {
-      (void)a; (void)off; (void)n; (void)tmp; (void)s;
+      (void)a; (void)off; (void)n; (void)tmp; (void)batch;
     }
   }
 };
@@ -990,8 +980,9 @@ static int forward_factored(const TS* A_diag, const TS* coeff_B, const TS* coeff
   const FactLayout L0 = fact_layout(chunk, H, d, du, rb, rq, T, stash != nullptr, false, St::BF16, compact, flags);
   int rc = TTC_LQR_OK;
   float* bas = reinterpret_cast<float*>(ws + L0.bas);
-  const float* Bs = St::in(B_basis, 0, nb, bas, s, rc);
-  const float* Gs = St::in(Q_basis, 0, nq, bas + nb, s, rc);
+  ConvBatch bases;
+  const float* Bs = St::in(B_basis, 0, nb, bas, bases);
+  const float* Gs = St::in(Q_basis, 0, nq, bas + nb, bases);
   for (int64_t n0 = 0; n0 < n_tokens && rc == TTC_LQR_OK; n0 += chunk) {
     const int64_t nc = (n0 + chunk <= n_tokens) ? chunk : (n_tokens - n0);
     const int64_t p0 = n0 * H;
@@ -999,12 +990,14 @@ static int forward_factored(const TS* A_diag, const TS* coeff_B, const TS* coeff
     size_t n[10];
     io_counts(nc, H, d, du, rb, rq, n);
     auto cin = [&](int k) { return reinterpret_cast<float*>(ws + L.cin[k]); };
-    const float* a = St::in(A_diag, p0 * d, n[0], cin(0), s, rc);
-    const float* r = St::in(R_inv, p0 * du, n[3], cin(3), s, rc);
-    const float* la = St::in(log_gamma_A, p0, n[5], cin(5), s, rc);
-    const float* lb = St::in(log_gamma_B, p0 * du, n[6], cin(6), s, rc);
-    const float* lq = St::in(log_gamma_Q, p0 * d, n[7], cin(7), s, rc);
-    const float* hz = St::in(h0, p0 * d, n[8], cin(8), s, rc);
+    ConvBatch batch = n0 == 0 ? bases : ConvBatch{};
+    const float* a = St::in(A_diag, p0 * d, n[0], cin(0), batch);
+    const float* r = St::in(R_inv, p0 * du, n[3], cin(3), batch);
+    const float* la = St::in(log_gamma_A, p0, n[5], cin(5), batch);
+    const float* lb = St::in(log_gamma_B, p0 * du, n[6], cin(6), batch);
+    const float* lq = St::in(log_gamma_Q, p0 * d, n[7], cin(7), batch);
+    const float* hz = St::in(h0, p0 * d, n[8], cin(8), batch);
+    rc = launch_bf16_to_f32(batch, s);
     if (rc != TTC_LQR_OK) return rc;
     float* Bx = reinterpret_cast<float*>(ws + L.Bx);
     float* Qx = reinterpret_cast<float*>(ws + L.Qx);
@@ -1015,8 +1008,8 @@ static int forward_factored(const TS* A_diag, const TS* coeff_B, const TS* coeff
       Qfx = K.Qf + p0 * dd;
     }
     // the expansion reads the coefficients as stored (bf16: widened in registers)
-    rc = expand_chunk(coeff_B + n0 * rb, coeff_Q + n0 * rq, coeff_Qf + p0 * rq, Bs, Gs, nc, H, d, du, rb, rq, Bx, Qx,
-                      Qfx, s);
+    rc = launch_expand(coeff_B + n0 * rb, coeff_Q + n0 * rq, coeff_Qf + p0 * rq, nc, H, rb, rq, Bs, Gs, d * d, Bx, Qx,
+                       Qfx, s);
     if (rc != TTC_LQR_OK) return rc;
     float* v1 = stash ? stash + p0 * dd : nullptr;
     float* q0 = stash ? stash + P * dd + p0 * (int64_t)du * du : nullptr;
@@ -1064,12 +1057,14 @@ static int backward_factored(const TS* A_diag, const TS* coeff_B, const TS* coef
   if (n_tokens == 0) {  // the basis gradients are sums over no tokens
     rc = launch_reduce(nullptr, 0, rb, nullptr, Eb, nullptr, gBs, 0, s);
     if (rc == TTC_LQR_OK) rc = launch_reduce(nullptr, 0, rq, nullptr, Eq, nullptr, gGs, 0, s);
-    St::flush(grad_B_basis, 0, nb, gBs, s, rc);
-    St::flush(grad_Q_basis, 0, nq, gGs, s, rc);
-    return rc;
+    ConvBatch out;
+    St::flush(grad_B_basis, 0, nb, gBs, out);
+    St::flush(grad_Q_basis, 0, nq, gGs, out);
+    return rc == TTC_LQR_OK ? launch_f32_to_bf16(out, s) : rc;
   }
-  const float* Bs = St::in(B_basis, 0, nb, bas, s, rc);
-  const float* Gs = St::in(Q_basis, 0, nq, bas + nb, s, rc);
+  ConvBatch bases;
+  const float* Bs = St::in(B_basis, 0, nb, bas, bases);
+  const float* Gs = St::in(Q_basis, 0, nq, bas + nb, bases);
   const int64_t P = n_tokens * H, dd = (int64_t)d * d;
   int64_t total_fb = 0;
   for (int64_t n0 = 0; n0 < n_tokens && rc == TTC_LQR_OK; n0 += chunk) {
@@ -1080,16 +1075,17 @@ static int backward_factored(const TS* A_diag, const TS* coeff_B, const TS* coef
     io_counts(nc, H, d, du, rb, rq, n);
     auto cin = [&](int k) { return reinterpret_cast<float*>(ws + L.cin[k]); };
     auto cg = [&](int k) { return reinterpret_cast<float*>(ws + L.cg[k]); };
-    const float* a = St::in(A_diag, p0 * d, n[0], cin(0), s, rc);
-    const float* cB = St::in(coeff_B, n0 * rb, n[1], cin(1), s, rc);
-    const float* cQ = St::in(coeff_Q, n0 * rq, n[2], cin(2), s, rc);
-    const float* r = St::in(R_inv, p0 * du, n[3], cin(3), s, rc);
-    const float* cQf = St::in(coeff_Qf, p0 * rq, n[4], cin(4), s, rc);
-    const float* la = St::in(log_gamma_A, p0, n[5], cin(5), s, rc);
-    const float* lb = St::in(log_gamma_B, p0 * du, n[6], cin(6), s, rc);
-    const float* lq = St::in(log_gamma_Q, p0 * d, n[7], cin(7), s, rc);
-    const float* hz = St::in(h0, p0 * d, n[8], cin(8), s, rc);
-    const float* dz = St::in(d_u, p0 * du, n[9], cin(9), s, rc);
+    ConvBatch batch = n0 == 0 ? bases : ConvBatch{};
+    const float* a = St::in(A_diag, p0 * d, n[0], cin(0), batch);
+    const float* cB = St::in(coeff_B, n0 * rb, n[1], cin(1), batch);
+    const float* cQ = St::in(coeff_Q, n0 * rq, n[2], cin(2), batch);
+    const float* r = St::in(R_inv, p0 * du, n[3], cin(3), batch);
+    const float* cQf = St::in(coeff_Qf, p0 * rq, n[4], cin(4), batch);
+    const float* la = St::in(log_gamma_A, p0, n[5], cin(5), batch);
+    const float* lb = St::in(log_gamma_B, p0 * du, n[6], cin(6), batch);
+    const float* lq = St::in(log_gamma_Q, p0 * d, n[7], cin(7), batch);
+    const float* hz = St::in(h0, p0 * d, n[8], cin(8), batch);
+    const float* dz = St::in(d_u, p0 * du, n[9], cin(9), batch);
     float* gA = St::out(grad_A_diag, p0 * d, cg(0));
     float* gcB = St::out(grad_coeff_B, n0 * rb, cg(1));
     float* gcQ = St::out(grad_coeff_Q, n0 * rq, cg(2));
@@ -1099,6 +1095,7 @@ static int backward_factored(const TS* A_diag, const TS* coeff_B, const TS* coef
     float* glB = St::out(grad_log_gamma_B, p0 * du, cg(6));
     float* glQ = St::out(grad_log_gamma_Q, p0 * d, cg(7));
     float* gh = St::out(grad_h0, p0 * d, cg(8));
+    rc = launch_bf16_to_f32(batch, s);
     if (rc != TTC_LQR_OK) return rc;
     float* Bx = reinterpret_cast<float*>(ws + L.Bx);
     float* Qx = reinterpret_cast<float*>(ws + L.Qx);
@@ -1112,7 +1109,7 @@ static int backward_factored(const TS* A_diag, const TS* coeff_B, const TS* coef
       Qx = K.Q + n0 * dd;
       Qfx = K.Qf + p0 * dd;
     } else {
-      rc = expand_chunk(cB, cQ, cQf, Bs, Gs, nc, H, d, du, rb, rq, Bx, Qx, Qfx, s);
+      rc = launch_expand(cB, cQ, cQf, nc, H, rb, rq, Bs, Gs, Eq, Bx, Qx, Qfx, s);
       if (rc != TTC_LQR_OK) return rc;
     }
     const float* v1 = with_stash ? stash + p0 * dd : nullptr;
@@ -1137,18 +1134,22 @@ static int backward_factored(const TS* A_diag, const TS* coeff_B, const TS* coef
     rc = launch_project_reduce(cB, nc, rb, gB, Eb, Bs, gcB, part, gBs, first, s);
     if (rc == TTC_LQR_OK) rc = launch_project_reduce(cQ, nc, rq, gQ, Eq, Gs, gcQ, part, gGs, first, s);
     if (rc == TTC_LQR_OK) rc = launch_project_reduce(cQf, Pc, rq, gQf, Eq, Gs, gcQf, part, gGs, 1, s);
-    St::flush(grad_A_diag, p0 * d, n[0], gA, s, rc);
-    St::flush(grad_coeff_B, n0 * rb, n[1], gcB, s, rc);
-    St::flush(grad_coeff_Q, n0 * rq, n[2], gcQ, s, rc);
-    St::flush(grad_R_inv, p0 * du, n[3], gR, s, rc);
-    St::flush(grad_coeff_Qf, p0 * rq, n[4], gcQf, s, rc);
-    St::flush(grad_log_gamma_A, p0, n[5], glA, s, rc);
-    St::flush(grad_log_gamma_B, p0 * du, n[6], glB, s, rc);
-    St::flush(grad_log_gamma_Q, p0 * d, n[7], glQ, s, rc);
-    St::flush(grad_h0, p0 * d, n[8], gh, s, rc);
+    ConvBatch out;
+    St::flush(grad_A_diag, p0 * d, n[0], gA, out);
+    St::flush(grad_coeff_B, n0 * rb, n[1], gcB, out);
+    St::flush(grad_coeff_Q, n0 * rq, n[2], gcQ, out);
+    St::flush(grad_R_inv, p0 * du, n[3], gR, out);
+    St::flush(grad_coeff_Qf, p0 * rq, n[4], gcQf, out);
+    St::flush(grad_log_gamma_A, p0, n[5], glA, out);
+    St::flush(grad_log_gamma_B, p0 * du, n[6], glB, out);
+    St::flush(grad_log_gamma_Q, p0 * d, n[7], glQ, out);
+    St::flush(grad_h0, p0 * d, n[8], gh, out);
+    if (n0 + nc == n_tokens) {
+      St::flush(grad_B_basis, 0, nb, gBs, out);
+      St::flush(grad_Q_basis, 0, nq, gGs, out);
+    }
+    if (rc == TTC_LQR_OK) rc = launch_f32_to_bf16(out, s);
   }
-  St::flush(grad_B_basis, 0, nb, gBs, s, rc);
-  St::flush(grad_Q_basis, 0, nq, gGs, s, rc);
   if (n_fallback && rc == TTC_LQR_OK) *n_fallback = total_fb;
   return rc;
 }

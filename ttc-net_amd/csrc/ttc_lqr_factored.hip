@@ -41,13 +41,29 @@ constexpr int kExpandChunk = 16;  // ranks whose loads are issued together
 __device__ __forceinline__ float coeff_value(const float* p) { return *p; }
 __device__ __forceinline__ float coeff_value(const uint16_t* p) { return __uint_as_float((uint32_t)*p << 16); }
 
+// Up to three such products in one launch (B, Q and Q_f of a chunk; workgroups first[k] .. of
+// product k): at a few tokens each is 4 us of launch, 13.3 -> 5 us for the three.
 template <typename TC>
-__global__ __launch_bounds__(256) void expand_kernel(const TC* __restrict__ coeff, int64_t M, int R,
-                                                     const float* __restrict__ basis, int E,
-                                                     float* __restrict__ out) {
+struct ExpandJobs {
+  const TC* coeff[3];
+  const float* basis[3];
+  float* out[3];
+  int64_t M[3];
+  int R[3];
+  unsigned first[3];
+};
+
+template <typename TC>
+__global__ __launch_bounds__(256) void expand_kernel(const ExpandJobs<TC> jobs, int E) {
+  const int job = blockIdx.x >= jobs.first[2] ? 2 : blockIdx.x >= jobs.first[1] ? 1 : 0;  // uniform
+  const TC* __restrict__ coeff = jobs.coeff[job];
+  const float* __restrict__ basis = jobs.basis[job];
+  float* __restrict__ out = jobs.out[job];
+  const int64_t M = jobs.M[job];
+  const int R = jobs.R[job];
   const int E4 = E >> 2;
   const int64_t nblk = (M + kExpandRows - 1) / kExpandRows;
-  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t t = (int64_t)(blockIdx.x - jobs.first[job]) * 256 + threadIdx.x;
   if (t >= nblk * E4) return;  // wave-uniform: nblk * E4 is a multiple of 64
   const int64_t t0 = t - (threadIdx.x & 63);  // the wave's first thread
   const int64_t mb_l = t0 / E4;
@@ -289,18 +305,33 @@ __global__ __launch_bounds__(64) void project_reduce_kernel(const float* __restr
   }
 }
 
-// out[j][i] = (accumulate ? out[j][i] : 0) + sum_{k in [j G, min(S, (j+1) G))} in[k][i], in the
-// order of k.  Grid: (ceil(n / 256), ceil(S / G)).
+// out[i] = (accumulate ? out[i] : 0) + sum_{k < S} in[k][i], in a fixed order: groups of kSlabGroup
+// slabs, each in order, then the groups in order.  A workgroup takes 32 columns and spreads the groups
+// over its eight rows of threads (S <= 2,048 slabs are at most 32 groups).  One launch, and S / 64 times
+// the loads in flight of a thread per column: 24.4 -> 11 us for 1,024 slabs of 4,096 values.
+constexpr int kSlabGroup = 64;
+constexpr int kSlabGroups = 32;
 __global__ __launch_bounds__(256) void sum_slabs_kernel(const float* __restrict__ in, int64_t S, int64_t n,
-                                                        int64_t G, float* __restrict__ out, int accumulate) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const int64_t j = blockIdx.y;
-  const int64_t k0 = j * G;
-  const int64_t k1 = (k0 + G < S) ? (k0 + G) : S;
-  float acc = accumulate ? out[j * n + i] : 0.f;
-  for (int64_t k = k0; k < k1; ++k) acc += in[k * n + i];
-  out[j * n + i] = acc;
+                                                        float* __restrict__ out, int accumulate) {
+  __shared__ float part[kSlabGroups][32];
+  const int col = threadIdx.x & 31, row = threadIdx.x >> 5;
+  const int64_t i = (int64_t)blockIdx.x * 32 + col;
+  const int groups = (int)((S + kSlabGroup - 1) / kSlabGroup);
+  if (i < n) {
+    for (int j = row; j < groups; j += 8) {
+      const int64_t k1 = (int64_t)(j + 1) * kSlabGroup < S ? (int64_t)(j + 1) * kSlabGroup : S;
+      float acc = 0.f;
+#pragma unroll 8
+      for (int64_t k = (int64_t)j * kSlabGroup; k < k1; ++k) acc += in[k * n + i];
+      part[j][col] = acc;
+    }
+  }
+  __syncthreads();
+  if (row == 0 && i < n) {
+    float acc = accumulate ? out[i] : 0.f;
+    for (int j = 0; j < groups; ++j) acc += part[j][col];
+    out[i] = acc;
+  }
 }
 
 __global__ __launch_bounds__(256) void zero_kernel(float* __restrict__ p, int64_t n) {
@@ -308,38 +339,64 @@ __global__ __launch_bounds__(256) void zero_kernel(float* __restrict__ p, int64_
   if (i < n) p[i] = 0.f;
 }
 
-constexpr int kSlabGroup = 64;  // first-level group of sum_slabs_kernel
-
 // bf16 storage (bit patterns) <-> fp32: widening is exact; narrowing rounds to nearest even
 // (NaN stays NaN), as torch's .to(torch.bfloat16).
-__global__ __launch_bounds__(256) void bf16_to_f32_kernel(const uint16_t* __restrict__ in, int64_t n,
-                                                          float* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) out[i] = __uint_as_float((uint32_t)in[i] << 16);
+// Each kernel converts all arrays of a ConvBatch (an entry point has up to 10 per chunk, 4-8 us of
+// launch each when they are small), 8 values a thread, as 16-byte accesses where both sides are aligned.
+__device__ __forceinline__ uint16_t to_bf16(float v) {
+  const uint32_t u = __float_as_uint(v);
+  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);  // NaN: quiet, keep the sign
+  return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
 }
 
-__global__ __launch_bounds__(256) void f32_to_bf16_kernel(const float* __restrict__ in, int64_t n,
-                                                          uint16_t* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t u = __float_as_uint(in[i]);
-  uint16_t r;
-  if ((u & 0x7fffffffu) > 0x7f800000u) r = (uint16_t)((u >> 16) | 0x40u);  // NaN: quiet, keep the sign
-  else r = (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
-  out[i] = r;
+__device__ __forceinline__ int conv_job(const ConvBatch& b) {  // uniform
+  int k = 0;
+  while (k + 1 < b.count && blockIdx.x >= b.first[k + 1]) ++k;
+  return k;
+}
+
+__global__ __launch_bounds__(256) void bf16_to_f32_kernel(const ConvBatch b) {
+  const int k = conv_job(b);
+  const uint16_t* in = static_cast<const uint16_t*>(b.src[k]);
+  float* out = static_cast<float*>(b.dst[k]);
+  const int64_t n = b.n[k], i = ((int64_t)(blockIdx.x - b.first[k]) * 256 + threadIdx.x) * 8;
+  if (i + 8 <= n && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0) {
+    const uint4 v = *reinterpret_cast<const uint4*>(in + i);
+    float4* o = reinterpret_cast<float4*>(out + i);
+    o[0] = make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                       __uint_as_float(v.y & 0xffff0000u));
+    o[1] = make_float4(__uint_as_float(v.z << 16), __uint_as_float(v.z & 0xffff0000u), __uint_as_float(v.w << 16),
+                       __uint_as_float(v.w & 0xffff0000u));
+  } else {
+    for (int64_t j = i; j < i + 8 && j < n; ++j) out[j] = __uint_as_float((uint32_t)in[j] << 16);
+  }
+}
+
+__global__ __launch_bounds__(256) void f32_to_bf16_kernel(const ConvBatch b) {
+  const int k = conv_job(b);
+  const float* in = static_cast<const float*>(b.src[k]);
+  uint16_t* out = static_cast<uint16_t*>(b.dst[k]);
+  const int64_t n = b.n[k], i = ((int64_t)(blockIdx.x - b.first[k]) * 256 + threadIdx.x) * 8;
+  if (i + 8 <= n && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0) {
+    const float4 x = *reinterpret_cast<const float4*>(in + i), y = *reinterpret_cast<const float4*>(in + i + 4);
+    auto two = [](float lo, float hi) { return (uint32_t)to_bf16(lo) | ((uint32_t)to_bf16(hi) << 16); };
+    *reinterpret_cast<uint4*>(out + i) = make_uint4(two(x.x, x.y), two(x.z, x.w), two(y.x, y.y), two(y.z, y.w));
+  } else {
+    for (int64_t j = i; j < i + 8 && j < n; ++j) out[j] = to_bf16(in[j]);
+  }
 }
 
 static bool launched() { return hipGetLastError() == hipSuccess; }
 
-int launch_bf16_to_f32(const uint16_t* in, int64_t n, float* out, hipStream_t s) {
-  if (n <= 0) return TTC_LQR_OK;
-  hipLaunchKernelGGL(bf16_to_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, in, n, out);
+int launch_bf16_to_f32(const ConvBatch& b, hipStream_t s) {
+  if (b.count == 0) return TTC_LQR_OK;
+  hipLaunchKernelGGL(bf16_to_f32_kernel, dim3(b.blocks), dim3(256), 0, s, b);
   return launched() ? TTC_LQR_OK : TTC_LQR_ELAUNCH;
 }
 
-int launch_f32_to_bf16(const float* in, int64_t n, uint16_t* out, hipStream_t s) {
-  if (n <= 0) return TTC_LQR_OK;
-  hipLaunchKernelGGL(f32_to_bf16_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, in, n, out);
+int launch_f32_to_bf16(const ConvBatch& b, hipStream_t s) {
+  if (b.count == 0) return TTC_LQR_OK;
+  hipLaunchKernelGGL(f32_to_bf16_kernel, dim3(b.blocks), dim3(256), 0, s, b);
   return launched() ? TTC_LQR_OK : TTC_LQR_ELAUNCH;
 }
 
@@ -362,28 +419,29 @@ int64_t factor_slabs(int64_t M, int R, int E) {
   return S < 1 ? 1 : S;
 }
 
-size_t factor_partial_floats(int64_t M, int R, int E) {
-  const int64_t S = factor_slabs(M, R, E);
-  const int64_t S2 = (S + kSlabGroup - 1) / kSlabGroup;
-  return (size_t)(S + S2) * (size_t)R * (size_t)E;
-}
+size_t factor_partial_floats(int64_t M, int R, int E) { return (size_t)factor_slabs(M, R, E) * (size_t)R * (size_t)E; }
 
 template <typename TC>
-static int launch_expand_t(const TC* coeff, int64_t M, int R, const float* basis, int E, float* out, hipStream_t s) {
+static int launch_expand_t(const TC* cB, const TC* cQ, const TC* cQf, int64_t N, int H, int rb, int rq,
+                           const float* Bs, const float* Gs, int E, float* B, float* Q, float* Qf, hipStream_t s) {
   if (E % 256 != 0) return TTC_LQR_EINVAL;
-  const int64_t threads = (M + kExpandRows - 1) / kExpandRows * (E / 4);
-  if (threads <= 0) return TTC_LQR_OK;
-  hipLaunchKernelGGL(expand_kernel<TC>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, coeff, M, R, basis,
-                     E, out);
+  if (N <= 0) return TTC_LQR_OK;
+  auto blocks = [&](int64_t M) { return ((M + kExpandRows - 1) / kExpandRows * (E / 4) + 255) / 256; };
+  const int64_t b1 = blocks(N), b2 = 2 * b1;
+  const ExpandJobs<TC> jobs{{cB, cQ, cQf}, {Bs, Gs, Gs}, {B, Q, Qf}, {N, N, N * H}, {rb, rq, rq},
+                            {0u, (unsigned)b1, (unsigned)b2}};
+  hipLaunchKernelGGL(expand_kernel<TC>, dim3((unsigned)(b2 + blocks(N * H))), dim3(256), 0, s, jobs, E);
   return launched() ? TTC_LQR_OK : TTC_LQR_ELAUNCH;
 }
 
-int launch_expand(const float* coeff, int64_t M, int R, const float* basis, int E, float* out, hipStream_t s) {
-  return launch_expand_t(coeff, M, R, basis, E, out, s);
+int launch_expand(const float* cB, const float* cQ, const float* cQf, int64_t N, int H, int rb, int rq,
+                  const float* Bs, const float* Gs, int E, float* B, float* Q, float* Qf, hipStream_t s) {
+  return launch_expand_t(cB, cQ, cQf, N, H, rb, rq, Bs, Gs, E, B, Q, Qf, s);
 }
 
-int launch_expand(const uint16_t* coeff, int64_t M, int R, const float* basis, int E, float* out, hipStream_t s) {
-  return launch_expand_t(coeff, M, R, basis, E, out, s);
+int launch_expand(const uint16_t* cB, const uint16_t* cQ, const uint16_t* cQf, int64_t N, int H, int rb, int rq,
+                  const float* Bs, const float* Gs, int E, float* B, float* Q, float* Qf, hipStream_t s) {
+  return launch_expand_t(cB, cQ, cQf, N, H, rb, rq, Bs, Gs, E, B, Q, Qf, s);
 }
 
 int launch_project(const float* X, int64_t M, int E, const float* basis, int R, float* out, hipStream_t s) {
@@ -398,16 +456,10 @@ int launch_project(const float* X, int64_t M, int E, const float* basis, int R, 
   return launched() ? TTC_LQR_OK : TTC_LQR_ELAUNCH;
 }
 
-// out = (accumulate ? out : 0) + the sum of the S slab partials of R x E values (sum_slabs_kernel
-// twice: groups of kSlabGroup slabs, then the groups).
-static int launch_sum_slabs(float* partial, int64_t S, int64_t n, float* out, int accumulate, hipStream_t s) {
-  const int64_t S2 = (S + kSlabGroup - 1) / kSlabGroup;
-  float* level2 = partial + S * n;
-  const unsigned bx = (unsigned)((n + 255) / 256);
-  hipLaunchKernelGGL(sum_slabs_kernel, dim3(bx, (unsigned)S2), dim3(256), 0, s, partial, S, n, (int64_t)kSlabGroup,
-                     level2, 0);
-  if (!launched()) return TTC_LQR_ELAUNCH;
-  hipLaunchKernelGGL(sum_slabs_kernel, dim3(bx, 1u), dim3(256), 0, s, level2, S2, n, S2, out, accumulate);
+// out = (accumulate ? out : 0) + the sum of the S <= 2,048 slab partials of n values.
+static int launch_sum_slabs(const float* partial, int64_t S, int64_t n, float* out, int accumulate, hipStream_t s) {
+  if (S > (int64_t)kSlabGroup * kSlabGroups) return TTC_LQR_EINVAL;
+  hipLaunchKernelGGL(sum_slabs_kernel, dim3((unsigned)((n + 31) / 32)), dim3(256), 0, s, partial, S, n, out, accumulate);
   return launched() ? TTC_LQR_OK : TTC_LQR_ELAUNCH;
 }
 

@@ -137,9 +137,12 @@ int launch_ham64_mfma(const float* A, const float* B, const float* Q, const floa
                       int32_t* status, hipStream_t s);
 // Low-rank front-end (ttc_lqr_factored.hip): expansion of coefficient x basis sums and
 // their chain rule.  Rows of E = d * du floats; ranks R <= 64; E in {256, 1024, 4096}.
-int launch_expand(const float* coeff, int64_t M, int R, const float* basis, int E, float* out, hipStream_t s);
-// the same with bf16 coefficients (bit patterns), widened in registers
-int launch_expand(const uint16_t* coeff, int64_t M, int R, const float* basis, int E, float* out, hipStream_t s);
+// B (rank rb, basis Bs), Q and Q_f (rank rq, basis Gs) of N tokens of H heads, in one launch; the
+// coefficients fp32, or bf16 bit patterns widened in registers
+int launch_expand(const float* cB, const float* cQ, const float* cQf, int64_t N, int H, int rb, int rq,
+                  const float* Bs, const float* Gs, int E, float* B, float* Q, float* Qf, hipStream_t s);
+int launch_expand(const uint16_t* cB, const uint16_t* cQ, const uint16_t* cQf, int64_t N, int H, int rb, int rq,
+                  const float* Bs, const float* Gs, int E, float* B, float* Q, float* Qf, hipStream_t s);
 int launch_project(const float* X, int64_t M, int E, const float* basis, int R, float* out, hipStream_t s);
 int launch_reduce(const float* coeff, int64_t M, int R, const float* X, int E, float* partial, float* out,
                   int accumulate, hipStream_t s);
@@ -151,8 +154,26 @@ int64_t factor_slabs(int64_t M, int R, int E);
 int launch_pack_upper(const float* in, int64_t P, int D, float* out, hipStream_t s);
 int launch_unpack_quu0(const float* packed, const float* B, const float* lgB, const float* Rinv, int64_t P, int H,
                        int D, float* v1, float* q0, hipStream_t s);
-int launch_bf16_to_f32(const uint16_t* in, int64_t n, float* out, hipStream_t s);
-int launch_f32_to_bf16(const float* in, int64_t n, uint16_t* out, hipStream_t s);
+// Arrays to convert in one launch: workgroups first[k] .. of 2,048 values each take array k.
+struct ConvBatch {
+  static constexpr int MAX = 12;
+  const void* src[MAX];
+  void* dst[MAX];
+  int64_t n[MAX];
+  unsigned first[MAX];
+  unsigned blocks = 0;
+  int count = 0;
+  void add(const void* from, void* to, int64_t values) {
+    if (values <= 0) return;
+    src[count] = from;
+    dst[count] = to;
+    n[count] = values;
+    first[count++] = blocks;
+    blocks += (unsigned)((values + 2047) / 2048);
+  }
+};
+int launch_bf16_to_f32(const ConvBatch& b, hipStream_t s);
+int launch_f32_to_bf16(const ConvBatch& b, hipStream_t s);
 size_t factor_partial_floats(int64_t M, int R, int E);
 // The body of ttc_lqr_backward (argument checks, then the backward over the given workspace);
 // ttc_lqr_backward_noalloc calls it with its fixed device scratch.
