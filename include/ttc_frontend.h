@@ -1,5 +1,6 @@
-/* ttc_frontend.h -- C ABI of the layer's front-end in libttc_lqr.so (status codes: ttc_lqr.h).
- * Device pointers, fp32, contiguous; work is enqueued on `stream` (a hipStream_t). */
+/* ttc_frontend.h -- C ABI of libttc_lqr.so around the solver: the layer's front-end and the padding of
+ * the solver's tensors (status codes: ttc_lqr.h).  Device pointers, contiguous arrays; work is enqueued
+ * on `stream` (a hipStream_t). */
 #ifndef TTC_FRONTEND_H
 #define TTC_FRONTEND_H
 
@@ -25,6 +26,13 @@ int ttc_lqr_front_end_backward(const float* proj, int64_t n_tokens, int32_t head
                                const float* grad_coeff_Q, const float* grad_R_inv, const float* grad_coeff_Qf,
                                const float* grad_log_gamma_A, const float* grad_log_gamma_B,
                                const float* grad_log_gamma_Q, const float* grad_h0, float* grad_proj, void* stream);
+
+/* Matrices padded from rows x cols to padded rows x padded cols (powers of two, columns at least 4), up
+ * to 12 arrays in one launch: shapes[5 k ..] = {matrices, rows, cols, padded rows, padded cols} of array k,
+ * fill[k] the value of its new elements (bytes 2: 0 or 1), src / dst (16-byte aligned) their device
+ * pointers; `src`, `dst`, `shapes` and `fill` themselves are host arrays.  bytes: 4 (fp32) or 2 (bf16). */
+int ttc_lqr_pad(const void* const* src, void* const* dst, const int64_t* shapes, const float* fill, int32_t count,
+                int32_t bytes, void* stream);
 
 #ifdef __cplusplus
 }

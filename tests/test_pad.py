@@ -1,0 +1,35 @@
+"""``ttc_lqr_pad`` against torch's pad: whole vectors and matrices, edges of the four-element groups, both
+storage types, and its argument checks."""
+import ctypes
+
+import pytest
+import torch
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,H,d,du,D", [(1, 1, 1, 1, 16), (3, 5, 15, 13, 16), (2, 3, 17, 16, 32), (257, 2, 24, 20, 32),
+                                        (1, 7, 63, 64, 64), (5, 1, 33, 2, 64)])
+def test_pad_equals_torch(dtype, N, H, d, du, D):
+    from ttc.solvers.hip_lqr import _pad_tensors
+    F = torch.nn.functional
+    g = torch.Generator(device="cuda").manual_seed(d)
+    mk = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)  # noqa: E731
+    xs = [mk(N, H, d), mk(N, d, du), mk(N, H, du), mk(N, H, d, d)]
+    got = _pad_tensors(xs, [(D,), (D, D), (D,), (D, D)], [0, 0, 1, 0])
+    want = [F.pad(xs[0], (0, D - d)), F.pad(xs[1], (0, D - du, 0, D - d)), F.pad(xs[2], (0, D - du), value=1.0),
+            F.pad(xs[3], (0, D - d, 0, D - d))]
+    for a, b in zip(got, want):
+        assert a.dtype == dtype and torch.equal(a, b)
+
+
+def test_pad_argument_validation():
+    from ttc.solvers._lib import lib
+    p = (ctypes.c_void_p * 1)(64)
+    call = lambda shape, n=1, size=4: lib.ttc_lqr_pad(p, p, (ctypes.c_int64 * 5)(*shape), (ctypes.c_float * 1)(0), n,  # noqa: E731
+                                                      size, None)
+    assert call((1, 1, 3, 1, 24)) == 1   # not a power of two
+    assert call((1, 1, 17, 1, 16)) == 1  # larger than the padded size
+    assert call((1, 1, 3, 1, 16), n=13) == 1
+    assert call((1, 1, 3, 1, 16), size=8) == 1
+    assert call((0, 1, 3, 1, 16)) == 0   # nothing to do

@@ -97,6 +97,9 @@ def _load():
     L.ttc_lqr_front_end.argtypes = [f32p, f32p, i64, i32, i32, i32, i32, i32] + [f32p] * 9 + [ctypes.c_void_p]
     L.ttc_lqr_front_end_backward.restype = ctypes.c_int
     L.ttc_lqr_front_end_backward.argtypes = [f32p, i64, i32, i32, i32, i32, i32] + [f32p] * 10 + [ctypes.c_void_p]
+    L.ttc_lqr_pad.restype = ctypes.c_int
+    L.ttc_lqr_pad.argtypes = [ctypes.POINTER(ctypes.c_void_p)] * 2 + [ctypes.POINTER(i64), ctypes.POINTER(ctypes.c_float),
+                                                                      i32, i32, ctypes.c_void_p]
     L.ttc_lqr_noalloc_scratch_bytes.restype = sz
     L.ttc_lqr_noalloc_scratch_bytes.argtypes = []
     L.ttc_lqr_backward_noalloc.restype = ctypes.c_int

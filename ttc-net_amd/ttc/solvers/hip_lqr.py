@@ -89,22 +89,40 @@ def _env_bytes(name: str, default: int) -> int:
     return int(float(v)) if v else default
 
 
+def _pad_tensors(xs, shapes, fills):
+    """``xs[k]`` (contiguous fp32 or bf16, all on one device; trailing dims ``(rows, cols)``, or ``(cols,)`` as
+    one row) padded with ``fills[k]`` to ``shapes[k]``, in one launch."""
+    n, dev = len(xs), xs[0].device
+    outs, dims = [], []
+    for x, shape in zip(xs, shapes):
+        k = len(shape)
+        outs.append(torch.empty(*x.shape[:-k], *shape, device=dev, dtype=x.dtype))
+        rows = (x.shape[-2], shape[0]) if k == 2 else (1, 1)
+        dims += [x.numel() // (rows[0] * x.shape[-1]), rows[0], x.shape[-1], rows[1], shape[-1]]
+    ptrs = ctypes.c_void_p * n
+    with torch.cuda.device(dev):
+        rc = lib.ttc_lqr_pad(ptrs(*[x.data_ptr() for x in xs]), ptrs(*[o.data_ptr() for o in outs]),
+                             (ctypes.c_int64 * (5 * n))(*dims), (ctypes.c_float * n)(*fills), n, xs[0].element_size(),
+                             _stream_handle(dev))
+    check(rc, "ttc_lqr_pad")
+    return outs
+
+
 def _pad_inputs(ins, d, du, Dp):
     """Zero-pad the nine solver inputs from (d, du) to (Dp, Dp)."""
     A_diag, B, Q, R_inv, Q_f, lgA, lgB, lgQ, h0 = ins
     if d == Dp and du == Dp:
         return ins
-    pd, pu = Dp - d, Dp - du
-    F = torch.nn.functional
-    A_diag = F.pad(A_diag, (0, pd))
-    B = F.pad(B, (0, pu, 0, pd))
-    Q = F.pad(Q, (0, pd, 0, pd))
-    R_inv = F.pad(R_inv, (0, pu), value=1.0)
-    Q_f = F.pad(Q_f, (0, pd, 0, pd))
-    lgB = F.pad(lgB, (0, pu))
-    lgQ = F.pad(lgQ, (0, pd))
-    h0 = F.pad(h0, (0, pd))
-    return [t.contiguous() for t in (A_diag, B, Q, R_inv, Q_f, lgA, lgB, lgQ, h0)]
+    xs = [A_diag, B, Q, R_inv, Q_f, lgB, lgQ, h0]
+    vec, mat = (Dp,), (Dp, Dp)
+    shapes, fills = [vec, mat, mat, vec, mat, vec, vec, vec], [0, 0, 0, 1, 0, 0, 0, 0]
+    if Dp in SUPPORTED_DIMS and all(x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() for x in xs):
+        xs = _pad_tensors(xs, shapes, fills)
+    else:
+        xs = [torch.nn.functional.pad(x, [v for n, m in zip(x.shape[:-len(s) - 1:-1], s[::-1]) for v in (0, m - n)],
+                                      value=f) for x, s, f in zip(xs, shapes, fills)]
+    A_diag, B, Q, R_inv, Q_f, lgB, lgQ, h0 = xs
+    return [A_diag, B, Q, R_inv, Q_f, lgA, lgB, lgQ, h0]
 
 
 def riccati_flags(precision: str, T: int, Dp: int) -> int:
@@ -338,8 +356,7 @@ class HipLQRSolveFunc(torch.autograd.Function):
         if du == Dp:
             dU = d_u.to(torch.float32).contiguous()
         else:
-            dU = torch.zeros(bs, nh, Dp, device=dev, dtype=torch.float32)
-            dU[..., :du] = d_u.to(torch.float32)
+            dU, = _pad_tensors([d_u.to(torch.float32).contiguous()], [(Dp,)], [0])
         g = {
             "A": torch.empty(bs, nh, Dp, device=dev), "B": torch.empty(bs, Dp, Dp, device=dev),
             "Q": torch.empty(bs, Dp, Dp, device=dev), "R": torch.empty(bs, nh, Dp, device=dev),
@@ -505,18 +522,12 @@ class HipLQRFactoredFunc(torch.autograd.Function):
         assert not (mode and bf16), "the fused rescale runs on fp32 storage; rescale bf16 outputs outside"
         Dp = padded_dim(d, du)
         flags = riccati_flags(precision, T, Dp)
-        F = torch.nn.functional
         xs = [x.detach().to(store).contiguous() for x in ins]
-        pd, pu = Dp - d, Dp - du
-        if pd or pu:  # zero-padded states / unit-cost dummy controls, as HipLQRSolveFunc
-            xs[0] = F.pad(xs[0], (0, pd))
-            xs[3] = F.pad(xs[3], (0, pu), value=1.0)
-            xs[6] = F.pad(xs[6], (0, pu))
-            xs[7] = F.pad(xs[7], (0, pd))
-            xs[8] = F.pad(xs[8], (0, pd))
-            xs[9] = F.pad(xs[9], (0, pu, 0, pd))
-            xs[10] = F.pad(xs[10], (0, pd, 0, pd))
-            xs = [t.contiguous() for t in xs]
+        if d != Dp or du != Dp:  # zero-padded states / unit-cost dummy controls, as HipLQRSolveFunc
+            at = [0, 3, 6, 7, 8, 9, 10]
+            vec, mat = (Dp,), (Dp, Dp)
+            for k, t in zip(at, _pad_tensors([xs[k] for k in at], [vec] * 5 + [mat] * 2, [0, 1, 0, 0, 0, 0, 0])):
+                xs[k] = t
         u = torch.empty(bs, nh, Dp, device=dev, dtype=torch.float32)
         status = torch.zeros(1, device=dev, dtype=torch.int32)
         policy = stash or os.environ.get("TTC_LQR_STASH", "auto")
@@ -584,8 +595,7 @@ class HipLQRFactoredFunc(torch.autograd.Function):
         if du == Dp:
             dU = d_u.to(store).contiguous()
         else:
-            dU = torch.zeros(bs, nh, Dp, device=dev, dtype=store)
-            dU[..., :du] = d_u.to(store)
+            dU, = _pad_tensors([d_u.to(store).contiguous()], [(Dp,)], [0])
         if mode:  # d_y -> d_u through the fused rescale
             dY, dU = dU, torch.empty_like(dU)
             with _stage(dev, "bwd:ttc_lqr_rescale_backward"):
