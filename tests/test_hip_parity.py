@@ -129,6 +129,38 @@ def test_d16_head_groups_matrix_core_backward(N, H, T):
     assert out["_fallback"] % 8 == 0
 
 
+@pytest.mark.parametrize("N,H,T", [(5, 3, 9), (3, 4, 33), (2, 7, 2), (4, 5, 1), (3, 9, 17), (2, 12, 40), (2, 15, 8)])
+def test_d64_ragged_head_groups(N, H, T):
+    """The d = 64 head-group backward at head counts that are no multiple of 8: the token's last group has
+    idle columns; one group per token (H < 8, head sums written directly) and two."""
+    out = check_case(f"ragged64 N={N} H={H}", bench_solver_inputs(N, H, 64, seed=N + H + T), T)
+    assert out["_fallback"] == 0
+    check_case(f"ragged64-recompute N={N} H={H}", bench_solver_inputs(N, H, 64, seed=N + H), T, stash="never")
+
+
+@pytest.mark.parametrize("N,H", [(6, 3), (5, 6), (4, 11)])
+def test_d64_ragged_head_groups_rejected(N, H):
+    """Barely discounted inputs with spread scales in some tokens: their groups are rejected and their
+    problems -- not the idle columns -- taken by the stable path one by one, beside accepted groups."""
+    T = 48
+    ins = bench_solver_inputs(N, H, 64, seed=N + H)
+    A_diag, B, Q, R_inv, Qf, lgA, lgB, lgQ, h0 = ins
+    A_diag[::2] *= 4.0
+    R_inv[::2] *= 20.0
+    for lg in (lgA, lgB, lgQ):
+        lg[::2] *= 0.01
+    pb = LQRProblem(*ins, T)
+    dU = torch.randn(pb.N, pb.H, pb.du, generator=torch.Generator().manual_seed(3)).double().numpy()
+    fast = run_hip(ins, T, dU, grad_limit=math.inf)
+    slow = run_hip(ins, T, dU, grad_limit=math.inf, stable=True)
+    print(f"fallback {fast['_fallback']}/{pb.P}", flush=True)
+    assert 0 < fast["_fallback"] < pb.P
+    ref = solve_grads(pb, dU)
+    for k in ["u"] + NAMES:
+        assert _relerr(fast[k], ref[k]) <= TOL, k
+        assert _relerr(fast[k], slow[k]) <= TOL, k
+
+
 def test_d16_head_groups_with_rejected_groups():
     """Config-5 stress problems regrouped to 16 heads per token: groups that fail the
     certificate go through the stable path as whole groups, and the head sums of grad_B /

@@ -180,23 +180,40 @@ __global__ void scatter_group_kernel(const int* __restrict__ list, int64_t base,
   copy_span(gQg + o * d * d, c.gQ + i * d * d, d * d);
 }
 
-// Problems of the listed head groups (8 per group, chunk-local indices) for the second tier.
-__global__ void expand_groups_kernel(const int* __restrict__ glist, int64_t ngroups, int* __restrict__ plist) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < ngroups * 8) plist[e] = glist[e / 8] * 8 + (int)(e % 8);
+// Groups per token, and group G's first problem and problem count.
+__host__ __device__ inline int groups_of(int H) { return (H + 7) / 8; }
+__device__ inline int64_t group_first(int64_t G, int H, int& count) {
+  const int gpt = groups_of(H);
+  const int64_t n = G / gpt;
+  const int h = 8 * (int)(G - n * gpt);
+  count = H - h < 8 ? H - h : 8;
+  return n * H + h;
 }
 
-// grad_B / grad_Q of the listed head groups as the sums of their eight problems' partials
-// (part, at the problems' own indices) into the group's slot of out -- the token's output when
-// H == 8, checked against the guard there (status non-null).
-__global__ void groupsum_kernel(const int* __restrict__ glist, int64_t ngroups, const float* __restrict__ part,
+// Problems of the listed head groups (chunk-local indices), their count in np.
+__global__ void expand_groups_kernel(const int* __restrict__ glist, int64_t ngroups, int H, int* __restrict__ plist,
+                                     int32_t* np) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= ngroups) return;
+  int count;
+  const int64_t p0 = group_first(glist[e], H, count);
+  const int at = atomicAdd(np, count);
+  for (int k = 0; k < count; ++k) plist[at + k] = (int)(p0 + k);
+}
+
+// grad_B / grad_Q of the listed head groups as the sums of their problems' partials (part, at the
+// problems' own indices) into the group's slot of out -- the token's output when H <= 8, checked
+// against the guard there (status non-null).
+__global__ void groupsum_kernel(const int* __restrict__ glist, int64_t ngroups, int H, const float* __restrict__ part,
                                 int DD, float* __restrict__ out, float grad_limit, int* __restrict__ status) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= ngroups * DD) return;
   const int64_t G = glist[e / DD];
   const int r = (int)(e % DD);
+  int count;
+  const int64_t p0 = group_first(G, H, count);
   float s = 0.f;
-  for (int k = 0; k < 8; ++k) s += part[(G * 8 + k) * DD + r];
+  for (int k = 0; k < count; ++k) s += part[(p0 + k) * DD + r];
   out[G * DD + r] = s;
   if (status != nullptr) {
     if (!isfinite(s)) atomicOr(status, TTC_LQR_STATUS_NONFINITE);
@@ -204,12 +221,12 @@ __global__ void groupsum_kernel(const int* __restrict__ glist, int64_t ngroups, 
   }
 }
 
-static int launch_groupsum(const int32_t* glist, int64_t ngroups, const float* part, int DD, float* out,
+static int launch_groupsum(const int32_t* glist, int64_t ngroups, int H, const float* part, int DD, float* out,
                            float limit, int32_t* status, hipStream_t s) {
   const int64_t total = ngroups * DD;
   if (total <= 0) return TTC_LQR_OK;
-  hipLaunchKernelGGL(groupsum_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, glist, ngroups, part,
-                     DD, out, limit, status);
+  hipLaunchKernelGGL(groupsum_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, glist, ngroups, H,
+                     part, DD, out, limit, status);
   return hipGetLastError() == hipSuccess ? TTC_LQR_OK : TTC_LQR_ELAUNCH;
 }
 
@@ -413,11 +430,18 @@ struct FastLayout {
   int64_t n3;  // problems the third rollout tier can take (0: no third tier)
 };
 
-// The fast path rolls head groups of 8 on the matrix cores in fp32 (H % 8 == 0), else one
-// problem per row-layout rollout (fp32, or fp64 under the long-horizon flags).
+// The fast path rolls head groups on the matrix cores in fp32 -- 8 heads, or at d = 64 from 3 heads on
+// up to 8 -- else one problem per row-layout rollout (fp32, or fp64 under the long-horizon flags).
+// A group takes as long with idle columns, so it pays where the row layout is that much slower:
+// fwd + bwd of 12,000 problems at d = 64, T = 64, by group / by problem 14.6 / 12.2 ms with 1 head, 10.9 /
+// 11.3 with 2, 10.3 / 11.9 with 3, 9.1 / 11.1 with 4, 8.6 / 11.0 with 12 (600 problems 1.30 / 1.41); at
+// d = 32, T = 100 it is even (2,000 problems 1.04 / 0.97 ms, 10,000 2.1 / 2.3 with 12 heads), at d = 16
+// slower.
+static bool ragged_groups(int H, int flags, int d) {
+  return d == 64 && H % 8 != 0 && H >= 3 && !fp64_rollout(flags, d);
+}
 static bool head_group_path(int H, int flags, int d) {
-  (void)d;
-  return H % 8 == 0 && !(flags & TTC_LQR_FLAG_ROW_KERNEL);
+  return (H % 8 == 0 || ragged_groups(H, flags, d)) && !(flags & TTC_LQR_FLAG_ROW_KERNEL);
 }
 
 // Under the long-horizon flags the head-group rollout is the first of two tiers: the problems
@@ -442,9 +466,12 @@ static FastLayout fast_layout(int64_t chunk_tokens, int H, int d, int du, int T,
   const size_t Pc = (size_t)chunk_tokens * (size_t)H;
   // partial grad_B / grad_Q sums, added up per token by the head sum: one per problem of the
   // row-layout rollouts (per problem index; under two tiers for the second tier's problems),
-  // one per head group (none when a group is the whole token: it writes the outputs)
-  const size_t gparts = groups ? (size_t)chunk_tokens * (size_t)(H == 8 ? 0 : H / 8) : 0;
-  const size_t parts = (!groups || tiers) ? Pc : 0;
+  // one per head group (none when a group is the whole token: it writes the outputs).  The problems
+  // of a rejected group of a ragged head count take the stable path one by one, as a second tier's
+  const bool singles = tiers || (groups && H % 8 != 0);
+  const size_t ngroups = (size_t)chunk_tokens * (size_t)groups_of(H);
+  const size_t gparts = groups && H > 8 ? ngroups : 0;
+  const size_t parts = (!groups || singles) ? Pc : 0;
   FastLayout L{};
   size_t off = 0;
   L.v1 = off;
@@ -462,11 +489,11 @@ static FastLayout fast_layout(int64_t chunk_tokens, int H, int d, int du, int T,
   L.list = off;
   off += align256(Pc * sizeof(int32_t));
   L.glist = off;
-  off += tiers ? align256(Pc / 8 * sizeof(int32_t)) : 0;
+  off += singles ? align256(ngroups * sizeof(int32_t)) : 0;
   L.plist = off;
-  off += tiers ? align256(Pc * sizeof(int32_t)) : 0;
+  off += singles ? align256(Pc * sizeof(int32_t)) : 0;
   L.cnt = off;  // [0]: rejected problems (or groups), [1] / [2]: the second / third tier's,
-  off += 256;   // [3]: the stable path's problems after the third tier
+  off += 256;   // [3]: the stable path's problems after the third tier, [6]: the rejected groups' problems
   L.n3 = tier3_problems((int64_t)Pc, H, flags, d, du);
   L.l3 = off;   // the third tier's list: count, then its problems from index 64
   off += L.n3 > 0 ? align256((size_t)(64 + L.n3) * sizeof(int32_t)) : 0;
@@ -569,7 +596,7 @@ static int backward_core(const float* A_diag, const float* B, const float* Q, co
     float* gQp = reinterpret_cast<float*>(ws + L.gQp);
     int32_t* list = reinterpret_cast<int32_t*>(ws + L.list);
     int32_t* cnt = reinterpret_cast<int32_t*>(ws + L.cnt);
-    hipLaunchKernelGGL(fill_i32_kernel, dim3(1), dim3(64), 0, s, cnt, (int64_t)6, 0);
+    hipLaunchKernelGGL(fill_i32_kernel, dim3(1), dim3(64), 0, s, cnt, (int64_t)7, 0);
     // a device count the host needs: one stream synchronisation
     auto read_count = [&](const int32_t* c, int64_t cap, int32_t& v) -> int {
       v = 0;
@@ -608,40 +635,45 @@ static int backward_core(const float* A_diag, const float* B, const float* Q, co
       return TTC_LQR_OK;
     };
     if (head_group_path(H, flags, d)) {
-      // head groups of 8 on the matrix cores in fp32: grad_B / grad_Q summed inside the kernel
-      // (straight into the outputs when a group is a token, H == 8)
-      const bool direct = H == 8;
-      const bool tiers = two_tier_path(H, flags, d);
+      // head groups on the matrix cores in fp32: grad_B / grad_Q summed inside the kernel
+      // (straight into the outputs when a group is a token, H <= 8)
+      const bool direct = H <= 8;
+      const bool tiers = two_tier_path(H, flags, d), ragged = H % 8 != 0;
+      const int64_t ngroups = nc * groups_of(H);
       float* gBg = direct ? grad_B + n0 * dd : reinterpret_cast<float*>(ws + L.gBg);
       float* gQg = direct ? grad_Q + n0 * dd : reinterpret_cast<float*>(ws + L.gQg);
-      int32_t* glist = tiers ? reinterpret_cast<int32_t*>(ws + L.glist) : list;
+      int32_t* glist = tiers || ragged ? reinterpret_cast<int32_t*>(ws + L.glist) : list;
       auto* launch = d == 16 ? launch_ham16_mfma : (d == 32 ? launch_ham32_mfma : launch_ham64_mfma);
       rc = launch(a, b, q, r, qf, la, lb, lq, hz, uz, dz, v1, q0, Pc, H, T, tau, gA, gR, gQf, glA, glB, glQ, gh, gBg,
                   gQg, grad_limit, glist, cnt, status, s);
       if (rc != TTC_LQR_OK) return rc;
       int32_t nfail = 0;
-      rc = read_count(cnt, Pc / 8, nfail);
+      rc = read_count(cnt, ngroups, nfail);
       if (rc != TTC_LQR_OK) return rc;
-      if (tiers) {
+      if (tiers || ragged) {
         // long horizons: the problems of the rejected groups rolled again one by one in fp64 on
-        // the row layout (which accepts most of them), the rest by the stable path, and the
-        // groups' grad_B / grad_Q summed from the per-problem partials of the two
+        // the row layout (which accepts most of them), the rest by the stable path (a ragged head
+        // count: all of them), and the groups' grad_B / grad_Q summed from the per-problem partials
         if (nfail > 0) {
           int32_t* plist = reinterpret_cast<int32_t*>(ws + L.plist);
-          const int64_t np = 8 * (int64_t)nfail;
-          hipLaunchKernelGGL(expand_groups_kernel, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, s, glist,
-                             (int64_t)nfail, plist);
+          hipLaunchKernelGGL(expand_groups_kernel, dim3((unsigned)((nfail + 255) / 256)), dim3(256), 0, s, glist,
+                             (int64_t)nfail, H, plist, cnt + 6);
           if (hipGetLastError() != hipSuccess) return TTC_LQR_ELAUNCH;
-          switch (d) {
+          int32_t np = 8 * nfail;
+          if (ragged) {  // straight to the stable path, one by one
+            rc = read_count(cnt + 6, Pc, np);
+            if (rc != TTC_LQR_OK) return rc;
+          }
+          if (tiers) switch (d) {
             case 16: rc = launch_ham_d16(a, b, q, r, qf, la, lb, lq, hz, uz, dz, v1, q0, np, H, T, tau, gA, gR, gQf, glA, glB, glQ, gh, gBp, gQp, grad_limit, list, cnt + 1, status, s, true, plist, rs.slot_of ? rs.slot_of + p0 : nullptr, rs.slots, rs.nslot); break;
             case 32: rc = launch_ham_d32(a, b, q, r, qf, la, lb, lq, hz, uz, dz, v1, q0, np, H, T, tau, gA, gR, gQf, glA, glB, glQ, gh, gBp, gQp, grad_limit, list, cnt + 1, status, s, true, plist); break;
             default: return TTC_LQR_EUNSUPPORTED;
           }
           if (rc != TTC_LQR_OK) return rc;
-          int32_t nfail2 = 0;
-          rc = read_count(cnt + 1, np, nfail2);
+          int32_t nfail2 = np;
+          if (tiers) rc = read_count(cnt + 1, np, nfail2);
           if (rc != TTC_LQR_OK) return rc;
-          const int32_t* slist = list;  // the stable path's problems
+          const int32_t* slist = tiers ? list : plist;  // the stable path's problems
           int32_t nstable = nfail2;
           if (L.n3 > 0 && nfail2 > 0) {
             // third tier: those that started from the fp32 V_1 get an fp64 one and roll again;
@@ -686,9 +718,9 @@ static int backward_core(const float* A_diag, const float* B, const float* Q, co
             rc = stable_problems(slist, nstable, -1);
           }
           if (rc != TTC_LQR_OK) return rc;
-          rc = launch_groupsum(glist, nfail, gBp, (int)(d * du), gBg, grad_limit, direct ? status : nullptr, s);
+          rc = launch_groupsum(glist, nfail, H, gBp, (int)(d * du), gBg, grad_limit, direct ? status : nullptr, s);
           if (rc != TTC_LQR_OK) return rc;
-          rc = launch_groupsum(glist, nfail, gQp, (int)dd, gQg, grad_limit, direct ? status : nullptr, s);
+          rc = launch_groupsum(glist, nfail, H, gQp, (int)dd, gQg, grad_limit, direct ? status : nullptr, s);
           if (rc != TTC_LQR_OK) return rc;
         }
       } else {
@@ -712,9 +744,9 @@ static int backward_core(const float* A_diag, const float* B, const float* Q, co
         }
       }
       if (!direct) {
-        rc = launch_headsum(gBg, nc, H / 8, (int)(d * du), grad_B + n0 * d * du, grad_limit, status, s);
+        rc = launch_headsum(gBg, nc, groups_of(H), (int)(d * du), grad_B + n0 * d * du, grad_limit, status, s);
         if (rc != TTC_LQR_OK) return rc;
-        rc = launch_headsum(gQg, nc, H / 8, (int)dd, grad_Q + n0 * dd, grad_limit, status, s);
+        rc = launch_headsum(gQg, nc, groups_of(H), (int)dd, grad_Q + n0 * dd, grad_limit, status, s);
         if (rc != TTC_LQR_OK) return rc;
       }
       continue;

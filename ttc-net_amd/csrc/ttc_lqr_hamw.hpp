@@ -4,8 +4,9 @@
 // The head-group rollout of lqr_ham16_mfma_kernel (the reference's forward Hamiltonian
 // differentiation, ttc/solvers/symplectic_iter.py:764-885, rolled from lambda_1 = V_1 h_1;
 // same recursion, certificate and outputs as lqr_ham_bwd_kernel) widened to D = 16 NW.
-// A workgroup of NW waves rolls one head group: 8 consecutive heads of one token (H % 8 == 0),
-// primal and adjoint, i.e. 16 trajectories.  Wave I owns state rows 16I..16I+15 of all 16
+// A workgroup of NW waves rolls one head group: 8 consecutive heads of one token (RAG: up to 8; the
+// token's last group takes what is left, its idle columns carry the last problem's constants with
+// h_0 = u_0 = d_u = 0, stay zero and are not stored), primal and adjoint, i.e. 16 trajectories.  Wave I owns state rows 16I..16I+15 of all 16
 // trajectories in the MFMA C layout (lane (g, c) holds rows 16I+4g..16I+4g+3 of trajectory
 // c; trajectory c is problem c & 7, adjoint when c >= 8).
 //
@@ -92,7 +93,8 @@ __device__ __forceinline__ void half_cross_blocks(const float* Xi, const float* 
   }
 }
 
-template <int D, bool DIRECT>
+// DIRECT: one group per token (H <= 8), which writes the token's sums.
+template <int D, bool DIRECT, bool RAG>
 __global__ __launch_bounds__(HamW<D>::THREADS) __attribute__((amdgpu_waves_per_eu(HamW<D>::MINW))) void lqr_hamw_mfma_kernel(
     const float* __restrict__ A_diag, const float* __restrict__ Bg, const float* __restrict__ Qg,
     const float* __restrict__ Rinv, const float* __restrict__ Qf, const float* __restrict__ lgA,
@@ -115,10 +117,15 @@ __global__ __launch_bounds__(HamW<D>::THREADS) __attribute__((amdgpu_waves_per_e
   const bool adj = c >= 8;
   const int r0 = 16 * I + 4 * g;  // first of my four state rows
   const int64_t G = blockIdx.x;
-  if (G * 8 >= P) return;         // whole workgroups only: no barrier follows
-  const int64_t p0 = G * 8;
-  const int64_t n = p0 / H;       // the group's token
-  const int64_t p = p0 + j;
+  const int gpt = RAG ? (H + 7) / 8 : H / 8;  // groups per token
+  const int64_t n = G / gpt;      // the group's token
+  if (n * H >= P) return;         // whole workgroups only: no barrier follows
+  const int64_t p0 = RAG ? n * H + 8 * (G - n * gpt) : G * 8;
+  // its problems; rows and columns beyond them repeat the last one's constants
+  const int cnt = RAG ? ((int)(n * H + H - p0) < 8 ? (int)(n * H + H - p0) : 8) : 8;
+  auto clampj = [&](int k) { return RAG && k >= cnt ? cnt - 1 : k; };
+  const bool live = !RAG || j < cnt;
+  const int64_t p = p0 + clampj(j);
   // row layout: D lanes per problem, PPP problems per wave and pass, two passes
   const int li = lane % D;
   const int slot = lane / D;
@@ -136,10 +143,10 @@ __global__ __launch_bounds__(HamW<D>::THREADS) __attribute__((amdgpu_waves_per_e
 #pragma unroll 1
   for (int pa = 0; pa < 2; ++pa) {
     const int jj = (pa * NW + I) * W::PPP + slot;
-    const int64_t pp = p0 + jj;
+    const int64_t pp = p0 + clampj(jj);
     float aug[D + 4];
     ld_global_row<D>(q0s + (pp * D + li) * D, *reinterpret_cast<float(*)[D]>(aug));
-    aug[D] = dU[pp * D + li];
+    aug[D] = RAG && jj >= cnt ? 0.f : dU[pp * D + li];
     aug[D + 1] = aug[D + 2] = aug[D + 3] = 0.f;
     float piv;
     int pos;
@@ -163,8 +170,9 @@ __global__ __launch_bounds__(HamW<D>::THREADS) __attribute__((amdgpu_waves_per_e
     }
   }
   const float la2 = lgA[p] * kLog2e;
-  v4f U = adj ? ld4(TS + c * LDT + r0) : ld4(u0g + p * D + r0);  // u_0 | w_0
-  v4f S = adj ? v4f{0.f, 0.f, 0.f, 0.f} : ld4(h0 + p * D + r0);   // h_0 | h~_0 = 0
+  const v4f zero4 = v4f{0.f, 0.f, 0.f, 0.f};
+  v4f U = adj ? ld4(TS + c * LDT + r0) : live ? ld4(u0g + p * D + r0) : zero4;  // u_0 | w_0
+  v4f S = adj || !live ? zero4 : ld4(h0 + p * D + r0);                          // h_0 | h~_0 = 0
   // matrix blocks [I][J] of the token as A operands: B, B', sym(Q)
   float Bm[NW][4], Bt[NW][4], Qa[NW][4];
   {
@@ -202,7 +210,7 @@ __global__ __launch_bounds__(HamW<D>::THREADS) __attribute__((amdgpu_waves_per_e
 #pragma unroll 1
   for (int pa = 0; pa < 2; ++pa) {
     const int jj = (pa * NW + I) * W::PPP + slot;
-    const int64_t pp = p0 + jj;
+    const int64_t pp = p0 + clampj(jj);
     float lam = 0.f, lamb = 0.f;
 #pragma unroll
     for (int k0 = 0; k0 < D; k0 += 16) {
@@ -374,7 +382,7 @@ __global__ __launch_bounds__(HamW<D>::THREADS) __attribute__((amdgpu_waves_per_e
   float gmax = 0.f;  // largest guarded gradient magnitude of the lane
 #pragma unroll 1
   for (int pa = 0; pa < 2; ++pa) {
-    const int jj = (pa * NW + I) * W::PPP + slot;
+    const int jj = clampj((pa * NW + I) * W::PPP + slot);  // (idle rows store the last problem's values again)
     const int64_t pp = p0 + jj;
     const float* hs = TS + jj * LDT;
     const float* hbs = TS + (8 + jj) * LDT;
@@ -448,7 +456,7 @@ __global__ __launch_bounds__(HamW<D>::THREADS) __attribute__((amdgpu_waves_per_e
   // Past the certificate every output of the group is finite (their magnitudes sum to the
   // finite `fin`), so the guard reduces to the largest magnitude against the limit.  The
   // reference's guard covers A_diag, B, Q, R_inv, Q_f and h0, not the log-discounts.
-  if (!adj) {
+  if (!adj && live) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) gmax = fmaxf(gmax, fmaxf(fabsf(fA[k]), fmaxf(fabsf(fR[k]), fabsf(fH0[k]))));
     st4(gA + p * D + r0, fA);
@@ -485,16 +493,20 @@ int launch_hamw_mfma_t(const float* A, const float* B, const float* Q, const flo
                        float* gBg, float* gQg, float limit, int32_t* fail_list, int32_t* fail_count,
                        int32_t* status, hipStream_t s) {
   if (P <= 0) return TTC_LQR_OK;
-  if (H % 8 != 0 || P % 8 != 0) return TTC_LQR_EINVAL;
-  const dim3 grid((unsigned)(P / 8)), block(HamW<D>::THREADS);
-  if (H == 8)
-    hipLaunchKernelGGL((lqr_hamw_mfma_kernel<D, true>), grid, block, HamW<D>::LDS_BYTES, s, A, B, Q, R, Qf, lA, lB,
-                       lQ, h0, u0, dU, v1s, q0s, P, H, T, tau, gA, gR, gQf, glA, glB, glQ, gh0, gBg, gQg, limit,
-                       fail_list, fail_count, status);
-  else
-    hipLaunchKernelGGL((lqr_hamw_mfma_kernel<D, false>), grid, block, HamW<D>::LDS_BYTES, s, A, B, Q, R, Qf, lA,
-                       lB, lQ, h0, u0, dU, v1s, q0s, P, H, T, tau, gA, gR, gQf, glA, glB, glQ, gh0, gBg, gQg, limit,
-                       fail_list, fail_count, status);
+  const dim3 grid((unsigned)(P / H * ((H + 7) / 8))), block(HamW<D>::THREADS);
+  auto run = [&](auto direct, auto rag) {
+    hipLaunchKernelGGL((lqr_hamw_mfma_kernel<D, decltype(direct)::value, decltype(rag)::value>), grid, block,
+                       HamW<D>::LDS_BYTES, s, A, B, Q, R, Qf, lA, lB, lQ, h0, u0, dU, v1s, q0s, P, H, T, tau, gA, gR,
+                       gQf, glA, glB, glQ, gh0, gBg, gQg, limit, fail_list, fail_count, status);
+  };
+  using Yes = std::true_type;
+  using No = std::false_type;
+  if (H == 8) run(Yes{}, No{});
+  else if (H % 8 == 0) run(No{}, No{});
+  else if constexpr (D == 64) {
+    if (H < 8) run(Yes{}, Yes{});
+    else run(No{}, Yes{});
+  } else return TTC_LQR_EINVAL;
   return hipGetLastError() == hipSuccess ? TTC_LQR_OK : TTC_LQR_ELAUNCH;
 }
 

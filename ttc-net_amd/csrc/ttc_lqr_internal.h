@@ -122,7 +122,8 @@ int launch_ham16_mfma(const float* A, const float* B, const float* Q, const floa
                       float* gA, float* gR, float* gQf, float* glA, float* glB, float* glQ, float* gh0,
                       float* gBg, float* gQg, float limit, int32_t* fail_list, int32_t* fail_count,
                       int32_t* status, hipStream_t s);
-// the same for d = 32 / 64 (d / 16 waves per head group; ttc_lqr_hamw.hpp)
+// the same for d = 32 / 64 (d / 16 waves per head group; ttc_lqr_hamw.hpp); d = 64 takes any head count, in
+// ceil(H / 8) groups of up to 8 heads per token (H <= 8: a group is a token)
 int launch_ham32_mfma(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                       const float* lA, const float* lB, const float* lQ, const float* h0, const float* u0,
                       const float* dU, const float* v1s, const float* q0s, int64_t P, int H, int T, float tau,
