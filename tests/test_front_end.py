@@ -87,3 +87,24 @@ def test_cpu_and_other_dtypes_use_the_operators():
         x = _proj(2, *dims, dt, "cpu")
         for u, v in zip(front_end(x, None, dims), front_end_torch(x, None, dims)):
             assert u.dtype == dt and torch.equal(u, v)
+
+
+@pytest.mark.gpu
+def test_no_grad_forward_writes_no_stash(monkeypatch):
+    """Under no_grad a layer whose parameters require gradients runs the forward without a stash (nothing
+    asks whether one fits), with the same bits as a recorded forward."""
+    from ttc import TTCLayer
+    from ttc.solvers import hip_lqr as hl
+    torch.manual_seed(0)
+    x = torch.randn(64, 32, device="cuda")
+    asked = []
+    fits = hl._stash_fits
+    monkeypatch.setattr(hl, "_stash_fits", lambda *a: asked.append(a) or fits(*a))
+    for factored in (True, False):
+        layer = TTCLayer(32, 32, 16, 8, 16, 16, factored=factored).cuda()
+        y = layer(x, T=8)
+        assert asked
+        asked.clear()
+        with torch.no_grad():
+            assert torch.equal(y, layer(x, T=8))
+        assert not asked

@@ -19,7 +19,7 @@ from __future__ import annotations
 
 import torch
 
-from .hip_lqr import HipLQRSolveFunc
+from .hip_lqr import HipLQRSolveFunc, _recorded
 
 __all__ = ["fused_lqr_solve", "FusedLQRSolveFunc"]
 
@@ -42,4 +42,5 @@ def fused_lqr_solve(A_diag, B, Q, R_inv_diag, Q_f, gamma_A, gamma_B, gamma_Q, h0
     """First optimal action ``u [N,H,du]`` of every (token, head) problem (reference
     ``fused_lqr_solve``, ``fused_lqr.py:294-304``); ``gamma_*`` are the log-discounts.  As in the
     reference, ``inv_guard`` lands in ``FusedLQRSolveFunc``'s ``cache_level`` slot."""
-    return FusedLQRSolveFunc.apply(A_diag, B, Q, R_inv_diag, Q_f, gamma_A, gamma_B, gamma_Q, h0, T, inv_guard)
+    ins = _recorded(A_diag, B, Q, R_inv_diag, Q_f, gamma_A, gamma_B, gamma_Q, h0)
+    return FusedLQRSolveFunc.apply(*ins, T, inv_guard)

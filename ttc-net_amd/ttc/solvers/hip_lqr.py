@@ -417,8 +417,18 @@ def hip_lqr_solve(A_diag: torch.Tensor, B: torch.Tensor, Q: torch.Tensor, R_inv_
     synchronisation in the forward, so it can be recorded by HIP graph capture) and raises the same
     ``RuntimeError`` from the backward or from :func:`check_deferred_status`.
     """
-    return HipLQRSolveFunc.apply(A_diag, B, Q, R_inv_diag, Q_f, log_gamma_A, log_gamma_B, log_gamma_Q, h0, T,
-                                 grad_limit, stash, precision, stable_backward, status_check)
+    ins = _recorded(A_diag, B, Q, R_inv_diag, Q_f, log_gamma_A, log_gamma_B, log_gamma_Q, h0)
+    return HipLQRSolveFunc.apply(*ins, T, grad_limit, stash, precision, stable_backward, status_check)
+
+
+def _recorded(*ins):
+    """The inputs of an autograd Function, detached where autograd does not record (``torch.no_grad``): the
+    Function's ``needs_input_grad`` is their ``requires_grad`` in either mode, so that a layer's
+    parameters would have the forward write a stash (and the expanded ``B``, ``Q``, ``Q_f``) that no
+    backward reads.  Forward-mode tangents, which the Functions refuse, are left on."""
+    if torch.is_grad_enabled() or torch.autograd.forward_ad._current_level >= 0:
+        return ins
+    return tuple(x.detach() for x in ins)
 
 
 def _workspace_budget(dev) -> int:
@@ -635,6 +645,6 @@ def hip_lqr_solve_factored(A_diag, coeff_B, coeff_Q, R_inv_diag, coeff_Qf, log_g
     """``hip_lqr_solve`` on the layer's low-rank factors (see :class:`HipLQRFactoredFunc`):
     equal to ``hip_lqr_solve(A_diag, einsum(coeff_B, B_basis), einsum(coeff_Q, Q_basis), R_inv,
     einsum(coeff_Qf, Q_basis), ...)`` with gradients for the coefficients and both bases."""
-    return HipLQRFactoredFunc.apply(A_diag, coeff_B, coeff_Q, R_inv_diag, coeff_Qf, log_gamma_A, log_gamma_B,
-                                    log_gamma_Q, h0, B_basis, Q_basis, T, grad_limit, stash, precision,
-                                    stable_backward, rescale, status_check)
+    ins = _recorded(A_diag, coeff_B, coeff_Q, R_inv_diag, coeff_Qf, log_gamma_A, log_gamma_B, log_gamma_Q, h0, B_basis,
+                    Q_basis)
+    return HipLQRFactoredFunc.apply(*ins, T, grad_limit, stash, precision, stable_backward, rescale, status_check)
