@@ -90,6 +90,31 @@ def test_cpu_and_other_dtypes_use_the_operators():
 
 
 @pytest.mark.gpu
+def test_transforms_and_tracing_see_the_operators():
+    """vmap, forward-mode AD (both interfaces), tracing and fake tensors, which see nothing of an autograd
+    Function, get the operators' results (the same formulas, so the same bits)."""
+    import torch.autograd.forward_ad as fwAD
+    dims = (2, 6, 5, 3, 4)
+    x = _proj(3, *dims, torch.float32, "cuda")
+    v = torch.linspace(-1, 1, x.numel(), device="cuda").reshape(x.shape)
+    for k in (0, 2, 3, 8):
+        want = torch.func.jvp(lambda t: front_end_torch(t, None, dims)[k], (x,), (v,))
+        got = torch.func.jvp(lambda t: front_end(t, None, dims)[k], (x,), (v,))
+        assert all(torch.equal(p, q) for p, q in zip(got, want))
+        with fwAD.dual_level():
+            y = fwAD.unpack_dual(front_end(fwAD.make_dual(x, v), None, dims)[k])
+            assert torch.equal(y.tangent, want[1])
+    xs = torch.stack([x, 2 * x])
+    want = torch.func.vmap(lambda t: front_end_torch(t, None, dims)[3])(xs)
+    assert torch.equal(torch.func.vmap(lambda t: front_end(t, None, dims)[3])(xs), want)
+    traced = torch.jit.trace(lambda t: front_end(t, None, dims)[3], x)
+    assert torch.allclose(traced(2 * x), want[1], rtol=1e-5, atol=0)
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode() as mode:
+        assert front_end(mode.from_tensor(x), None, dims)[3].shape == (3, 2, 5)
+
+
+@pytest.mark.gpu
 def test_no_grad_forward_writes_no_stash(monkeypatch):
     """Under no_grad a layer whose parameters require gradients runs the forward without a stash (nothing
     asks whether one fits), with the same bits as a recorded forward."""

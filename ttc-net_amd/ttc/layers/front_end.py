@@ -3,8 +3,9 @@ the split of the projection, ``l2norm`` / softplus / clamp and the log-discounts
 
 :func:`front_end` takes the projection ``[N, row]`` and returns ``(A_diag, coeff_B, coeff_Q, R_inv,
 coeff_Qf, log_gamma_A, log_gamma_B, log_gamma_Q, h0)``.  fp32 CUDA projections go through one kernel
-each way (``ttc_lqr_front_end`` / ``_backward``, contiguous outputs); anything else runs
-:func:`front_end_torch`, the same formulas as torch operators.  The backward differentiates
+each way (``ttc_lqr_front_end`` / ``_backward``, contiguous outputs); anything else, and any call under a
+functorch transform, forward-mode AD or tracing, runs :func:`front_end_torch`, the same formulas as
+torch operators.  The backward differentiates
 :func:`front_end_torch` when it is itself recorded (``create_graph=True``), so second derivatives
 of the front-end are what autograd gives for the operators.
 """
@@ -92,9 +93,17 @@ class _FrontEndFunc(torch.autograd.Function):
         return d_proj, d_bias, None
 
 
+def _traced(*xs) -> bool:
+    """Whether operators are observed one by one (functorch transforms, forward-mode tangents, tracing and
+    compilation, tensor subclasses such as fake tensors): none of these sees into an autograd Function."""
+    return (any(type(x) not in (torch.Tensor, torch.nn.Parameter) for x in xs if x is not None)
+            or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0
+            or torch.jit.is_tracing() or torch.compiler.is_compiling())
+
+
 def front_end(proj: torch.Tensor, bias: torch.Tensor | None, dims):
     """``dims = (heads, h_dim, u_dim, b_rank, q_rank)``."""
-    if proj.is_cuda and proj.dtype == torch.float32 and proj.dim() == 2 and (
+    if not _traced(proj, bias) and proj.is_cuda and proj.dtype == torch.float32 and proj.dim() == 2 and (
             bias is None or (bias.device == proj.device and bias.dtype == torch.float32)):
         return _FrontEndFunc.apply(proj, bias, dims)
     return front_end_torch(proj, bias, dims)
