@@ -1157,3 +1157,13 @@ def test_against_reference_riccati_and_kkt_restatements(cfg, n_tok):
         print(f"   {name} vs fp64: " + " ".join(f"{k}:{v:.1e}" for k, v in ref_errs.items()), flush=True)
         assert max(errs.values()) <= TOL, (name, errs)
         assert max(ref_errs.values()) <= TOL, (name, ref_errs)
+
+
+@pytest.mark.parametrize("stable,tol", [(True, 1e-6), (False, 1e-5)])
+@pytest.mark.parametrize("n_tok,heads,T", [(1, 1, 1), (1, 3, 2), (1, 5, 3), (3, 7, 17), (5, 4, 40), (2, 9, 600)])
+def test_fp64_row_layout_backward_d16(n_tok, heads, T, stable, tol):
+    """The fp64 backward kernels whose products go by DPP: problem counts around a wave's four and a
+    workgroup's sixteen, the shortest horizons (no reverse step, one, two) and a long one.  The stable
+    path works in fp64 throughout (the outputs' fp32 rounding and their head sums, a few 2^-24); the
+    rollout starts from a V_1 and u_0 rounded to fp32, which its certificate lets grow to 1e-5 at most."""
+    check_case("fp64-row", bench_solver_inputs(n_tok, heads, 16, seed=T), T, precision="fp64", stable=stable, tol=tol)

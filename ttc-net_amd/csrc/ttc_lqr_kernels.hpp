@@ -33,6 +33,7 @@
 
 #include "ttc_lqr.h"
 #include "ttc_lqr_internal.h"
+#include "ttc_lqr_dpp64.h"
 
 
 namespace ttc {
@@ -44,15 +45,21 @@ constexpr int STASH_NONE = 0;   // u only
 constexpr int STASH_GAINS = 1;  // every gain K_t [P,T,du,d] + Quu_0 [P,du,du] (stable backward)
 constexpr int STASH_V1 = 2;     // V_1 [P,d,d] + Quu_0 [P,du,du] (fast backward)
 
-template <int D>
+template <int D, int PPB_ = (D == 16) ? 16 : (D == 32 ? 4 : 1)>
 struct Geo {
-  static constexpr int PPB = (D == 16) ? 16 : (D == 32 ? 4 : 1);  // problems per block
+  static constexpr int PPB = PPB_;  // problems per block
   static constexpr int THREADS = PPB * D;
   static constexpr int LDM = D + kPad;                  // LDS row stride (elements)
   static constexpr int MAT = D * LDM;
   static constexpr int NVEC = 12;                       // D-element vector slots per problem
   static constexpr int PER_PROB = MAT + NVEC * D + 4;   // +4 elements: bank skew between problems
 };
+
+// The backward kernels' blocks.  In fp64 at d = 16 a block is one wave: the calls are short lists of
+// problems, whose waves share a CU's load and LDS ports unless each gets a CU of its own (stable path
+// of 32 problems x 1,024 steps 2.17 -> 1.52 ms).
+template <int D, typename R>
+using BwdGeo = std::conditional_t<D == 16 && std::is_same<R, double>::value, Geo<16, 4>, Geo<D>>;
 
 // Order LDS traffic between lanes of one wave: stores before this point are
 // visible to loads after it (LDS executes one wave's requests in order).
@@ -558,8 +565,15 @@ __device__ __forceinline__ void flag_value(double v, float limit, int& flags) {
   flag_value<D>((float)v, limit, flags);
 }
 
+// Steps whose gains the fp64 d = 16 kernel has in flight, phase 1 and 2.  Its bound is one wave's
+// serial step (about 0.7 us for the two phases: 224 DPP multiply-adds, five library exponentials and
+// the loads).  32 problems x 1,024 steps: 2.88 ms with the vectors broadcast through LDS by four
+// waves of a workgroup, 2.36 with DPP, 1.52 with a wave per workgroup (its own CU's load port for the
+// gains), 1.43 with 3 and 2 steps in flight, 1.51 with 4 and 3 (accumulator registers as spill space).
+constexpr int kAhead1 = 3, kAhead2 = 2;
+
 template <int D, typename R = float>
-__global__ __launch_bounds__(Geo<D>::THREADS) void lqr_bwd_kernel(
+__global__ __launch_bounds__((BwdGeo<D, R>::THREADS)) void lqr_bwd_kernel(
     const float* __restrict__ A_diag, const float* __restrict__ Bg, const float* __restrict__ Qg,
     const float* __restrict__ Rinv, const float* __restrict__ Qf, const float* __restrict__ lgA,
     const float* __restrict__ lgB, const float* __restrict__ lgQ, const float* __restrict__ h0,
@@ -570,7 +584,7 @@ __global__ __launch_bounds__(Geo<D>::THREADS) void lqr_bwd_kernel(
     float* __restrict__ gBp, float* __restrict__ gQp, float grad_limit, int* __restrict__ status,
     const int32_t* __restrict__ gidx = nullptr, const double* __restrict__ gsl = nullptr,
     const double* __restrict__ q0sl = nullptr) {
-  using G = Geo<D>;
+  using G = BwdGeo<D, R>;
   extern __shared__ __align__(16) float smem_f[];
   R* const smem = reinterpret_cast<R*>(smem_f);
   const R* const kst = reinterpret_cast<const R*>(kstash);  // gains K_t in the forward sweep's type
@@ -619,16 +633,9 @@ __global__ __launch_bounds__(Geo<D>::THREADS) void lqr_bwd_kernel(
   const R lgB_i = lgB[p * D + li];
   const R lgQ_i = lgQ[p * D + li];
   const R lgA_p = lgA[p];
-  R Brow[D], Bcol[D], Qrow[D];
-  {
-    const float* qg = Qg + n * D * D;
+  R Brow[D];
 #pragma unroll
-    for (int c = 0; c < D; ++c) {
-      Brow[c] = Bs[li * G::LDM + c];
-      Bcol[c] = Bs[c * G::LDM + li];
-      Qrow[c] = R(0.5) * (qg[li * D + c] + qg[c * D + li]);
-    }
-  }
+  for (int c = 0; c < D; ++c) Brow[c] = Bs[li * G::LDM + c];
 
   // adjoint feed-forward at t = 0: w0 = -Quu_0^{-1} d_u
   R w0_i;
@@ -647,53 +654,78 @@ __global__ __launch_bounds__(Geo<D>::THREADS) void lqr_bwd_kernel(
     wave_sync();
   }
 
-  // phase 1: rollouts, t = 0..T-1.  At d = 16 each step's gain row is loaded one step ahead
-  // (in fp64 a wave runs alone on its SIMD, so nothing else hides the load's latency); at
-  // d = 32 / 64 the extra registers would spill.
+  // phase 1: rollouts, t = 0..T-1.  At d = 16 the gain rows are loaded ahead of their steps (in fp64 a
+  // wave runs alone on its SIMD, so nothing else hides a load's latency): kAhead1 rows in flight in
+  // fp64, one in fp32; at d = 32 / 64 the extra registers would spill.
   constexpr bool PF = D == 16;
+  constexpr bool DPP = D == 16 && std::is_same<R, double>::value;  // products by DPP, not through LDS
+  constexpr int A1 = DPP ? kAhead1 : 1, A2 = DPP ? kAhead2 : 1;
   R h_i = h0[p * D + li];
   R hb_i = R(0);
-  R knext[PF ? D : 1];
-  if constexpr (PF) ld_global_row<D>(kp + li * D, knext);
-  for (int t = 0; t < T; ++t) {
+  R kn[A1][PF ? D : 1];
+  if constexpr (PF) {
+#pragma unroll
+    for (int a = 0; a < A1; ++a) ld_global_row<D>(kp + ((int64_t)(a < T ? a : T - 1) * D + li) * D, kn[a]);
+  }
+  auto roll = [&](const int t, R(&next)[PF ? D : 1]) {
     const R tp1 = (R)(t + 1);
     const R alpha_i = fma(a_i, exp(lgA_p * tp1), R(1));
     const R beta_i = exp(lgB_i * tp1);
     R krow[D];
     if constexpr (PF) {
 #pragma unroll
-      for (int c = 0; c < D; ++c) krow[c] = knext[c];
-      if (t + 1 < T) ld_global_row<D>(kp + ((int64_t)(t + 1) * D + li) * D, knext);
+      for (int c = 0; c < D; ++c) krow[c] = next[c];
+      if (t + A1 < T) ld_global_row<D>(kp + ((int64_t)(t + A1) * D + li) * D, next);
     }
-    v0[li] = h_i;
-    v1[li] = hb_i;
-    wave_sync();
-    R hv[D], hbv[D];
-    ld_row<D>(v0, hv);
-    ld_row<D>(v1, hbv);
-    if constexpr (!PF) ld_global_row<D>(kp + ((int64_t)t * D + li) * D, krow);
     R u_i = R(0), w_i = (t == 0) ? w0_i : R(0);
-#pragma unroll
-    for (int c = 0; c < D; ++c) {
-      u_i = fma(krow[c], hv[c], u_i);
-      w_i = fma(krow[c], hbv[c], w_i);
-    }
-    v2[li] = beta_i * u_i;
-    v3[li] = beta_i * w_i;
-    wave_sync();
-    R bu[D], bw[D];
-    ld_row<D>(v2, bu);
-    ld_row<D>(v3, bw);
     R hn = alpha_i * h_i, hbn = alpha_i * hb_i;
+    if constexpr (DPP) {
+      dpp_dot2(u_i, w_i, krow, h_i, hb_i);
+      dpp_dot2(hn, hbn, Brow, beta_i * u_i, beta_i * w_i);
+    } else {
+      v0[li] = h_i;
+      v1[li] = hb_i;
+      wave_sync();
+      R hv[D], hbv[D];
+      ld_row<D>(v0, hv);
+      ld_row<D>(v1, hbv);
+      if constexpr (!PF) ld_global_row<D>(kp + ((int64_t)t * D + li) * D, krow);
 #pragma unroll
-    for (int j = 0; j < D; ++j) {
-      hn = fma(Brow[j], bu[j], hn);
-      hbn = fma(Brow[j], bw[j], hbn);
+      for (int c = 0; c < D; ++c) {
+        u_i = fma(krow[c], hv[c], u_i);
+        w_i = fma(krow[c], hbv[c], w_i);
+      }
+      v2[li] = beta_i * u_i;
+      v3[li] = beta_i * w_i;
+      wave_sync();
+      R bu[D], bw[D];
+      ld_row<D>(v2, bu);
+      ld_row<D>(v3, bw);
+#pragma unroll
+      for (int j = 0; j < D; ++j) {
+        hn = fma(Brow[j], bu[j], hn);
+        hbn = fma(Brow[j], bw[j], hbn);
+      }
     }
     if (valid) traj[((int64_t)p * T + t) * D + li] = mk4<R>(h_i, hb_i, u_i, w_i);
     h_i = hn;
     hb_i = hbn;
-    wave_sync();
+    if constexpr (!DPP) wave_sync();
+  };
+  for (int t0 = 0; t0 < T; t0 += A1) {
+#pragma unroll
+    for (int a = 0; a < A1; ++a)
+      if (t0 + a < T) roll(t0 + a, kn[a]);  // uniform
+  }
+
+  R Bcol[D], Qrow[D];
+  {
+    const float* qg = Qg + n * D * D;
+#pragma unroll
+    for (int c = 0; c < D; ++c) {
+      Bcol[c] = Bs[c * G::LDM + li];
+      Qrow[c] = R(0.5) * (qg[li * D + c] + qg[c * D + li]);
+    }
   }
 
   // phase 2: costates lambda_{t+1}, gradients, t = T-1..0
@@ -725,30 +757,29 @@ __global__ __launch_bounds__(Geo<D>::THREADS) void lqr_bwd_kernel(
 #pragma unroll
   for (int c = 0; c < D; ++c) { gBrow[c] = R(0); gQrow[c] = R(0); }
 
-  // at d = 16 the step's trajectory entry and gain column are loaded one step ahead, as in phase 1
-  auto trn = traj[((int64_t)p * T + (T - 1)) * D + li];
-  R kcn[PF ? D : 1];
+  // at d = 16 the steps' trajectory entries and gain columns are loaded ahead, as in phase 1
+  typename Traj4<R>::type trn[A2];
+  R kcn[A2][PF ? D : 1];
   if constexpr (PF) {
 #pragma unroll
-    for (int c = 0; c < D; ++c) kcn[c] = R(0);
-    if (T - 1 >= 1) {
+    for (int a = 0; a < A2; ++a) {
+      const int64_t t = T - 1 - a > 0 ? T - 1 - a : 0;
+      trn[a] = traj[((int64_t)p * T + t) * D + li];
 #pragma unroll
-      for (int c = 0; c < D; ++c) kcn[c] = kp[((int64_t)(T - 1) * D + c) * D + li];  // K_{T-1}[c, li]
+      for (int c = 0; c < D; ++c) kcn[a][c] = kp[(t * D + c) * D + li];  // K_t[c, li]
     }
   }
-  for (int t = T - 1; t >= 0; --t) {
-    const auto tr = PF ? trn : traj[((int64_t)p * T + t) * D + li];
+  auto back = [&](const int t, typename Traj4<R>::type& trx, R(&next)[PF ? D : 1]) {
+    const auto tr = PF ? trx : traj[((int64_t)p * T + t) * D + li];
     const R h_t = tr.x, hb_t = tr.y, u_i = tr.z, w_i = tr.w;
     R kcol[D];
     if constexpr (PF) {
 #pragma unroll
-      for (int c = 0; c < D; ++c) kcol[c] = kcn[c];
-      if (t >= 1) {  // uniform
-        trn = traj[((int64_t)p * T + (t - 1)) * D + li];
-        if (t - 1 >= 1) {
+      for (int c = 0; c < D; ++c) kcol[c] = next[c];
+      if (t >= A2) {  // uniform
+        trx = traj[((int64_t)p * T + (t - A2)) * D + li];
 #pragma unroll
-          for (int c = 0; c < D; ++c) kcn[c] = kp[((int64_t)(t - 1) * D + c) * D + li];
-        }
+        for (int c = 0; c < D; ++c) next[c] = kp[((int64_t)(t - A2) * D + c) * D + li];
       }
     }
     const R tp1 = (R)(t + 1);
@@ -759,50 +790,63 @@ __global__ __launch_bounds__(Geo<D>::THREADS) void lqr_bwd_kernel(
     const R gAt = fma(h_t, lamb_i, hb_t * lam_i);
     gA_i = fma(gAt, eA, gA_i);
     glgA_part = fma(gAt * a_i, tp1 * eA, glgA_part);
-    v0[li] = lam_i;
-    v1[li] = lamb_i;
-    v2[li] = beta_i * u_i;
-    v3[li] = beta_i * w_i;
-    wave_sync();
-    R lv[D], lbv[D], bu[D], bw[D];
-    ld_row<D>(v0, lv);
-    ld_row<D>(v1, lbv);
-    ld_row<D>(v2, bu);
-    ld_row<D>(v3, bw);
     // B: lamb u' + lam w' (torch_lqr.py:53), chained through B_t = B diag(beta_t)
     R btl = R(0), btlb = R(0);
+    if constexpr (DPP) {
+      dpp_dot2(btl, btlb, Bcol, lam_i, lamb_i);
+      dpp_outer2(gBrow, beta_i * w_i, lam_i, beta_i * u_i, lamb_i);
+    } else {
+      v0[li] = lam_i;
+      v1[li] = lamb_i;
+      v2[li] = beta_i * u_i;
+      v3[li] = beta_i * w_i;
+      wave_sync();
+      R lv[D], lbv[D], bu[D], bw[D];
+      ld_row<D>(v0, lv);
+      ld_row<D>(v1, lbv);
+      ld_row<D>(v2, bu);
+      ld_row<D>(v3, bw);
 #pragma unroll
-    for (int c = 0; c < D; ++c) {
-      gBrow[c] = fma(lamb_i, bu[c], fma(lam_i, bw[c], gBrow[c]));
-      btl = fma(Bcol[c], lv[c], btl);
-      btlb = fma(Bcol[c], lbv[c], btlb);
+      for (int c = 0; c < D; ++c) {
+        gBrow[c] = fma(lamb_i, bu[c], fma(lam_i, bw[c], gBrow[c]));
+        btl = fma(Bcol[c], lv[c], btl);
+        btlb = fma(Bcol[c], lbv[c], btlb);
+      }
     }
     glgB_i = fma(tp1 * beta_i, fma(u_i, btlb, w_i * btl), glgB_i);
     // R = 1/R_inv:  d/dR_inv = -(u w) / R_inv^2   (torch_lqr.py:59)
     gr_i = fma(-u_i * w_i, rr_i * rr_i, gr_i);
     if (t >= 1) {
       const R q_i = exp(lgQ_i * (R)t);
-      // closed-loop correction c = R u + B_t' lambda_{t+1}
-      v4[li] = q_i * h_t;
-      v5[li] = q_i * hb_t;
-      v6[li] = fma(u_i, rr_i, beta_i * btl);
-      v7[li] = fma(w_i, rr_i, beta_i * btlb);
-      wave_sync();
-      R qh[D], qhb[D], cu[D], cw[D];
-      ld_row<D>(v4, qh);
-      ld_row<D>(v5, qhb);
-      ld_row<D>(v6, cu);
-      ld_row<D>(v7, cw);
+      // closed-loop correction c = R u + B_t' lambda_{t+1}; Q_t = D_t Q D_t:  gradient
+      // D_t sym(h hb') D_t  (torch_lqr.py:55)
+      const R cu_i = fma(u_i, rr_i, beta_i * btl), cw_i = fma(w_i, rr_i, beta_i * btlb);
       R Qh = R(0), Qhb = R(0), kcu = R(0), kcw = R(0);
+      if constexpr (DPP) {
+        const R qh_i = q_i * h_t, qhb_i = q_i * hb_t;
+        dpp_dot2(Qh, Qhb, Qrow, qh_i, qhb_i);
+        dpp_dot2(kcu, kcw, kcol, cu_i, cw_i);
+        dpp_outer2(gQrow, qh_i, R(0.5) * qhb_i, qhb_i, R(0.5) * qh_i);
+      } else {
+        v4[li] = q_i * h_t;
+        v5[li] = q_i * hb_t;
+        v6[li] = cu_i;
+        v7[li] = cw_i;
+        wave_sync();
+        R qh[D], qhb[D], cu[D], cw[D];
+        ld_row<D>(v4, qh);
+        ld_row<D>(v5, qhb);
+        ld_row<D>(v6, cu);
+        ld_row<D>(v7, cw);
 #pragma unroll
-      for (int c = 0; c < D; ++c) {
-        Qh = fma(Qrow[c], qh[c], Qh);
-        Qhb = fma(Qrow[c], qhb[c], Qhb);
-        // Q_t = D_t Q D_t:  gradient D_t sym(h hb') D_t  (torch_lqr.py:55)
-        gQrow[c] = fma(R(0.5) * q_i, fma(h_t, qhb[c], hb_t * qh[c]), gQrow[c]);
-        const R kji = PF ? kcol[c] : kp[((int64_t)t * D + c) * D + li];  // K_t[c, li]
-        kcu = fma(kji, cu[c], kcu);
-        kcw = fma(kji, cw[c], kcw);
+        for (int c = 0; c < D; ++c) {
+          Qh = fma(Qrow[c], qh[c], Qh);
+          Qhb = fma(Qrow[c], qhb[c], Qhb);
+          gQrow[c] = fma(R(0.5) * q_i, fma(h_t, qhb[c], hb_t * qh[c]), gQrow[c]);
+          const R kji = PF ? kcol[c] : kp[((int64_t)t * D + c) * D + li];  // K_t[c, li]
+          kcu = fma(kji, cu[c], kcu);
+          kcw = fma(kji, cw[c], kcw);
+        }
       }
       Qh *= q_i;
       Qhb *= q_i;
@@ -812,7 +856,12 @@ __global__ __launch_bounds__(Geo<D>::THREADS) void lqr_bwd_kernel(
     } else {
       gh0_i = alpha_i * lamb_i;  // torch_lqr.py:61 (lambda_0 = A_0' lambda_1)
     }
-    wave_sync();
+    if constexpr (!DPP) wave_sync();
+  };
+  for (int t0 = T - 1; t0 >= 0; t0 -= A2) {
+#pragma unroll
+    for (int a = 0; a < A2; ++a)
+      if (t0 - a >= 0) back(t0 - a, trn[a], kcn[a]);  // uniform
   }
   const R glgA_p = group_sum<D>(glgA_part, v0, li);
   // the reference's guard covers A_diag, B, Q, R_inv, Q_f and h0 (B and Q: the head sums,
@@ -871,7 +920,7 @@ __device__ __forceinline__ double rcpr(double x) { return 1.0 / x; }
 #define TTC_HAM64_WAVES 2  // waves per SIMD of the fp64 rollout (registers capped; its loop keeps them all)
 #endif
 template <int D, typename R = float, bool LISTED = false>
-__global__ __launch_bounds__(Geo<D>::THREADS)
+__global__ __launch_bounds__((BwdGeo<D, R>::THREADS))
 __attribute__((amdgpu_waves_per_eu(std::is_same<R, double>::value ? TTC_HAM64_WAVES : 1))) void lqr_ham_bwd_kernel(
     const float* __restrict__ A_diag, const float* __restrict__ Bg, const float* __restrict__ Qg,
     const float* __restrict__ Rinv, const float* __restrict__ Qf, const float* __restrict__ lgA,
@@ -883,7 +932,7 @@ __attribute__((amdgpu_waves_per_eu(std::is_same<R, double>::value ? TTC_HAM64_WA
     float grad_limit, int* __restrict__ fail_list, int* __restrict__ fail_count, int* __restrict__ status,
     const int* __restrict__ plist, const int32_t* __restrict__ slot_of, const double* __restrict__ slots,
     int64_t nslot) {
-  using G = Geo<D>;
+  using G = BwdGeo<D, R>;
   extern __shared__ __align__(16) float smem_f[];
   R* const smem = reinterpret_cast<R*>(smem_f);
   const int li = threadIdx.x % D;
@@ -1038,24 +1087,31 @@ __attribute__((amdgpu_waves_per_eu(std::is_same<R, double>::value ? TTC_HAM64_WA
     wave_sync();
   }
 
+  // products by DPP, not through LDS: 0.90 -> 0.60 ms for a short list's 1,024 steps
+  constexpr bool DPP = D == 16 && std::is_same<R, double>::value;
   for (int t = 1; t < T; ++t) {
     const R tf = (R)t;
     // state cost on h_t:  Qc_t = D_t Q D_t,  D_t = diag(exp(lgQ t))   (torch_lqr.py:55 + chain rule)
     const R q_i = exp2r(lq2_i * tf);
     const R qh_i = q_i * h_i, qhb_i = q_i * hb_i;
-    v0[li] = qh_i;
-    v1[li] = qhb_i;
-    wave_sync();
-    R qh[D], qhb[D];
-    ld_row<D>(v0, qh);
-    ld_row<D>(v1, qhb);
     R Qh = R(0), Qhb = R(0);
+    // with twice the symmetric gradient of Qc_t (halved after the loop)
+    if constexpr (DPP) {
+      dpp_dot2(Qh, Qhb, Qrow, qh_i, qhb_i);
+      dpp_outer2(gQrow, qh_i, qhb_i, qhb_i, qh_i);
+    } else {
+      v0[li] = qh_i;
+      v1[li] = qhb_i;
+      wave_sync();
+      R qh[D], qhb[D];
+      ld_row<D>(v0, qh);
+      ld_row<D>(v1, qhb);
 #pragma unroll
-    for (int c = 0; c < D; ++c) {
-      Qh = fma(Qrow[c], qh[c], Qh);
-      Qhb = fma(Qrow[c], qhb[c], Qhb);
-      // twice the symmetric gradient of Qc_t (halved after the loop)
-      gQrow[c] = fma(qh_i, qhb[c], fma(qhb_i, qh[c], gQrow[c]));
+      for (int c = 0; c < D; ++c) {
+        Qh = fma(Qrow[c], qh[c], Qh);
+        Qhb = fma(Qrow[c], qhb[c], Qhb);
+        gQrow[c] = fma(qh_i, qhb[c], fma(qhb_i, qh[c], gQrow[c]));
+      }
     }
     Qh *= q_i;
     Qhb *= q_i;
@@ -1068,32 +1124,42 @@ __attribute__((amdgpu_waves_per_eu(std::is_same<R, double>::value ? TTC_HAM64_WA
     const R ia = rcpr(alpha_i);
     const R lam_n = (lam_i - Qh) * ia;
     const R lamb_n = (lamb_i - Qhb) * ia;
-    v2[li] = lam_n;
-    v3[li] = lamb_n;
-    wave_sync();
-    R lv[D], lbv[D];
-    ld_row<D>(v2, lv);
-    ld_row<D>(v3, lbv);
     R btl = R(0), btlb = R(0);
+    if constexpr (DPP) {
+      dpp_dot2(btl, btlb, Bcol, lam_n, lamb_n);
+    } else {
+      v2[li] = lam_n;
+      v3[li] = lamb_n;
+      wave_sync();
+      R lv[D], lbv[D];
+      ld_row<D>(v2, lv);
+      ld_row<D>(v3, lbv);
 #pragma unroll
-    for (int c = 0; c < D; ++c) {
-      btl = fma(Bcol[c], lv[c], btl);
-      btlb = fma(Bcol[c], lbv[c], btlb);
+      for (int c = 0; c < D; ++c) {
+        btl = fma(Bcol[c], lv[c], btl);
+        btlb = fma(Bcol[c], lbv[c], btlb);
+      }
     }
     const R u_i = -r_i * beta_i * btl;
     const R w_i2 = -r_i * beta_i * btlb;
-    v4[li] = beta_i * u_i;
-    v5[li] = beta_i * w_i2;
-    wave_sync();
-    R bu[D], bw[D];
-    ld_row<D>(v4, bu);
-    ld_row<D>(v5, bw);
     R hn = alpha_i * h_i, hbn = alpha_i * hb_i;
+    if constexpr (DPP) {
+      const R bu_i = beta_i * u_i, bw_i = beta_i * w_i2;
+      dpp_dot2(hn, hbn, Brow, bu_i, bw_i);
+      dpp_outer2(gBrow, bw_i, lam_n, bu_i, lamb_n);
+    } else {
+      v4[li] = beta_i * u_i;
+      v5[li] = beta_i * w_i2;
+      wave_sync();
+      R bu[D], bw[D];
+      ld_row<D>(v4, bu);
+      ld_row<D>(v5, bw);
 #pragma unroll
-    for (int j = 0; j < D; ++j) {
-      hn = fma(Brow[j], bu[j], hn);
-      hbn = fma(Brow[j], bw[j], hbn);
-      gBrow[j] = fma(lamb_n, bu[j], fma(lam_n, bw[j], gBrow[j]));
+      for (int j = 0; j < D; ++j) {
+        hn = fma(Brow[j], bu[j], hn);
+        hbn = fma(Brow[j], bw[j], hbn);
+        gBrow[j] = fma(lamb_n, bu[j], fma(lam_n, bw[j], gBrow[j]));
+      }
     }
     const R gAt = fma(h_i, lamb_n, hb_i * lam_n);
     gA_i = fma(gAt, eA, gA_i);
@@ -1104,7 +1170,7 @@ __attribute__((amdgpu_waves_per_eu(std::is_same<R, double>::value ? TTC_HAM64_WA
     hb_i = hbn;
     lam_i = lam_n;
     lamb_i = lamb_n;
-    wave_sync();
+    if constexpr (!DPP) wave_sync();
   }
 
 #pragma unroll
@@ -1371,16 +1437,16 @@ inline void launch_rescue_k(const float* A, const float* B, const float* Q, cons
 // ---------------------------------------------------------------------------
 // launch helpers (instantiated per D in ttc_lqr_d*.hip)
 // ---------------------------------------------------------------------------
-template <int D>
+template <typename G>
 inline int ntok_lds_for(int H) {
-  constexpr int PPB = Geo<D>::PPB;
+  constexpr int PPB = G::PPB;
   const int span = (PPB - 1) / H + 2;
   return span < PPB ? span : PPB;
 }
 
-template <int D>
+template <typename G>
 inline size_t lds_bytes(int H, size_t elem = sizeof(float)) {
-  return elem * ((size_t)ntok_lds_for<D>(H) * Geo<D>::MAT + (size_t)Geo<D>::PPB * Geo<D>::PER_PROB);
+  return elem * ((size_t)ntok_lds_for<G>(H) * G::MAT + (size_t)G::PPB * G::PER_PROB);
 }
 
 template <int D, typename RT, int SM, bool WU>
@@ -1388,8 +1454,8 @@ inline void launch_fwd_k(const float* A, const float* B, const float* Q, const f
                          const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H,
                          int T, float* u, float* st_a, float* st_b, int32_t* status, hipStream_t s) {
   const dim3 grid((unsigned)((P + Geo<D>::PPB - 1) / Geo<D>::PPB)), block(Geo<D>::THREADS);
-  hipLaunchKernelGGL((lqr_fwd_kernel<D, RT, SM, WU>), grid, block, lds_bytes<D>(H, sizeof(RT)), s, A, B, Q, R, Qf,
-                     lA, lB, lQ, h0, P, H, T, ntok_lds_for<D>(H), u, st_a, st_b, status);
+  hipLaunchKernelGGL((lqr_fwd_kernel<D, RT, SM, WU>), grid, block, lds_bytes<Geo<D>>(H, sizeof(RT)), s, A, B, Q, R, Qf,
+                     lA, lB, lQ, h0, P, H, T, ntok_lds_for<Geo<D>>(H), u, st_a, st_b, status);
 }
 
 // Forward launch by stash mode: sm = STASH_NONE (u), STASH_GAINS (gains + Quu_0 into
@@ -1444,14 +1510,15 @@ inline int launch_ham(const float* A, const float* B, const float* Q, const floa
                       hipStream_t s, const int32_t* plist = nullptr, const int32_t* slot_of = nullptr,
                       const double* slots = nullptr, int64_t nslot = 0) {
   if (P <= 0) return TTC_LQR_OK;
-  const dim3 grid((unsigned)((P + Geo<D>::PPB - 1) / Geo<D>::PPB)), block(Geo<D>::THREADS);
+  using G = BwdGeo<D, RT>;
+  const dim3 grid((unsigned)((P + G::PPB - 1) / G::PPB)), block(G::THREADS);
   if (plist != nullptr)
-    hipLaunchKernelGGL((lqr_ham_bwd_kernel<D, RT, true>), grid, block, lds_bytes<D>(H, sizeof(RT)), s, A, B, Q, R, Qf,
-                       lA, lB, lQ, h0, u0, dU, v1s, q0s, P, H, T, ntok_lds_for<D>(H), tau, gA, gR, gQf, glA, glB, glQ,
+    hipLaunchKernelGGL((lqr_ham_bwd_kernel<D, RT, true>), grid, block, lds_bytes<G>(H, sizeof(RT)), s, A, B, Q, R, Qf,
+                       lA, lB, lQ, h0, u0, dU, v1s, q0s, P, H, T, ntok_lds_for<G>(H), tau, gA, gR, gQf, glA, glB, glQ,
                        gh0, gBp, gQp, limit, fail_list, fail_count, status, plist, slot_of, slots, nslot);
   else
-    hipLaunchKernelGGL((lqr_ham_bwd_kernel<D, RT, false>), grid, block, lds_bytes<D>(H, sizeof(RT)), s, A, B, Q, R,
-                       Qf, lA, lB, lQ, h0, u0, dU, v1s, q0s, P, H, T, ntok_lds_for<D>(H), tau, gA, gR, gQf, glA, glB,
+    hipLaunchKernelGGL((lqr_ham_bwd_kernel<D, RT, false>), grid, block, lds_bytes<G>(H, sizeof(RT)), s, A, B, Q, R,
+                       Qf, lA, lB, lQ, h0, u0, dU, v1s, q0s, P, H, T, ntok_lds_for<G>(H), tau, gA, gR, gQf, glA, glB,
                        glQ, gh0, gBp, gQp, limit, fail_list, fail_count, status, plist, nullptr, nullptr,
                        (int64_t)0);
   return hipGetLastError() == hipSuccess ? TTC_LQR_OK : TTC_LQR_ELAUNCH;
@@ -1466,10 +1533,11 @@ inline int launch_bwd(const float* A, const float* B, const float* Q, const floa
                       float* gQp, float limit, int32_t* status, hipStream_t s, const int32_t* gidx = nullptr,
                       const double* gsl = nullptr, const double* q0sl = nullptr) {
   if (P <= 0) return TTC_LQR_OK;
-  const dim3 grid((unsigned)((P + Geo<D>::PPB - 1) / Geo<D>::PPB)), block(Geo<D>::THREADS);
-  hipLaunchKernelGGL((lqr_bwd_kernel<D, RT>), grid, block, lds_bytes<D>(H, sizeof(RT)), s, A, B, Q, R, Qf, lA, lB,
+  using G = BwdGeo<D, RT>;
+  const dim3 grid((unsigned)((P + G::PPB - 1) / G::PPB)), block(G::THREADS);
+  hipLaunchKernelGGL((lqr_bwd_kernel<D, RT>), grid, block, lds_bytes<G>(H, sizeof(RT)), s, A, B, Q, R, Qf, lA, lB,
                      lQ, h0, dU,
-                     kst, q0s, P, H, T, ntok_lds_for<D>(H), traj, gA, gR, gQf, glA, glB, glQ, gh0, gBp, gQp,
+                     kst, q0s, P, H, T, ntok_lds_for<G>(H), traj, gA, gR, gQf, glA, glB, glQ, gh0, gBp, gQp,
                      limit, status, gidx, gsl, q0sl);
   return hipGetLastError() == hipSuccess ? TTC_LQR_OK : TTC_LQR_ELAUNCH;
 }
