@@ -44,6 +44,7 @@ def metric_for(d, T):
 
 
 PEAK_FP32_MFMA = 157.3e12   # MI355X dense fp32 matrix peak (published)
+PEAK_BF16_MFMA = 2.5e15     # dense bf16
 PEAK_FP64 = 78.6e12         # MI355X fp64 peak (published; vector and matrix)
 PEAK_HBM = 8.0e12
 
@@ -422,6 +423,12 @@ def flops_fwd(d, T):
     return T * (4 * d * d * d + 2 * d ** 3)
 
 
+def fwd_peak(d):
+    """The forward sweep's matrix peak: fp32 instructions at d = 16, six bf16 products for each fp32
+    product at d = 32 and 64."""
+    return PEAK_FP32_MFMA if d == 16 else PEAK_BF16_MFMA / 6
+
+
 def flops_bwd(d, T):
     return T * (7 * d * d + 11 * d * d)
 
@@ -544,7 +551,7 @@ def main():
     achieved = F_fwd * P / (fwd_gpu_ms * 1e-3)
     fwd_bytes = 4 * (3 * d + 2 * d + d * d + 1 + d) + 4 * (d * d + d * d) / H
     traffic = traffic_from_profiles(f"lqr_fwd_cfg{args.config}")
-    kern = f"lqr_fwd_blk_kernel<{d}>" + (" (symplectic sweep)" if d in (16, 32, 64) else "")
+    kern = "lqr_sym16_kernel (symplectic sweep)" if d == 16 else f"lqr_symw_kernel<{d}> (symplectic sweep)"
     # precision="auto" at T >= 512 (d <= 32): the same fp32 matrix-core sweep, the problems its
     # certificate rejects (a few per cent) recomputed in fp64 (d = 16 on the matrix cores, d = 32
     # by the row-layout sweep); priced against the fp32 matrix peak as a whole
@@ -582,7 +589,7 @@ def main():
         "tokens_per_s_fwd": N / (fwd_gpu_ms * 1e-3),
         "fwd_bwd_tflops": (F_fwd + flops_bwd(d, T)) * P / step_s / 1e12,
         "roofline": {"bound": "mfma+fp64" if long_h else "mfma", "achieved": achieved / 1e12,
-                     "peak": PEAK_FP32_MFMA / 1e12, "unit": "TFLOP/s", "frac": achieved / PEAK_FP32_MFMA,
+                     "peak": fwd_peak(d) / 1e12, "unit": "TFLOP/s", "frac": achieved / fwd_peak(d),
                      "traffic": traffic, "kernel": kern, "flops_per_problem": F_fwd,
                      "algorithmic_bytes_per_problem": fwd_bytes},
     }
@@ -657,6 +664,7 @@ def extra_entry(cfg, tokens, dev, bf16=False):
     re_ = time_solver(ins_e, du_e, Te, 3, 1, grad_limit=ce.get("grad_limit", 1e6))
     ach = flops_fwd(de, Te) * Pe / (re_["fwd_ms"] * 1e-3)
     ach_fb = (flops_fwd(de, Te) + flops_bwd(de, Te)) * Pe / (re_["step_ms"] * 1e-3)
+    least_s = Pe * (flops_fwd(de, Te) / fwd_peak(de) + flops_bwd(de, Te) / PEAK_FP32_MFMA)
     e = {"config": f"cfg{cfg}" + ("-bf16" if bf16 else ""), "x": xs_e, "d": de, "T": Te, "heads": He,
          "problems": Pe, "storage": "bf16 (factored inputs, d_u and gradients)" if bf16 else "fp32",
          "fwd_ms": re_["fwd_ms"], "fwd_solves_per_s": Pe / (re_["fwd_ms"] * 1e-3),
@@ -664,8 +672,8 @@ def extra_entry(cfg, tokens, dev, bf16=False):
          "tokens_per_s_fwd_bwd": ins_e[0].shape[0] / (re_["step_ms"] * 1e-3),
          "bwd_fallback_problems": re_["bwd_fallback_problems"],
          "peak_mem_bytes_fwd_bwd": re_["peak_mem_bytes"],
-         "roofline_frac": ach / PEAK_FP32_MFMA, "achieved_tflops": ach / 1e12,
-         "fwd_bwd_tflops": ach_fb / 1e12, "fwd_bwd_frac": ach_fb / PEAK_FP32_MFMA,
+         "roofline_frac": ach / fwd_peak(de), "achieved_tflops": ach / 1e12,
+         "fwd_bwd_tflops": ach_fb / 1e12, "fwd_bwd_frac": least_s / (re_["step_ms"] * 1e-3),
          "traffic": None if bf16 else traffic_from_profiles(f"lqr_fwd_cfg{cfg}")}
     if Te >= 512 and de <= 32:
         # precision "auto": the fp32 symplectic sweep, its rejected problems and the backward in fp64
@@ -696,7 +704,7 @@ def full_size_entry(cfg, dev):
          "tokens_per_s_fwd_bwd": ins_f[0].shape[0] / (re_["step_ms"] * 1e-3),
          "bwd_fallback_problems": re_["bwd_fallback_problems"],
          "peak_mem_bytes_fwd_bwd": re_["peak_mem_bytes"],
-         "roofline_frac": ach / PEAK_FP32_MFMA, "achieved_tflops": ach / 1e12,
+         "roofline_frac": ach / fwd_peak(de), "achieved_tflops": ach / 1e12,
          "wall_s": None}
     del ins_f, du_f
     torch.cuda.empty_cache()

@@ -64,7 +64,8 @@ extern "C" {
 #define TTC_LQR_FLAG_FP64_RICCATI 1
 /* TTC_LQR_FLAG_ROW_KERNEL selects the row-layout (vector-ALU only) fp32 kernels -- the
  * forward sweep and the backward's Hamiltonian rollout, one problem per d lanes -- instead
- * of the matrix-core kernels (which roll the backward over head groups of 8 when H % 8 == 0).
+ * of the matrix-core kernels (which roll the backward over head groups of 8 when H % 8 == 0, at
+ * d = 64 of up to 8 when H >= 3).
  * Results agree to fp32 rounding; it serves as an independent cross-check and as a fallback. */
 #define TTC_LQR_FLAG_ROW_KERNEL 2
 /* TTC_LQR_FLAG_STABLE_BWD makes ttc_lqr_backward take the stable path for every problem
@@ -75,8 +76,7 @@ extern "C" {
  * factorisation) at every horizon step on the matrix cores, instead of the default
  * symplectic sweep (three matrix products per step, one pivoted solve at the end, a
  * conditioning certificate per problem and a row-layout recompute of the problems that
- * miss it; at d = 32 for even head counts, at d = 64 for head counts that are multiples of
- * 4, otherwise Riccati steps anyway).  Same results to fp32 rounding. */
+ * miss it).  Same results to fp32 rounding. */
 #define TTC_LQR_FLAG_RICCATI_STEPS 8
 /* TTC_LQR_FLAG_COMPACT_STASH (factored entry points only): the stash holds only the upper
  * triangle of each problem's V_1 (ttc_lqr_compact_stash_bytes: d(d+1)/2 floats per problem,
