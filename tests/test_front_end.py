@@ -53,6 +53,55 @@ def test_front_end_kernel(shape, with_bias):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(9, 2, 6, 5, 3, 4), (7, 3, 65, 3, 2, 70)])
+def test_front_end_keeps_nan_and_infinity(shape):
+    """NaN and infinities in the projection, the bias and the gradients come out where the operators have them,
+    forward and backward, and leave the other segments alone; finite values agree to fp32 rounding."""
+    N, H, d, du, rb, rq = shape
+    dims, nan, inf = shape[1:], float("nan"), float("inf")
+    x = _proj(*shape, torch.float32, "cuda")
+    head = 3 * d + 2 * du + rq + 1
+    at = [0, d, 2 * d, 2 * d + du, 2 * d + du + rq, 2 * d + du + rq + 1, head - 1]  # h0, A, R, coeff_Qf, lgA, lgB, lgQ
+    for n, v in ((2, nan), (3, inf), (4, -inf)):
+        for k, c in enumerate(at):  # alternating heads
+            x[n, (k % H) * head + c] = v
+        x[n, H * head] = x[n, H * head + rb] = v
+    bias = torch.linspace(-2, 1, 1 + du + d, device="cuda")
+    bias[[2, 1, 3, 1 + du]] = torch.tensor([nan, inf, -inf, nan], device="cuda")
+    g = torch.Generator().manual_seed(5)
+    ws = None
+    got = []
+    for f in (front_end, front_end_torch):
+        a, b = x.clone().requires_grad_(True), bias.clone().requires_grad_(True)
+        ys = f(a, b, dims)
+        if ws is None:
+            ws = [torch.randn(y.shape, generator=g).cuda() for y in ys]
+            ws[6][-1, 0, 0] = inf  # reaches the bias whose relu is off
+        got.append([y.detach() for y in ys] + list(torch.autograd.grad(ys, [a, b], ws)))
+    for p, q in zip(*got):
+        assert torch.equal(p.isnan(), q.isnan()) and torch.equal(p.isinf(), q.isinf())
+        assert torch.equal(p[q.isinf()], q[q.isinf()])
+        ok = q.isfinite()
+        scale = max(float(q[ok].abs().max()), 1.0)
+        assert float((p - q)[ok].abs().max()) <= (max(dims) / 2 + 10) * 2.0 ** -24 * 8 * scale
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("factored", [True, False])
+def test_layer_raises_on_a_nan_bias(factored):
+    """A NaN in ``bias_gamma`` reaches the solver, whose status word raises."""
+    from ttc import TTCLayer
+    torch.manual_seed(0)
+    layer = TTCLayer(32, 32, 16, 2, 8, 8, gamma_bias=True, factored=factored).cuda()
+    x = torch.randn(5, 32, device="cuda")
+    layer(x, T=4)
+    with torch.no_grad():
+        layer.bias_gamma[3] = float("nan")
+    with pytest.raises(RuntimeError):
+        layer(x, T=4)
+
+
+@pytest.mark.gpu
 def test_front_end_second_derivative_and_partial_gradients():
     """Under create_graph the backward is differentiable, as the operators' is; outputs without a
     gradient count as zero."""

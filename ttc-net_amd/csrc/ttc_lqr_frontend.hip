@@ -113,7 +113,10 @@ __global__ __launch_bounds__(256) void front_end_kernel(const float* __restrict_
   row += D.rq;
   for (int i = lane; i < 1 + D.du + D.d; i += 64) {
     float v = -softplus(row[i]);
-    if (bias != nullptr) v -= fmaxf(-bias[i], 0.f);
+    if (bias != nullptr) {  // relu that keeps NaN, as torch's does (fmaxf(NaN, 0) is 0)
+      const float m = -bias[i];
+      v -= m < 0.f ? 0.f : m;
+    }
     if (i == 0) lA[p] = v;
     else if (i <= D.du) lB[p * D.du + i - 1] = v;
     else lQ[p * D.d + i - 1 - D.du] = v;
