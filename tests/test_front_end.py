@@ -102,6 +102,26 @@ def test_layer_raises_on_a_nan_bias(factored):
 
 
 @pytest.mark.gpu
+def test_front_end_beyond_one_launch():
+    """2^26 + 6 (token, head) units, more than the 2^32 - 1 threads of one launch hold: both ends of the
+    tokens, and the seam of the two launches, get the operators' values, forward and backward.  The
+    norms' gradients are differences of two terms of at most s = 1 / |v| <= 5 here (inputs of magnitude
+    1/2 to 3/2, softplus at least 0.2), with about four roundings each: 8 * 2^-24 * 5 apart at most."""
+    N, dims = (1 << 25) + 3, (1, 1, 1, 0, 0)
+    proj = torch.rand(N, 6, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3)) * 2 - 1
+    proj = (proj + proj.sign() * 0.5).requires_grad_(True)
+    ys = front_end(proj, None, dims)
+    ws = [torch.ones_like(y) for y in ys]
+    (g,) = torch.autograd.grad(ys, proj, ws)
+    for part in (slice(0, 64), slice(N // 2, N // 2 + 64), slice(N - 128, N)):
+        p = proj.detach()[part].clone().requires_grad_(True)
+        want = front_end_torch(p, None, dims)
+        (gw,) = torch.autograd.grad(want, p, [w[part] for w in ws])
+        for a, b in zip([y[part] for y in ys] + [g[part]], list(want) + [gw]):
+            assert torch.allclose(a, b, rtol=1e-5, atol=3e-6)
+
+
+@pytest.mark.gpu
 def test_front_end_second_derivative_and_partial_gradients():
     """Under create_graph the backward is differentiable, as the operators' is; outputs without a
     gradient count as zero."""

@@ -86,13 +86,13 @@ __device__ __forceinline__ void norm_segment_backward(const float* __restrict__ 
 }
 
 __global__ __launch_bounds__(256) void front_end_kernel(const float* __restrict__ proj, const float* __restrict__ bias,
-                                                        int64_t N, FrontDims D, float* __restrict__ A,
+                                                        int64_t N, int64_t first, FrontDims D, float* __restrict__ A,
                                                         float* __restrict__ cB, float* __restrict__ cQ,
                                                         float* __restrict__ R, float* __restrict__ cQf,
                                                         float* __restrict__ lA, float* __restrict__ lB,
                                                         float* __restrict__ lQ, float* __restrict__ h0) {
   const int lane = threadIdx.x & 63;
-  const int64_t unit = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t unit = first + (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int64_t n = unit / (D.H + 1);
   if (n >= N) return;
   const int h = (int)(unit % (D.H + 1));
@@ -124,12 +124,12 @@ __global__ __launch_bounds__(256) void front_end_kernel(const float* __restrict_
 }
 
 __global__ __launch_bounds__(256) void front_end_backward_kernel(
-    const float* __restrict__ proj, int64_t N, FrontDims D, const float* __restrict__ gA, const float* __restrict__ gcB,
-    const float* __restrict__ gcQ, const float* __restrict__ gR, const float* __restrict__ gcQf,
-    const float* __restrict__ glA, const float* __restrict__ glB, const float* __restrict__ glQ,
-    const float* __restrict__ gh0, float* __restrict__ dproj) {
+    const float* __restrict__ proj, int64_t N, int64_t first, FrontDims D, const float* __restrict__ gA,
+    const float* __restrict__ gcB, const float* __restrict__ gcQ, const float* __restrict__ gR,
+    const float* __restrict__ gcQf, const float* __restrict__ glA, const float* __restrict__ glB,
+    const float* __restrict__ glQ, const float* __restrict__ gh0, float* __restrict__ dproj) {
   const int lane = threadIdx.x & 63;
-  const int64_t unit = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t unit = first + (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int64_t n = unit / (D.H + 1);
   if (n >= N) return;
   const int h = (int)(unit % (D.H + 1));
@@ -157,9 +157,26 @@ __global__ __launch_bounds__(256) void front_end_backward_kernel(
   }
 }
 
-static bool front_args_ok(int64_t n, int H, int d, int du, int rb, int rq) {
-  // (grid: one wave per token and head)
-  return n >= 0 && H > 0 && d > 0 && du > 0 && rb >= 0 && rq >= 0 && H < (1 << 20) && n <= ((int64_t)1 << 32) / (H + 1);
+// A launch takes at most 2^32 - 1 threads: units (one wave each) beyond that go in further launches.
+constexpr int64_t kFrontUnits = 4 * (((int64_t)1 << 24) - 1);
+
+// Any sizes whose element offsets fit 64 bits.
+static bool front_args_ok(int64_t n, int64_t H, int64_t d, int64_t du, int64_t rb, int64_t rq) {
+  if (n < 0 || H < 1 || d < 1 || du < 1 || rb < 0 || rq < 0) return false;
+  constexpr int64_t lim = (int64_t)1 << 31;
+  const int64_t head = 3 * d + 2 * du + rq + 1;
+  if (H + 1 >= lim || head >= lim || rb + rq >= lim) return false;
+  return n <= ((int64_t)1 << 62) / (head * H + rb + rq);
+}
+
+template <typename F>
+static int front_launches(int64_t units, F&& launch) {
+  for (int64_t first = 0; first < units; first += kFrontUnits) {
+    const int64_t left = units - first, now = left < kFrontUnits ? left : kFrontUnits;
+    launch(first, dim3((unsigned)((now + 3) / 4)));
+    if (hipGetLastError() != hipSuccess) return TTC_LQR_ELAUNCH;
+  }
+  return TTC_LQR_OK;
 }
 
 }  // namespace ttc
@@ -177,12 +194,11 @@ int ttc_lqr_front_end(const float* proj, const float* gamma_bias, int64_t n_toke
   if (!proj || !A_diag || (b_rank > 0 && !coeff_B) || (q_rank > 0 && (!coeff_Q || !coeff_Qf)) || !R_inv ||
       !log_gamma_A || !log_gamma_B || !log_gamma_Q || !h0)
     return TTC_LQR_EINVAL;
-  const int64_t units = n_tokens * (heads + 1);
-  hipLaunchKernelGGL(front_end_kernel, dim3((unsigned)((units + 3) / 4)), dim3(256), 0,
-                     reinterpret_cast<hipStream_t>(stream), proj, gamma_bias, n_tokens,
-                     FrontDims{heads, d, du, b_rank, q_rank}, A_diag, coeff_B, coeff_Q, R_inv, coeff_Qf, log_gamma_A,
-                     log_gamma_B, log_gamma_Q, h0);
-  return hipGetLastError() == hipSuccess ? TTC_LQR_OK : TTC_LQR_ELAUNCH;
+  return front_launches(n_tokens * ((int64_t)heads + 1), [&](int64_t first, dim3 grid) {
+    hipLaunchKernelGGL(front_end_kernel, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream), proj, gamma_bias,
+                       n_tokens, first, FrontDims{heads, d, du, b_rank, q_rank}, A_diag, coeff_B, coeff_Q, R_inv,
+                       coeff_Qf, log_gamma_A, log_gamma_B, log_gamma_Q, h0);
+  });
 }
 
 int ttc_lqr_front_end_backward(const float* proj, int64_t n_tokens, int32_t heads, int32_t d, int32_t du,
@@ -193,12 +209,12 @@ int ttc_lqr_front_end_backward(const float* proj, int64_t n_tokens, int32_t head
   if (!front_args_ok(n_tokens, heads, d, du, b_rank, q_rank)) return TTC_LQR_EINVAL;
   if (n_tokens == 0) return TTC_LQR_OK;
   if (!proj || !grad_proj) return TTC_LQR_EINVAL;
-  const int64_t units = n_tokens * (heads + 1);
-  hipLaunchKernelGGL(front_end_backward_kernel, dim3((unsigned)((units + 3) / 4)), dim3(256), 0,
-                     reinterpret_cast<hipStream_t>(stream), proj, n_tokens, FrontDims{heads, d, du, b_rank, q_rank},
-                     grad_A_diag, grad_coeff_B, grad_coeff_Q, grad_R_inv, grad_coeff_Qf, grad_log_gamma_A,
-                     grad_log_gamma_B, grad_log_gamma_Q, grad_h0, grad_proj);
-  return hipGetLastError() == hipSuccess ? TTC_LQR_OK : TTC_LQR_ELAUNCH;
+  return front_launches(n_tokens * ((int64_t)heads + 1), [&](int64_t first, dim3 grid) {
+    hipLaunchKernelGGL(front_end_backward_kernel, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream), proj,
+                       n_tokens, first, FrontDims{heads, d, du, b_rank, q_rank}, grad_A_diag, grad_coeff_B,
+                       grad_coeff_Q, grad_R_inv, grad_coeff_Qf, grad_log_gamma_A, grad_log_gamma_B, grad_log_gamma_Q,
+                       grad_h0, grad_proj);
+  });
 }
 
 }  // extern "C"
