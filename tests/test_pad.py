@@ -23,6 +23,22 @@ def test_pad_equals_torch(dtype, N, H, d, du, D):
         assert a.dtype == dtype and torch.equal(a, b)
 
 
+@pytest.mark.gpu
+def test_pad_beyond_one_launch():
+    """2^34 padded values and a few more, which are more than the 2^32 - 1 threads of one launch (four values
+    each) write: both ends, and the seam of the two launches, hold the inputs and the fill."""
+    from ttc.solvers.hip_lqr import _pad_tensors
+    M = (1 << 22) + 5
+    if torch.cuda.mem_get_info()[0] < 48 << 30:
+        pytest.skip("needs 36 GB")
+    x = torch.randn(M, 2, 3, device="cuda").to(torch.bfloat16)
+    (got,) = _pad_tensors([x], [(64, 64)], [1])
+    assert got.shape == (M, 64, 64)
+    for part in (slice(0, 8), slice((1 << 22) - 8, M)):
+        want = torch.nn.functional.pad(x[part], (0, 61, 0, 62), value=1.0)
+        assert torch.equal(got[part], want)
+
+
 def test_pad_argument_validation():
     from ttc.solvers._lib import lib
     p = (ctypes.c_void_p * 1)(64)

@@ -1,5 +1,5 @@
 // ttc_lqr_pad.hip -- zero-padding of the solver's tensors from (d, du) to the kernels' state size (16,
-// 32 or 64), all of a call in one launch.  As torch operators each tensor is a fill and a copy: 16
+// 32 or 64), all of a call in one launch (up to 64 GB).  As torch operators each tensor is a fill and a copy: 16
 // launches and their dispatch were 85 us of a small call; here it is one launch of about 5 us, one
 // write per output element (four a thread, 16 bytes) and one read per input element.
 #include <hip/hip_runtime.h>
@@ -34,11 +34,12 @@ __device__ __forceinline__ float get(const float* p) { return *p; }
 __device__ __forceinline__ float get(const uint16_t* p) { return __uint_as_float((uint32_t)*p << 16); }
 
 template <typename T>
-__global__ __launch_bounds__(256) void pad_kernel(const PadJobs jobs) {
+__global__ __launch_bounds__(256) void pad_kernel(const PadJobs jobs, unsigned block0) {
+  const unsigned block = block0 + blockIdx.x;
   int k = 0;
-  while (k + 1 < jobs.count && blockIdx.x >= jobs.first[k + 1]) ++k;  // uniform
+  while (k + 1 < jobs.count && block >= jobs.first[k + 1]) ++k;  // uniform
   const int lr = jobs.lrows[k], lc = jobs.lcols[k], rows = jobs.rows[k], cols = jobs.cols[k];
-  const int64_t e = ((int64_t)(blockIdx.x - jobs.first[k]) * 256 + threadIdx.x) * 4;
+  const int64_t e = ((int64_t)(block - jobs.first[k]) * 256 + threadIdx.x) * 4;
   const int64_t m = e >> (lr + lc);
   if (m >= jobs.M[k]) return;
   const int j = (int)(e & ((1 << lc) - 1)), i = (int)((e >> lc) & ((1 << lr) - 1));
@@ -84,9 +85,14 @@ extern "C" int ttc_lqr_pad(const void* const* src, void* const* dst, const int64
     if (blocks > 0x7fffffff) return TTC_LQR_EINVAL;
   }
   if (jobs.count == 0) return TTC_LQR_OK;
-  const dim3 grid((unsigned)blocks), block(256);
+  // a launch takes at most 2^32 - 1 threads (64 GB of fp32 outputs): the rest in further launches
+  constexpr int64_t kMostBlocks = ((int64_t)1 << 24) - 1;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (bytes == 4) hipLaunchKernelGGL(pad_kernel<float>, grid, block, 0, st, jobs);
-  else hipLaunchKernelGGL(pad_kernel<uint16_t>, grid, block, 0, st, jobs);
-  return hipGetLastError() == hipSuccess ? TTC_LQR_OK : TTC_LQR_ELAUNCH;
+  for (int64_t b = 0; b < blocks; b += kMostBlocks) {
+    const dim3 grid((unsigned)(blocks - b < kMostBlocks ? blocks - b : kMostBlocks)), block(256);
+    if (bytes == 4) hipLaunchKernelGGL(pad_kernel<float>, grid, block, 0, st, jobs, (unsigned)b);
+    else hipLaunchKernelGGL(pad_kernel<uint16_t>, grid, block, 0, st, jobs, (unsigned)b);
+    if (hipGetLastError() != hipSuccess) return TTC_LQR_ELAUNCH;
+  }
+  return TTC_LQR_OK;
 }
