@@ -9,7 +9,7 @@ from ttc.layers.front_end import front_end, front_end_torch
 
 # (tokens, heads, d, du, b_rank, q_rank): one wave's width and its neighbours, ranks beyond it, no rank
 SHAPES = [(1, 1, 1, 1, 1, 1), (3, 2, 16, 16, 16, 16), (5, 3, 63, 20, 65, 7), (2, 8, 64, 64, 32, 64), (4, 1, 65, 3, 0, 130),
-          (33, 5, 24, 20, 8, 33)]
+          (33, 5, 24, 20, 8, 33), (3, 2, 7, 0, 4, 4), (2, 1, 0, 5, 1, 0)]
 
 
 def _proj(N, H, d, du, rb, rq, dtype, device):
@@ -145,6 +145,7 @@ def test_front_end_argument_validation():
     assert lib.ttc_lqr_front_end(p, None, 0, 1, 4, 4, 2, 2, *[p] * 9, None) == 0      # nothing to do
     assert lib.ttc_lqr_front_end(None, None, 1, 1, 4, 4, 2, 2, *[p] * 9, None) == 1
     assert lib.ttc_lqr_front_end(p, None, 1, 0, 4, 4, 2, 2, *[p] * 9, None) == 1
+    assert lib.ttc_lqr_front_end(p, None, 1, 1, 4, -1, 2, 2, *[p] * 9, None) == 1
     assert lib.ttc_lqr_front_end(p, None, 1, 1, 4, 4, 2, 2, *[p] * 8, None, None) == 1
     assert lib.ttc_lqr_front_end_backward(p, 1, 1, 4, 4, 2, 2, *[p] * 9, None, None) == 1
     assert lib.ttc_lqr_front_end_backward(p, 0, 1, 4, 4, 2, 2, *[None] * 9, None, None) == 0

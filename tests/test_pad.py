@@ -24,6 +24,32 @@ def test_pad_equals_torch(dtype, N, H, d, du, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("d,du", [(5, 0), (0, 3), (0, 0)])
+def test_sizes_without_elements(d, du):
+    """No controls or no states: the solvers and the layer pad them like any other size, u is empty or zero
+    and so are the gradients."""
+    from ttc import TTCLayer
+    from ttc.solvers.hip_lqr import hip_lqr_solve, hip_lqr_solve_factored
+    N, H, r = 3, 2, 4
+    ones = lambda *s: torch.ones(*s, device="cuda", requires_grad=True)  # noqa: E731
+    lgs = [ones(N, H), ones(N, H, du), ones(N, H, d)]
+    ins = [ones(N, H, d), ones(N, d, du), ones(N, d, d), ones(N, H, du), ones(N, H, d, d), *lgs, ones(N, H, d)]
+    fact = [ones(N, H, d), ones(N, r), ones(N, r), ones(N, H, du), ones(N, H, r), *lgs, ones(N, H, d),
+            ones(r, d, du), ones(r, d, d)]
+    for solve, xs in ((hip_lqr_solve, ins), (hip_lqr_solve_factored, fact)):
+        u = solve(*xs, 4)
+        assert u.shape == (N, H, du) and not u.any()
+        for x, g in zip(xs, torch.autograd.grad(u.sum(), xs)):
+            assert g.shape == x.shape and not g.any()
+    if d:
+        layer = TTCLayer(8, 8, d, H, r, r, u_dim=du).cuda()
+        x = torch.randn(N, 8, device="cuda", requires_grad=True)
+        y = layer(x, T=4)
+        y.sum().backward()
+        assert y.shape == (N, 8) and not y.any() and not x.grad.any()
+
+
+@pytest.mark.gpu
 def test_pad_beyond_one_launch():
     """2^34 padded values and a few more, which are more than the 2^32 - 1 threads of one launch (four values
     each) write: both ends, and the seam of the two launches, hold the inputs and the fill."""

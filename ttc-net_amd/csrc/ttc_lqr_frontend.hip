@@ -162,12 +162,14 @@ constexpr int64_t kFrontUnits = 4 * (((int64_t)1 << 24) - 1);
 
 // Any sizes whose element offsets fit 64 bits.
 static bool front_args_ok(int64_t n, int64_t H, int64_t d, int64_t du, int64_t rb, int64_t rq) {
-  if (n < 0 || H < 1 || d < 1 || du < 1 || rb < 0 || rq < 0) return false;
+  if (n < 0 || H < 1 || d < 0 || du < 0 || rb < 0 || rq < 0) return false;
   constexpr int64_t lim = (int64_t)1 << 31;
   const int64_t head = 3 * d + 2 * du + rq + 1;
   if (H + 1 >= lim || head >= lim || rb + rq >= lim) return false;
   return n <= ((int64_t)1 << 62) / (head * H + rb + rq);
 }
+
+static bool given(const void* p, int64_t elements) { return elements == 0 || p != nullptr; }
 
 template <typename F>
 static int front_launches(int64_t units, F&& launch) {
@@ -191,8 +193,8 @@ int ttc_lqr_front_end(const float* proj, const float* gamma_bias, int64_t n_toke
                       float* h0, void* stream) {
   if (!front_args_ok(n_tokens, heads, d, du, b_rank, q_rank)) return TTC_LQR_EINVAL;
   if (n_tokens == 0) return TTC_LQR_OK;
-  if (!proj || !A_diag || (b_rank > 0 && !coeff_B) || (q_rank > 0 && (!coeff_Q || !coeff_Qf)) || !R_inv ||
-      !log_gamma_A || !log_gamma_B || !log_gamma_Q || !h0)
+  if (!proj || !given(A_diag, d) || !given(coeff_B, b_rank) || !given(coeff_Q, q_rank) || !given(R_inv, du) ||
+      !given(coeff_Qf, q_rank) || !log_gamma_A || !given(log_gamma_B, du) || !given(log_gamma_Q, d) || !given(h0, d))
     return TTC_LQR_EINVAL;
   return front_launches(n_tokens * ((int64_t)heads + 1), [&](int64_t first, dim3 grid) {
     hipLaunchKernelGGL(front_end_kernel, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream), proj, gamma_bias,

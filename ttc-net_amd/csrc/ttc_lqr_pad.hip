@@ -68,9 +68,9 @@ extern "C" int ttc_lqr_pad(const void* const* src, void* const* dst, const int64
   for (int k = 0; k < count; ++k) {
     const int64_t* s = shapes + 5 * k;  // matrices, rows, cols, padded rows, padded cols
     const int lr = log2of(s[3]), lc = log2of(s[4]);
-    if (s[0] < 0 || s[1] < 1 || s[2] < 1 || s[1] > s[3] || s[2] > s[4] || lr < 0 || lc < 2) return TTC_LQR_EINVAL;
+    if (s[0] < 0 || s[1] < 0 || s[2] < 0 || s[1] > s[3] || s[2] > s[4] || lr < 0 || lc < 2) return TTC_LQR_EINVAL;
     if (s[0] == 0) continue;
-    if (!src[k] || !dst[k]) return TTC_LQR_EINVAL;
+    if ((!src[k] && s[1] > 0 && s[2] > 0) || !dst[k]) return TTC_LQR_EINVAL;
     const int c = jobs.count++;
     jobs.src[c] = src[k];
     jobs.dst[c] = dst[k];

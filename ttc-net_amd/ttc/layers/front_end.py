@@ -88,7 +88,7 @@ class _FrontEndFunc(torch.autograd.Function):
                                                     torch.cuda.current_stream(p.device).cuda_stream)
             check(rc, "ttc_lqr_front_end_backward")
         if need_bias:
-            zero = lambda g, n: bias.new_zeros(n) if g is None else g.reshape(-1, n).sum(0)  # noqa: E731
+            zero = lambda g, n: bias.new_zeros(n) if g is None else g.reshape(N * H, n).sum(0)  # noqa: E731
             d_bias = torch.cat([zero(grads[5], 1), zero(grads[6], ud), zero(grads[7], hd)])
             d_bias = d_bias.masked_fill(bias >= 0, 0.0)  # relu's gradient: 0 where it is off, NaN passes
         return d_proj, d_bias, None

@@ -98,7 +98,7 @@ def _pad_tensors(xs, shapes, fills):
         k = len(shape)
         outs.append(torch.empty(*x.shape[:-k], *shape, device=dev, dtype=x.dtype))
         rows = (x.shape[-2], shape[0]) if k == 2 else (1, 1)
-        dims += [x.numel() // (rows[0] * x.shape[-1]), rows[0], x.shape[-1], rows[1], shape[-1]]
+        dims += [math.prod(x.shape[:-k]), rows[0], x.shape[-1], rows[1], shape[-1]]
     ptrs = ctypes.c_void_p * n
     with torch.cuda.device(dev):
         rc = lib.ttc_lqr_pad(ptrs(*[x.data_ptr() for x in xs]), ptrs(*[o.data_ptr() for o in outs]),
