@@ -129,6 +129,24 @@ def test_d16_head_groups_matrix_core_backward(N, H, T):
     assert out["_fallback"] % 8 == 0
 
 
+@pytest.mark.parametrize("N,H", [(10, 8), (400, 6), (1000, 8), (1001, 6), (4100, 1)])
+def test_d16_problems_ignore_their_wave_mates(N, H):
+    """A problem whose Quu_0 is indefinite is solved with row exchanges; every other problem of its wave (heads of
+    its token, or other tokens' at head counts that are no multiple of 4) keeps its bits.  Controls
+    of growing reach make Quu_0's largest entries lie off its diagonal, so that row exchanges would
+    change them."""
+    from ttc.solvers.hip_lqr import hip_lqr_solve
+    T = 5
+    ins = [t.cuda() for t in bench_solver_inputs(N, H, 16, seed=N)]
+    ins[1], ins[3] = ins[1] * torch.logspace(-1, 1, 16, device="cuda"), ins[3] * 20.0
+    u = hip_lqr_solve(*ins, T)
+    bad = torch.zeros(N, H, dtype=torch.bool, device="cuda")
+    bad[1::7, H // 2] = True
+    ins[3] = torch.where(bad[..., None] & (torch.arange(16, device="cuda") == 3), -0.002 * ins[3], ins[3])
+    v = hip_lqr_solve(*ins, T)
+    assert torch.equal(u[~bad], v[~bad]) and not torch.equal(u[bad], v[bad])
+
+
 @pytest.mark.parametrize("N,H,T", [(5, 3, 9), (3, 4, 33), (2, 7, 2), (4, 5, 1), (3, 9, 17), (2, 12, 40), (2, 15, 8)])
 def test_d64_ragged_head_groups(N, H, T):
     """The d = 64 head-group backward at head counts that are no multiple of 8: the token's last group has

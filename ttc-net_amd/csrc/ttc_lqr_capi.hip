@@ -298,8 +298,8 @@ static int fwd_d(int d, const float* a, const float* b, const float* q, const fl
   flags = forward_flags(flags, d, H, sm);
   switch (d) {
     case 16:
-      return launch_fwd_d16(a, b, q, r, qf, la, lb, lq, hz, P, H, T, u, st_a, st_b, sm, status, s, flags, rescue_ws,
-                            rs);
+      return launch_fwd_d16(a, b, q, r, qf, la, lb, lq, hz, P, H, T, u, st_a, st_b, sm, status, s, flags, call,
+                            rescue_ws, rs);
     case 32:
       return launch_fwd_d32(a, b, q, r, qf, la, lb, lq, hz, P, H, T, u, st_a, st_b, sm, status, s, flags, call,
                             rescue_ws);

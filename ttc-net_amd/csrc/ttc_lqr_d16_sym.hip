@@ -8,9 +8,9 @@ namespace ttc {
 template <int SM, bool WU>
 static void launch_s16(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                        const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T,
-                       float* u, float* st_a, float* st_b, int32_t* status, hipStream_t s, bool fp64_rescue,
-                       int32_t* rescue_ws, RescueSlots rs) {
-  launch_sym16<SM, WU>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s);
+                       float* u, float* st_a, float* st_b, int32_t* status, hipStream_t s, int64_t call,
+                       bool fp64_rescue, int32_t* rescue_ws, RescueSlots rs) {
+  launch_sym16<SM, WU>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, call);
   if (fp64_rescue) {
     // long horizons: the rejected problems are the ill-conditioned ones, recomputed in fp64 --
     // listed, on the matrix cores (the LU row-layout sweep finishing any whose Cholesky breaks
@@ -35,20 +35,20 @@ static void launch_s16(const float* A, const float* B, const float* Q, const flo
 int launch_fwd_d16_sym(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                        const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H,
                        int T, float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s,
-                       bool fp64_rescue, int32_t* rescue_ws, RescueSlots rs) {
+                       int64_t call, bool fp64_rescue, int32_t* rescue_ws, RescueSlots rs) {
   if (P <= 0) return TTC_LQR_OK;
   switch (sm) {
     case STASH_NONE:
-      launch_s16<STASH_NONE, true>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, fp64_rescue,
-                                   rescue_ws, rs);
+      launch_s16<STASH_NONE, true>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, call,
+                                   fp64_rescue, rescue_ws, rs);
       break;
     case STASH_V1:
       if (u != nullptr)
-        launch_s16<STASH_V1, true>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, fp64_rescue,
-                                   rescue_ws, rs);
+        launch_s16<STASH_V1, true>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, call,
+                                   fp64_rescue, rescue_ws, rs);
       else
-        launch_s16<STASH_V1, false>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, fp64_rescue,
-                                    rescue_ws, rs);
+        launch_s16<STASH_V1, false>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s, call,
+                                    fp64_rescue, rescue_ws, rs);
       break;
     default:
       return TTC_LQR_EINVAL;

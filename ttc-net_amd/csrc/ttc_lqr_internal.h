@@ -28,11 +28,13 @@ int launch_fwd_d16_mfma(const float* A, const float* B, const float* Q, const fl
                         const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H,
                         int T, float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s);
 // fp64_rescue: the problems the symplectic sweep's certificate rejects are recomputed by the
-// fp64 row-layout sweep (TTC_LQR_FLAG_FP64_RESCUE) instead of the fp32 rescue tiers.
+// fp64 row-layout sweep (TTC_LQR_FLAG_FP64_RESCUE) instead of the fp32 rescue tiers.  call: the problems of
+// the whole call, which choose the kernel's form.
 int launch_fwd_d16_sym(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                        const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H,
                        int T, float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s,
-                       bool fp64_rescue, int32_t* rescue_ws = nullptr, RescueSlots rs = RescueSlots{});
+                       int64_t call, bool fp64_rescue, int32_t* rescue_ws = nullptr,
+                       RescueSlots rs = RescueSlots{});
 // d = 16, fp64 on the matrix cores (ttc_lqr_d16_f64.hip): the rescue of the problems a symplectic
 // sweep marked (sm = STASH_NONE / STASH_V1; rescue_ws of rescue_ws_bytes(P)), and every gain
 // K_t plus Quu_0 of P problems in fp64 (the stable backward).
@@ -68,7 +70,7 @@ int launch_fwd_d64_mfma(const float* A, const float* B, const float* Q, const fl
 int launch_fwd_d16(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                   const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T,
                   float* u, float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s, int flags,
-                  int32_t* rescue_ws = nullptr, RescueSlots rs = RescueSlots{});
+                  int64_t call, int32_t* rescue_ws = nullptr, RescueSlots rs = RescueSlots{});
 int launch_bwd_d16(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                   const float* lA, const float* lB, const float* lQ, const float* h0, const float* dU,
                   const float* kst, const float* q0s, int64_t P, int H, int T, void* traj, bool fp64, float* gA,

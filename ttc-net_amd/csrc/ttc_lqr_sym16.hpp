@@ -309,14 +309,15 @@ lqr_sym16_kernel(const float* __restrict__ A_diag, const float* __restrict__ Bg,
   int pos = c;
   {
     // Quu_0 is positive definite for a certified problem: elimination without row exchanges by DPP
-    // broadcasts; a wave where a pivot says otherwise is solved again with partial pivoting
-    float x[17];
+    // broadcasts; a problem where a pivot says otherwise is solved again with partial pivoting (by the
+    // whole wave, taken by that problem alone: no problem's bits depend on its wave-mates)
+    float x[17], xpiv;
 #pragma unroll
     for (int k = 0; k < 17; ++k) x[k] = row[k];
-    bool bad;
-    gj_spd16x1(x, c, piv, bad);
+    bool bad;  // the same on a problem's 16 lanes
+    gj_spd16x1(x, c, xpiv, bad);
     if (__any(bad)) gauss_jordan<D, D + 4, 4, D + 1>(row, c, buf, piv, pos);
-    else row[D] = x[16];
+    if (!bad) row[D] = x[16], piv = xpiv, pos = c;
   }
   const float u0 = -row[D] / piv;
   if (store) {
@@ -344,19 +345,20 @@ inline void launch_sym16_ppw(const float* A, const float* B, const float* Q, con
                      status);
 }
 
-// Problems per wave, by what 1,024 SIMDs have to do (whole call, T = 64): one up to 2,048 problems (512:
-// 115 us against 133 with two and 168 with four), two up to 4,096 (162 / 178 us with four; odd head
-// counts one, 164), four above (8,160: 226 us against 222 with two, 65,280: 960 / 1,020), sharing the
-// token's operands when the head count is a multiple of four; otherwise a copy each, since waves with
-// idle slots cost more (524,280 problems: 7.2 ms; by token 7.3 with 2 heads, 7.1 with 3 and 6, 8.2 with
-// 1 and 5; shared by four 6.7).
+// Problems per wave, by what 1,024 SIMDs have to do for the whole call's problems (these P may be a chunk of
+// them, and the forms give the same bits only as far as the compiler treats them alike).  Whole call,
+// T = 64: one up to 2,048 problems (512: 115 us against 133 with two and 168 with four), two up to 4,096
+// (162 / 178 us with four; odd head counts one, 164), four above (8,160: 226 us against 222 with two,
+// 65,280: 960 / 1,020), sharing the token's operands when the head count is a multiple of four; otherwise
+// a copy each, since waves with idle slots cost more (524,280 problems: 7.2 ms; by token 7.3 with 2
+// heads, 7.1 with 3 and 6, 8.2 with 1 and 5; shared by four 6.7).
 template <int SM, bool WU>
 inline void launch_sym16(const float* A, const float* B, const float* Q, const float* R, const float* Qf,
                          const float* lA, const float* lB, const float* lQ, const float* h0, int64_t P, int H, int T,
-                         float* u, float* st_a, float* st_b, int32_t* status, hipStream_t s) {
-  if (P <= 2048 || (P <= 4096 && H % 2 != 0))
+                         float* u, float* st_a, float* st_b, int32_t* status, hipStream_t s, int64_t call) {
+  if (call <= 2048 || (call <= 4096 && H % 2 != 0))
     launch_sym16_ppw<1, true, SM, WU>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s);
-  else if (P <= 4096)
+  else if (call <= 4096)
     launch_sym16_ppw<2, true, SM, WU>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s);
   else if (H % 4 == 0)
     launch_sym16_ppw<4, true, SM, WU>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s);
