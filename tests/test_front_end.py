@@ -185,6 +185,52 @@ def test_transforms_and_tracing_see_the_operators():
 
 
 @pytest.mark.gpu
+def test_dispatch_modes_and_batched_gradients_see_the_operators():
+    """Dispatch modes over plain tensors (make_fx on real tensors, a mode that counts) record the operators, not
+    empty outputs that a kernel fills unseen; batched gradients pass the backward; all with the operators'
+    values, forward and backward."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils._python_dispatch import TorchDispatchMode
+    dims = (2, 6, 5, 3, 4)
+    x = _proj(3, *dims, torch.float32, "cuda")
+    bias = torch.linspace(-2, 1, 12, device="cuda")
+
+    def step(f):
+        def run(t, b):
+            t, b = t.detach().requires_grad_(), b.detach().requires_grad_()
+            ys = f(t, b, dims)
+            return [*ys, *torch.autograd.grad(sum((y * y).sum() for y in ys), (t, b))]
+        return run
+
+    traced = make_fx(step(front_end))(x, bias)
+    for p, q in zip(traced(2 * x, 0.5 * bias), step(front_end_torch)(2 * x, 0.5 * bias)):
+        assert torch.equal(p, q)
+
+    class Names(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.seen = getattr(self, "seen", set()) | {func.overloadpacket}
+            return func(*args, **(kwargs or {}))
+
+    with Names() as mode:
+        front_end(x, bias, dims)
+    assert torch.ops.aten.softplus in mode.seen
+    t = x.clone().requires_grad_()
+    b = bias.clone().requires_grad_()
+    ys = front_end(t, b, dims)
+    with Names() as mode:
+        torch.autograd.grad(ys, (t, b), [torch.ones_like(y) for y in ys], retain_graph=True)
+    assert torch.ops.aten.softplus_backward in mode.seen
+
+    def jacobian(f):
+        t, b = x.clone().requires_grad_(), bias.clone().requires_grad_()
+        y = f(t, b, dims)[3]
+        seeds = torch.eye(y.numel(), device="cuda").reshape(-1, *y.shape)
+        return torch.autograd.grad(y, (t, b), seeds, is_grads_batched=True, allow_unused=True)
+    for p, q in zip(jacobian(front_end), jacobian(front_end_torch)):
+        assert (p is None and q is None) or torch.equal(p, q)
+
+
+@pytest.mark.gpu
 def test_no_grad_forward_writes_no_stash(monkeypatch):
     """Under no_grad a layer whose parameters require gradients runs the forward without a stash (nothing
     asks whether one fits), with the same bits as a recorded forward."""

@@ -4,10 +4,10 @@ the split of the projection, ``l2norm`` / softplus / clamp and the log-discounts
 :func:`front_end` takes the projection ``[N, row]`` and returns ``(A_diag, coeff_B, coeff_Q, R_inv,
 coeff_Qf, log_gamma_A, log_gamma_B, log_gamma_Q, h0)``.  fp32 CUDA projections go through one kernel
 each way (``ttc_lqr_front_end`` / ``_backward``, contiguous outputs); anything else, and any call under a
-functorch transform, forward-mode AD or tracing, runs :func:`front_end_torch`, the same formulas as
-torch operators.  The backward differentiates
-:func:`front_end_torch` when it is itself recorded (``create_graph=True``), so second derivatives
-of the front-end are what autograd gives for the operators.
+functorch transform, forward-mode AD, a dispatch mode or tracing, runs :func:`front_end_torch`, the same
+formulas as torch operators.  The backward differentiates :func:`front_end_torch` when it is itself
+recorded (``create_graph=True``) or so observed (batched gradients), so second derivatives of the
+front-end are what autograd gives for the operators.
 """
 from __future__ import annotations
 
@@ -67,12 +67,16 @@ class _FrontEndFunc(torch.autograd.Function):
         need_proj, need_bias = ctx.needs_input_grad[:2]
         if all(g is None for g in grads):
             return None, None, None
-        if torch.is_grad_enabled():  # recorded: differentiable operators
-            out = front_end_torch(proj, bias, ctx.dims)
-            pairs = [(o, g) for o, g in zip(out, grads) if g is not None]
-            wrt = [t for t, need in ((proj, need_proj), (bias, need_bias)) if need]
-            got = iter(torch.autograd.grad([o for o, _ in pairs], wrt, [g for _, g in pairs], create_graph=True,
-                                           allow_unused=True))
+        recorded = torch.is_grad_enabled()
+        if recorded or _traced(proj, bias, *grads):  # differentiable operators, seen one by one
+            with torch.enable_grad():
+                if not recorded:
+                    proj, bias = (t if t is None else t.detach().requires_grad_() for t in (proj, bias))
+                out = front_end_torch(proj, bias, ctx.dims)
+                pairs = [(o, g) for o, g in zip(out, grads) if g is not None]
+                wrt = [t for t, need in ((proj, need_proj), (bias, need_bias)) if need]
+                got = iter(torch.autograd.grad([o for o, _ in pairs], wrt, [g for _, g in pairs],
+                                               create_graph=recorded, allow_unused=True))
             return next(got) if need_proj else None, next(got) if need_bias else None, None
         H, hd, ud, rb, rq = ctx.dims
         N = proj.shape[0]
@@ -95,11 +99,14 @@ class _FrontEndFunc(torch.autograd.Function):
 
 
 def _traced(*xs) -> bool:
-    """Whether operators are observed one by one (functorch transforms, forward-mode tangents, tracing and
-    compilation, tensor subclasses such as fake tensors): none of these sees into an autograd Function."""
-    return (any(type(x) not in (torch.Tensor, torch.nn.Parameter) for x in xs if x is not None)
-            or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0
-            or torch.jit.is_tracing() or torch.compiler.is_compiling())
+    """Whether operators are observed one by one (functorch transforms, batched gradients, forward-mode
+    tangents, tracing and compilation, dispatch modes such as ``make_fx``'s, tensor subclasses such as fake
+    tensors): none of these sees the kernel."""
+    return (any(type(x) not in (torch.Tensor, torch.nn.Parameter) or not torch._C._has_storage(x)
+                for x in xs if x is not None)
+            or torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack() > 0
+            or torch.autograd.forward_ad._current_level >= 0 or torch.jit.is_tracing()
+            or torch.compiler.is_compiling())
 
 
 def front_end(proj: torch.Tensor, bias: torch.Tensor | None, dims):
