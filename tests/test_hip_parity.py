@@ -179,6 +179,27 @@ def test_d64_ragged_head_groups_rejected(N, H):
         assert _relerr(fast[k], slow[k]) <= TOL, k
 
 
+@pytest.mark.parametrize("N,H", [(6, 3), (5, 7), (4, 11)])
+def test_d64_ragged_groups_second_rollout(N, H):
+    """One barely discounted head with spread scales in some tokens: its group is rejected, but only that head's
+    problems take the stable path -- the others' own rollouts are accepted."""
+    T = 48
+    ins = bench_solver_inputs(N, H, 64, seed=N + H)
+    A_diag, B, Q, R_inv, Qf, lgA, lgB, lgQ, h0 = ins
+    A_diag[::2, 1] *= 4.0
+    R_inv[::2, 1] *= 20.0
+    for lg in (lgA, lgB, lgQ):
+        lg[::2, 1] *= 0.01
+    pb = LQRProblem(*ins, T)
+    dU = torch.randn(pb.N, pb.H, pb.du, generator=torch.Generator().manual_seed(3)).double().numpy()
+    fast = run_hip(ins, T, dU, grad_limit=math.inf)
+    print(f"fallback {fast['_fallback']}/{pb.P}", flush=True)
+    assert 0 < fast["_fallback"] <= (N + 1) // 2
+    ref = solve_grads(pb, dU)
+    for k in ["u"] + NAMES:
+        assert _relerr(fast[k], ref[k]) <= TOL, k
+
+
 def test_d16_head_groups_with_rejected_groups():
     """Config-5 stress problems regrouped to 16 heads per token: groups that fail the
     certificate go through the stable path as whole groups, and the head sums of grad_B /
