@@ -147,6 +147,20 @@ def test_d16_problems_ignore_their_wave_mates(N, H):
     assert torch.equal(u[~bad], v[~bad]) and not torch.equal(u[bad], v[bad])
 
 
+@pytest.mark.parametrize("N,H,T", [(24, 5, 96), (12, 11, 160), (30, 1, 200), (24, 4, 96), (3, 5, 512)])
+@pytest.mark.parametrize("stash", ["always", "never"])
+def test_d32_rejected_problems_in_fp64(N, H, T, stash):
+    """Layer inputs with widely spread token scales at d = 32: the problems the sweep's certificate rejects are
+    recomputed in fp64 at odd head counts as at even ones, below and from the horizon on from which the
+    odd ones sweep in fp64 throughout.  In fp32 they leave u 1e-5 to 2e-3 off; certified
+    problems are within 1e-5."""
+    x = make_x(4, n_tokens=N, seed=T) / 0.02
+    x = x * torch.exp(1.5 * torch.randn(N, 1, generator=torch.Generator().manual_seed(T)))
+    ins = [t[:, :H].contiguous() if t.shape[:2] == (N, 32) and k not in (1, 2) else t
+           for k, t in enumerate(layer_solver_inputs(4, x))]
+    check_case(f"rejected32 N={N} H={H}", ins, T, grad_limit=math.inf, stash=stash, tol=1e-5)
+
+
 @pytest.mark.parametrize("N,H,T", [(5, 3, 9), (3, 4, 33), (2, 7, 2), (4, 5, 1), (3, 9, 17), (2, 12, 40), (2, 15, 8)])
 def test_d64_ragged_head_groups(N, H, T):
     """The d = 64 head-group backward at head counts that are no multiple of 8: the token's last group has

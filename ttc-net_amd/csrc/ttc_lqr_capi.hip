@@ -254,15 +254,12 @@ static bool fp64_rollout(int flags, int d) {
   return (flags & (TTC_LQR_FLAG_FP64_RICCATI | TTC_LQR_FLAG_FP64_RESCUE)) != 0 && d <= 32;
 }
 
-// Flags of a forward sweep (stash mode sm): TTC_LQR_FLAG_FP64_FALLBACK's forward is
-// TTC_LQR_FLAG_FP64_RESCUE's -- the fp32 symplectic sweep with its rejected problems recomputed in
-// fp64, and the stable path's gains in fp64 -- except at d = 32 with an odd head count, whose
-// rejected problems take the fp32 tiers for u and the stash (TTC_LQR_FLAG_FP64_RESCUE itself sweeps
-// every problem of an odd head count in fp64 there).
-static int forward_flags(int flags, int d, int H, int sm) {
+// Flags of a forward sweep: TTC_LQR_FLAG_FP64_FALLBACK's forward is TTC_LQR_FLAG_FP64_RESCUE's -- the
+// fp32 symplectic sweep with its rejected problems recomputed in fp64, and the stable path's gains
+// in fp64.  It keeps its own bit beside the other's, by which launch_fwd_d32 tells the two apart.
+static int forward_flags(int flags) {
   if (!(flags & TTC_LQR_FLAG_FP64_FALLBACK)) return flags;
-  flags &= ~TTC_LQR_FLAG_FP64_FALLBACK;
-  if (sm != kStashGains && d == 32 && H % 2 != 0) return flags;
+  if (flags & TTC_LQR_FLAG_FP64_RESCUE) return flags & ~TTC_LQR_FLAG_FP64_FALLBACK;
   return flags | TTC_LQR_FLAG_FP64_RESCUE;
 }
 
@@ -295,7 +292,7 @@ static int fwd_d(int d, const float* a, const float* b, const float* q, const fl
                  const float* la, const float* lb, const float* lq, const float* hz, int64_t P, int H, int T, float* u,
                  float* st_a, float* st_b, int sm, int32_t* status, hipStream_t s, int flags, int64_t call,
                  int32_t* rescue_ws = nullptr, RescueSlots rs = RescueSlots{}) {
-  flags = forward_flags(flags, d, H, sm);
+  flags = forward_flags(flags);
   switch (d) {
     case 16:
       return launch_fwd_d16(a, b, q, r, qf, la, lb, lq, hz, P, H, T, u, st_a, st_b, sm, status, s, flags, call,

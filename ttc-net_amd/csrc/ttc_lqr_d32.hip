@@ -9,10 +9,14 @@ int launch_fwd_d32(const float* A, const float* B, const float* Q, const float* 
                   int64_t call, int32_t* rescue_ws) {
   // fp32 sweeps without per-step gains run on the matrix cores unless the row-layout kernel
   // is asked for: the certified symplectic sweep by default, per-step Riccati when asked for.
-  // fp64 rescue of a symplectic sweep at even head counts; odd ones, per-step Riccati and the
-  // row-layout kernel run fp64 throughout
+  // fp64 rescue of a symplectic sweep; without one (the stable backward's gains, row-layout or
+  // Riccati-step kernels asked for) the sweep is fp64 throughout.  So it is at odd head counts under
+  // TTC_LQR_FLAG_FP64_RESCUE itself (long horizons), which has always promised them that: 5 heads,
+  // 64 tokens, T = 512 end 2e-8 (u) and 2e-7 (gradients) from 64 bits in 34.8 ms, where the certified
+  // fp32 sweep of the even counts ends 1.4e-6 and 2.2e-6 away in 0.6 ms.
+  const bool odd = H % 2 != 0 && !(flags & TTC_LQR_FLAG_FP64_FALLBACK);
   if ((flags & TTC_LQR_FLAG_FP64_RESCUE) &&
-      (sm == STASH_GAINS || (flags & (TTC_LQR_FLAG_ROW_KERNEL | TTC_LQR_FLAG_RICCATI_STEPS)) || H % 2 != 0))
+      (sm == STASH_GAINS || (flags & (TTC_LQR_FLAG_ROW_KERNEL | TTC_LQR_FLAG_RICCATI_STEPS)) || odd))
     flags |= TTC_LQR_FLAG_FP64_RICCATI;
   if (!(flags & (TTC_LQR_FLAG_FP64_RICCATI | TTC_LQR_FLAG_ROW_KERNEL)) && sm != STASH_GAINS)
     return launch_fwd_d32_mfma(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, sm, status, s,
