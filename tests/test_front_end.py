@@ -22,34 +22,57 @@ def _proj(N, H, d, du, rb, rq, dtype, device):
     return x.to(device=device, dtype=dtype)
 
 
+def _reference64(proj, bias, dims):
+    """The front-end in the dtype of its arguments throughout (``front_end_torch`` normalises in fp32), and per
+    normalised output the factor s = 1 / sqrt(|v|^2 + 1e-6) of its rows."""
+    H, d, du, rb, rq = dims
+    head = [d, d, du, rq, 1 + du + d]
+    heads, cB, cQ = torch.split(proj, [sum(head) * H, rb, rq], dim=-1)
+    h0, A, R, cQf, lg = torch.split(heads.reshape(-1, H, sum(head)), head, dim=-1)
+    F = torch.nn.functional
+    vs = [A, cB, F.softplus(cQ), F.softplus(R), F.softplus(cQf)]
+    ss = [torch.rsqrt((v * v).sum(-1, keepdim=True) + 1e-6) for v in vs]
+    A, cB, cQ, R, cQf = (v * s for v, s in zip(vs, ss))
+    lg = -F.softplus(lg) - (0 if bias is None else F.relu(-bias))
+    lgA, lgB, lgQ = torch.split(lg, [1, du, d], dim=-1)
+    return (A, cB, cQ, torch.clamp(R, min=1e-6), cQf, lgA.squeeze(-1), lgB, lgQ, h0), ss
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("with_bias", [False, True])
 def test_front_end_kernel(shape, with_bias):
-    """Values and gradients, relative to each output's largest entry: a sum of n squares in fp32, a
-    reciprocal root, exp and log1p leave at most (n / 2 + 10) 2^-24 of it."""
+    """Values and gradients against 64 bits, to first order in u = 2^-24.  A softplus (expf, log1pf) is 6 u off; a sum
+    of n products in a wave adds n / 64 + 6 roundings; so s = rsqrt(sum + 1e-6) is (n / 128 + 12) u off
+    and a value (n / 128 + 20) u of itself.  The gradient s g_i - v_i (v . g) s^3 has terms of at most
+    s |g_i| and s |g|, off by (n / 128 + 20) u and (5 n / 128 + 65) u with the softplus's derivative."""
     N, H, d, du, rb, rq = shape
     dims = (H, d, du, rb, rq)
-    tol = (max(d, du, rb, rq) / 2 + 10) * 2.0 ** -24 * 4
+    n, u = max(d, du, rb, rq), 2.0 ** -24
     a = _proj(*shape, torch.float32, "cuda").requires_grad_(True)
     b = a.detach().double().cpu().requires_grad_(True)
     bias = torch.linspace(-2, 1, 1 + du + d) if with_bias else None
     ba = None if bias is None else bias.cuda().requires_grad_(True)
     bb = None if bias is None else bias.double().requires_grad_(True)
-    ya, yb = front_end(a, ba, dims), front_end_torch(b, bb, dims)
+    ya, (yb, ss) = front_end(a, ba, dims), _reference64(b, bb, dims)
     g = torch.Generator().manual_seed(9)
     # (R's clamp is a step in its gradient: entries within rounding of it are left out)
-    ws = [torch.randn(y.shape, generator=g, dtype=torch.float64) for y in yb]
+    ws = [torch.randn(y.shape, generator=g).double() for y in yb]
     ws[3] = ws[3] * ((yb[3].detach() - 1e-6).abs() > 1e-9)
     ins_a, ins_b = [a] + ([ba] if with_bias else []), [b] + ([bb] if with_bias else [])
     ga = torch.autograd.grad([(y * w.float().cuda()).sum() for y, w in zip(ya, ws)], ins_a)
     gb = torch.autograd.grad([(y * w).sum() for y, w in zip(yb, ws)], ins_b)
-    # l2norm in front_end_torch works in fp32 whatever the input; redo it in 64 bits for the bound
     for x, y in list(zip(ya, yb)) + list(zip(ga, gb)):
         assert x.is_contiguous() and x.shape == y.shape
-        if y.numel():
-            scale = max(float(y.detach().abs().max()), 1e-30)
-            assert float((x.detach().double().cpu() - y.detach()).abs().max()) <= 2 * tol * scale + 1e-12
+    for x, y in zip(ya, yb):
+        assert bool(((x.detach().double().cpu() - y.detach()).abs() <= (n / 128 + 20) * u * y.detach().abs()).all())
+    size = [s.detach() * (w.abs() + w.norm(dim=-1, keepdim=True)) for s, w in zip(ss, ws)]
+    lg = torch.cat([ws[5].unsqueeze(-1), ws[6], ws[7]], dim=-1)
+    heads = torch.cat([ws[8], size[0], size[3], size[4], lg], dim=-1)
+    size = torch.cat([heads.reshape(N, -1), size[1], size[2]], dim=-1).abs()
+    assert bool(((ga[0].double().cpu() - gb[0]).abs() <= (n / 25 + 65) * u * size).all())
+    if with_bias:
+        assert bool(((ga[1].double().cpu() - gb[1]).abs() <= (N * H + 1) * u * lg.abs().sum((0, 1))).all())
 
 
 @pytest.mark.gpu
