@@ -11,7 +11,9 @@
 // most of a decode step (160 us of kernels, 520 us with their dispatch) and at 2,048 tokens half of
 // a training step; here it is one kernel each way.  One wave per (token, head) and one for the
 // token's shared coefficients: a row's segments are read coalesced, their sums of squares reduced in
-// the wave, and at large token counts the pass is two memory touches per value.
+// the wave.  Large calls are not bound by memory either: 51 MB in 48 us (1,021 tokens of 32 heads, d =
+// 32), 1.1 TB/s -- at d = 16 a segment fills 16 of the 64 lanes, the five norms' reductions depend on
+// shuffles one after the other, and each softplus is evaluated again when its value is written.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>

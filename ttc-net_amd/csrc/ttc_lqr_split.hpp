@@ -3,7 +3,11 @@
 // A float has a 24-bit significand and a bf16 number an 8-bit one with the same exponent range, so
 // x = hi + mid + lo with hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi - mid): both
 // differences are exact in fp32, and round-to-nearest leaves |mid| <= 2^-9 |x| and a remainder of
-// at most 6 bits for lo, so the sum is exact.  A product of two such numbers keeps the six terms
+// at most 6 bits for lo, so the sum is exact -- where all three are normal bf16 numbers: below about
+// 2^-108 first lo, then mid fall under 2^-126 and |x| keeps fewer bits, and above 3.39e38 hi rounds to
+// infinity (the sweeps' certificate then fails on the NaN that follows, and the problem is recomputed
+// in fp32 or fp64).  The sweeps rescale their columns to [1, 2) every 8 steps, so only state costs that
+// are all that small reach the lower range.  A product of two such numbers keeps the six terms
 //   hi hi, hi mid, mid hi, hi lo, mid mid, lo hi
 // (each exact in the fp32 accumulator's product) and drops mid lo + lo mid + lo lo, below
 // 2^-26 |x y|: under the half ulp of the fp32 product that one fused multiply-add rounds.  The sum

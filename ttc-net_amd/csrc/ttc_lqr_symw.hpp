@@ -19,12 +19,16 @@
 // two tiles.)  In both, group v of four registers is the rows row(v) .. + 3 and a k-block is two groups.
 //
 // Bound at d = 64: 288 matrix instructions per problem-step (9,200 busy cycles per SIMD) beside about
-// 1,300 vector instructions, and the power they draw: at 32,768 problems x 128 steps the matrix cores
-// are busy 67 % of the time at 1.27 PFLOP/s (bf16), and the clock falls from 2.4 to 1.8 GHz, so that
+// 1,550 vector instructions (its share of the final solve included), and the power they draw: at 131,072 problems x 128 steps the matrix cores
+// are busy 68 % of the time at 1.38 PFLOP/s (bf16), and the clock averages 1.95 of 2.4 GHz, so that
 // fewer cycles (dot-product residuals, 6.55e7, against masked subtractions and interleaved issue,
-// 5.64e7) gave the same time.  47.1 -> 30.5 ms there against the fp32 matrix cores (90 % of their
-// peak); 256 problems 1.65 -> 0.66 ms; one head (1,024 problems), which ran Riccati steps, 3.87 ->
-// 1.75 ms.
+// 5.64e7, at 32,768 problems) gave the same time.  47.1 -> 30.5 ms there against the fp32 matrix cores
+// (90 % of their peak); with 16 columns a wave 256 problems 1.65 -> 0.42 ms, and one head (1,024
+// problems), which ran Riccati steps, 3.87 -> 1.16 ms.  Problems that the certificate rejects pay for
+// this sweep and then for Riccati steps, at every head count: where a fifth of the problems are
+// rejected (token scales spread by e^N(0,1.5), T = 256) a head count that ran Riccati steps alone loses,
+// 4.4 -> 6.0 ms with 3 heads x 256 tokens and 4.3 -> 5.3 with one head x 512; with 12 heads x 128, a
+// multiple of 4, which had an fp32 sweep before, 13.9 -> 7.5 ms.
 // At d = 32 the matrix cores (36 instructions of 34 cycles per problem-step) and the vector ALU (375
 // instructions) bound it together, and the waves to overlap them decide: 131,072 problems x 256 steps
 // 36.8 ms with two waves per SIMD (workgroups of 8 waves), 30.6 with three of 4 waves, 29.4 with
@@ -490,8 +494,9 @@ inline void launch_symw(const float* A, const float* B, const float* Q, const fl
   // SIMDs idle or with one wave (measured, T = 128, whole call: d = 64, 256 problems 476 against 644 us,
   // 512 663 / 677, 1,024 1,157 / 1,097; d = 32, 512 problems 248 / 318, 1,024 301 / 325, 2,048 482 /
   // 443); the operands are read from LDS twice as often, which costs 9 % when the chip is full, so at
-  // d = 64 also for the odd head counts whose idle waves cost more (1 head 29.1 / 38.2 ms, 3 heads
-  // 29.2 / 35.6, 5 heads 28.9 / 31.9 for 30,000 problems; at 9 heads 10 / 9 of the wide form's time)
+  // d = 64 also for the odd head counts whose idle waves cost more (30,000 problems, narrow / wide: 1 head
+  // 29.1 / 38.2 ms, 3 heads 29.2 / 35.6, 5 heads 28.9 / 31.9, 7 heads 29.3 / 30.3, 9 heads 29.2 / 29.9,
+  // 11 heads 29.2 / 28.9; the wide form's idle half problem is one part in H + 1 of its work)
   if (call * D <= 32768 || (D == 64 && H % 2 != 0 && H <= 9))
     launch_symw_cw<D, 16, SM, WU>(A, B, Q, R, Qf, lA, lB, lQ, h0, P, H, T, u, st_a, st_b, status, s);
   else
