@@ -174,6 +174,23 @@ def test_front_end_argument_validation():
     assert lib.ttc_lqr_front_end_backward(p, 0, 1, 4, 4, 2, 2, *[None] * 9, None, None) == 0
 
 
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_front_end_compiles_as_one_graph(device):
+    """``torch.compile(fullgraph=True)`` of the layer's front-end traces the operators, forward and backward."""
+    from ttc import TTCLayer
+    torch.manual_seed(0)
+    layer = TTCLayer(8, 8, 4, 2, 3, 3, gamma_bias=True, solver_impl="riccati" if device == "cpu" else "hip").to(device)
+    x = torch.randn(5, 8, device=device)
+    for f in (layer.solver_inputs, layer.factored_inputs):
+        torch._dynamo.reset()
+        got, want = torch.compile(f, backend="aot_eager", fullgraph=True)(x), f(x)
+        assert all(torch.allclose(p, q, rtol=1e-5, atol=1e-7) for p, q in zip(got, want))
+        ws = list(layer.parameters())
+        gs = [torch.autograd.grad(sum((y * y).sum() for y in ys), ws, allow_unused=True) for ys in (got, want)]
+        assert all(p is None or torch.allclose(p, q, rtol=1e-4, atol=1e-6) for p, q in zip(*gs))
+    torch._dynamo.reset()
+
+
 def test_cpu_and_other_dtypes_use_the_operators():
     dims = (2, 6, 5, 3, 4)
     for dt in (torch.float32, torch.bfloat16):

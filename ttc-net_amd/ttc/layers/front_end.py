@@ -102,11 +102,12 @@ def _traced(*xs) -> bool:
     """Whether operators are observed one by one (functorch transforms, batched gradients, forward-mode
     tangents, tracing and compilation, dispatch modes such as ``make_fx``'s, tensor subclasses such as fake
     tensors): none of these sees the kernel."""
+    if torch.compiler.is_compiling():  # first: a full-graph compilation can trace none of the rest
+        return True
     return (any(type(x) not in (torch.Tensor, torch.nn.Parameter) or not torch._C._has_storage(x)
                 for x in xs if x is not None)
             or torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack() > 0
-            or torch.autograd.forward_ad._current_level >= 0 or torch.jit.is_tracing()
-            or torch.compiler.is_compiling())
+            or torch.autograd.forward_ad._current_level >= 0 or torch.jit.is_tracing())
 
 
 def front_end(proj: torch.Tensor, bias: torch.Tensor | None, dims):
