@@ -162,6 +162,23 @@ def test_front_end_second_derivative_and_partial_gradients():
     assert float(p.sum()) == 3 * 2 * 6
 
 
+@pytest.mark.gpu
+def test_other_sizes_broadcast_or_raise():
+    """A projection of another width raises and a bias of another size broadcasts or raises, as in the operators:
+    the kernel, which would read beyond either, is not launched."""
+    dims = (2, 6, 5, 3, 4)
+    x = _proj(3, *dims, torch.float32, "cuda")
+    for wrong in (x[:, :-1], torch.cat([x, x], dim=1), x[:, :40]):
+        with pytest.raises(RuntimeError):
+            front_end(wrong, None, dims)
+    for bias in (torch.full((1,), -0.5, device="cuda"), torch.full((), -0.5, device="cuda")[None]):
+        for p, q in zip(front_end(x, bias, dims), front_end_torch(x, bias, dims)):
+            assert torch.equal(p, q)
+    for n in (11, 13, 24):
+        with pytest.raises(RuntimeError):
+            front_end(x, torch.zeros(n, device="cuda"), dims)
+
+
 def test_front_end_argument_validation():
     from ttc.solvers._lib import lib
     p = ctypes.c_void_p(16)

@@ -111,8 +111,12 @@ def _traced(*xs) -> bool:
 
 
 def front_end(proj: torch.Tensor, bias: torch.Tensor | None, dims):
-    """``dims = (heads, h_dim, u_dim, b_rank, q_rank)``."""
-    if not _traced(proj, bias) and proj.is_cuda and proj.dtype == torch.float32 and proj.dim() == 2 and (
-            bias is None or (bias.device == proj.device and bias.dtype == torch.float32)):
+    """``dims = (heads, h_dim, u_dim, b_rank, q_rank)``.  The kernel takes exactly the sizes that these give; the
+    operators broadcast any other bias, or raise."""
+    H, hd, ud, rb, rq = dims
+    if not _traced(proj, bias) and proj.is_cuda and proj.dtype == torch.float32 and (
+            proj.dim() == 2 and proj.shape[1] == (3 * hd + 2 * ud + rq + 1) * H + rb + rq) and (
+            bias is None or (bias.device == proj.device and bias.dtype == torch.float32
+                             and bias.shape == (1 + ud + hd,))):
         return _FrontEndFunc.apply(proj, bias, dims)
     return front_end_torch(proj, bias, dims)
