@@ -6,8 +6,8 @@
 // same recursion, certificate and outputs as lqr_ham_bwd_kernel) widened to D = 16 NW.
 // A workgroup of NW waves rolls one head group: 8 consecutive heads of one token (RAG: up to 8; the
 // token's last group takes what is left, its idle columns carry the last problem's constants with
-// h_0 = u_0 = d_u = 0, stay zero and are not stored), primal and adjoint, i.e. 16 trajectories.  Wave I owns state rows 16I..16I+15 of all 16
-// trajectories in the MFMA C layout (lane (g, c) holds rows 16I+4g..16I+4g+3 of trajectory
+// h_0 = u_0 = d_u = 0, stay zero and are not stored), primal and adjoint, i.e. 16 trajectories.  Wave
+// I owns state rows 16I..16I+15 of all 16 trajectories in the MFMA C layout (lane (g, c) holds rows 16I+4g..16I+4g+3 of trajectory
 // c; trajectory c is problem c & 7, adjoint when c >= 8).
 //
 // Each per-step product -- Q (q o S), B' Lambda, B (beta o U) -- is for wave I the row block

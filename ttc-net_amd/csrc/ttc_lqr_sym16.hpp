@@ -2,7 +2,8 @@
 // then the final solve and Riccati step 0.
 //
 // One wave holds PPW problems -- with TOK heads of one token and one register copy of B, B' and -sym(Q),
-// else any consecutive problems with a copy each -- as Y-hat = [Y1'; Y2'] in the MFMA C layout: lane 16 g + c holds rows 4 g + r of column c.  Per step
+// else any consecutive problems with a copy each -- as Y-hat = [Y1'; Y2'] in the MFMA C layout: lane
+// 16 g + c holds rows 4 g + r of column c.  Per step
 //   M = R^{-1} B_k' Y2'      Y1' <- A_k^{-1} (Y1' + B_k M)      Y2' <- A_k Y2' + Qc_k Y1'
 // (the reference's transposed row-block update, symplectic_iter.py:226-251, with V_t = Y1^{-1} Y2) is
 // three products of four v_mfma_f32_16x16x4f32; 12 and about 33 vector instructions per problem.  Fp32
@@ -39,8 +40,8 @@ __attribute__((amdgpu_waves_per_eu(Sym16<PPW, TOK>::MINW, Sym16<PPW, TOK>::MINW)
 lqr_sym16_kernel(const float* __restrict__ A_diag, const float* __restrict__ Bg, const float* __restrict__ Qg,
                  const float* __restrict__ Rinv, const float* __restrict__ Qf, const float* __restrict__ lgA,
                  const float* __restrict__ lgB, const float* __restrict__ lgQ, const float* __restrict__ h0,
-                 int64_t P, int H, int T, int PB, float* __restrict__ u_out, float* __restrict__ kstash, float* __restrict__ q0stash,
-                 int* __restrict__ status) {
+                 int64_t P, int H, int T, int PB, float* __restrict__ u_out, float* __restrict__ kstash,
+                 float* __restrict__ q0stash, int* __restrict__ status) {
   using G = Sym16<PPW, TOK>;
   constexpr int D = 16, LDX = G::LDX, NBQ = G::NBQ;
   extern __shared__ __align__(16) float sm[];

@@ -19,10 +19,10 @@
 // two tiles.)  In both, group v of four registers is the rows row(v) .. + 3 and a k-block is two groups.
 //
 // Bound at d = 64: 288 matrix instructions per problem-step (9,200 busy cycles per SIMD) beside about
-// 1,550 vector instructions (its share of the final solve included), and the power they draw: at 131,072 problems x 128 steps the matrix cores
-// are busy 68 % of the time at 1.38 PFLOP/s (bf16), and the clock averages 1.95 of 2.4 GHz, so that
-// fewer cycles (dot-product residuals, 6.55e7, against masked subtractions and interleaved issue,
-// 5.64e7, at 32,768 problems) gave the same time.  47.1 -> 30.5 ms there against the fp32 matrix cores
+// 1,550 vector instructions (its share of the final solve included), and the power they draw: at
+// 131,072 problems x 128 steps the matrix cores are busy 68 % of the time at 1.38 PFLOP/s (bf16), and
+// the clock averages 1.95 of 2.4 GHz, so that fewer cycles (dot-product residuals, 6.55e7, against
+// masked subtractions and interleaved issue, 5.64e7, at 32,768 problems) gave the same time.  47.1 -> 30.5 ms there against the fp32 matrix cores
 // (90 % of their peak); with 16 columns a wave 256 problems 1.65 -> 0.42 ms, and one head (1,024
 // problems), which ran Riccati steps, 3.87 -> 1.16 ms.  Problems that the certificate rejects pay for
 // this sweep and then for Riccati steps, at every head count: where a fifth of the problems are
